@@ -51,6 +51,27 @@ def test_mlp_gradients_match_reference(B):
     assert abs(float(tr.loss) - loss_ref) <= 1e-4 * abs(loss_ref)
 
 
+@pytest.mark.parametrize("B", [1, 31, 33, 8192 + 32 * 3 + 5])
+def test_mlp_gradients_at_row_block_edges(B):
+    """A training workgroup takes 32 rows at a time: fewer rows than one
+    block, one row past it, and a batch beyond one round of the grid
+    (256 workgroups) that ends in a partial block. The same bounds as
+    test_mlp_gradients_match_reference; a second call gives the same bits,
+    the sums having a fixed order."""
+    from yggdrax_amd import learned
+    p = learned.init_params(5)
+    x, t, m = _batch(B, 2)
+    m[0] = 1.0
+    tr = learned.Trainer(p, B)
+    dev = [torch.from_numpy(a).cuda() for a in (x, t, m)]
+    g = tr.gradients(*dev)
+    loss = float(tr.loss)
+    loss_ref, g_ref = mlp_ref.loss_and_grad(p, x, t, m)
+    np.testing.assert_allclose(g.cpu().numpy(), g_ref, rtol=1e-3, atol=1e-5 * np.abs(g_ref).max())
+    assert abs(loss - loss_ref) <= 1e-4 * abs(loss_ref)
+    assert torch.equal(tr.gradients(*dev), g) and float(tr.loss) == loss
+
+
 def test_mlp_training_reduces_loss():
     from yggdrax_amd import learned
     rng = np.random.default_rng(0)

@@ -175,168 +175,265 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const uint16_t* __restrict__ 
   }
 }
 
-// ---- training: layer kernels over a batch (row-major activations) -------
-// On the matrix cores with v_mfma_f32_16x16x4_f32 (fp32 operands, fp32
-// accumulation; the sums run in a different order than a scalar loop, the
-// products are the same). Operand layouts on wave64 (lane l):
+constexpr float kLn2 = 0.69314718055994531f;
+constexpr float kMaxLogRate = 30.0f;
+
+// ---- training: one kernel for a batch's gradients, one for the update ----
+// k_train_grads: a workgroup takes kRows batch rows at a time through the
+// forward pass, the masked Poisson loss (rate 2^y, y clamped at 30; per
+// element m (2^y - t y ln 2) / B, gradient m (2^y - t) ln 2 / B) and the
+// backward pass with every activation and delta in LDS, and keeps its weight
+// gradients in MFMA accumulators until its last rows. It then writes one
+// slice of partial sums (the parameters' layout, the loss after them);
+// k_train_update adds the slices in a fixed order and takes the Adam step.
+//
+// The products run on v_mfma_f32_16x16x4_f32 (fp32 operands and sums):
 //   A[m][k]: lane l holds A[l % 16][l / 16]
 //   B[k][n]: lane l holds B[l / 16][l % 16]
 //   D[m][n]: lane l holds D[4 (l / 16) + j][l % 16], j = 0..3
-// (the D layout of the 16x16x16 bf16 form above). Operands past a matrix's
-// edge are zero, so any size works with whole 16 x 16 tiles.
+// and where k runs along a row of LDS, step s of lane group q takes
+// k = 16 q + s, so that a lane's operands of four steps are one 16-byte read.
+//
+// Bound by its own chain of ten phases (each a few thousand MFMA cycles a
+// workgroup), no longer by eighteen dependent launches; kRows = 32 gives a
+// batch of 4096 a workgroup on every second CU and halves the slices'
+// traffic against 16.
+// A step of 4096 rows takes 22 us, against
+// 208 us for eighteen launches (a layer at a time through memory, 4-byte
+// operand reads).
+constexpr int kRows = 32;
+constexpr int kLd = kH + 4;     // LDS row: 16-byte aligned, bank-shifted
+constexpr int kTrainBlocks = 256;
+constexpr int kSlice = (kParams + 1 + 15) / 16 * 16;  // floats per slice, loss at kParams
+
 __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// y[b][o] = act(sum_i W[o][i] x[b][i] + bias[o]): one wavefront per 16
-// batch rows, every 16-output tile (m = row, n = output, k = input).
-__global__ __launch_bounds__(256) void k_lin_fwd(const uint16_t* __restrict__ W,
-                                                 const uint16_t* __restrict__ bias,
-                                                 const float* __restrict__ x, int B, int nin,
-                                                 int nout, int relu, float* __restrict__ y) {
-  const int lane = (int)lane_id(), r = lane % 16, q = lane / 16;
-  const int64_t b0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / YGG_WAVE * 16;
-  if (b0 >= B) return;
-  for (int n0 = 0; n0 < nout; n0 += 16) {
-    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = 0; k0 < nin; k0 += 4) {
-      const int64_t b = b0 + r;
-      const int k = k0 + q, o = n0 + r;
-      const float av = (b < B && k < nin) ? x[b * nin + k] : 0.0f;
-      const float bv = (o < nout && k < nin) ? bf16_to_f32(W[o * nin + k]) : 0.0f;
-      acc = mfma4(av, bv, acc);
+// acc[16 x 16] += A-row r times B-row r over k = 0..63 (both rows in LDS).
+__device__ __forceinline__ f32x4_t dot_rows(const float* a, const float* b, int q, f32x4_t acc) {
+#pragma unroll
+  for (int s = 0; s < 16; s += 4) {
+    const f32x4_t av = *(const f32x4_t*)(a + 16 * q + s), bv = *(const f32x4_t*)(b + 16 * q + s);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = mfma4(av[j], bv[j], acc);
+  }
+  return acc;
+}
+
+// acc[16 x 16] += A-row r times B-column (LDS rows k, column c) over k = 0..63.
+__device__ __forceinline__ f32x4_t dot_cols(const float* a, const float (*b)[kLd], int c, int q,
+                                            f32x4_t acc) {
+#pragma unroll
+  for (int s = 0; s < 16; s += 4) {
+    const f32x4_t av = *(const f32x4_t*)(a + 16 * q + s);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = mfma4(av[j], b[16 * q + s + j][c], acc);
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(256) void k_train_grads(const uint16_t* __restrict__ W,
+                                                     const float* __restrict__ x,
+                                                     const float* __restrict__ target,
+                                                     const float* __restrict__ mask, int64_t B,
+                                                     float* __restrict__ partial) {
+  __shared__ __align__(16) float s_w2[kH][kLd], s_w3[kH][kLd];
+  __shared__ __align__(16) float s_a1[kRows][kLd], s_a2[kRows][kLd], s_a3[kRows][kLd];
+  __shared__ __align__(16) float s_d[2][kRows][kLd];
+  __shared__ float s_w1[kH][kIn + 1], s_w4[kOut][kH], s_x[kRows][kIn + 1], s_dy[kRows][kOut + 1];
+  __shared__ float s_loss[2];
+  const int tid = threadIdx.x, lane = (int)lane_id(), r = lane % 16, q = lane / 16;
+  const int w = tid / YGG_WAVE, n0 = 16 * w;
+  for (int e = tid; e < kH * kH; e += 256) {
+    s_w2[e / kH][e % kH] = bf16_to_f32(W[kOffW2 + e]);
+    s_w3[e / kH][e % kH] = bf16_to_f32(W[kOffW3 + e]);
+  }
+  for (int e = tid; e < kH * kIn; e += 256) s_w1[e / kIn][e % kIn] = bf16_to_f32(W[kOffW1 + e]);
+  if (tid < kOut * kH) s_w4[tid / kH][tid % kH] = bf16_to_f32(W[kOffW4 + tid]);
+  const float bias1 = bf16_to_f32(W[kOffB1 + n0 + r]), bias2 = bf16_to_f32(W[kOffB2 + n0 + r]),
+              bias3 = bf16_to_f32(W[kOffB3 + n0 + r]),
+              bias4 = r < kOut ? bf16_to_f32(W[kOffB4 + r]) : 0.0f;
+  // this workgroup's gradients: wavefront w holds outputs [16 w, 16 w + 16)
+  // of the hidden layers, thread tid one weight of the last and one bias
+  f32x4_t g1 = {0.0f, 0.0f, 0.0f, 0.0f}, g2[4], g3[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) g2[t] = g3[t] = g1;
+  float g4 = 0.0f, gb = 0.0f, loss = 0.0f;
+
+  for (int64_t base = (int64_t)blockIdx.x * kRows; base < B; base += (int64_t)gridDim.x * kRows) {
+    const int rows = B - base < kRows ? (int)(B - base) : kRows;
+    __syncthreads();  // weights staged; the previous rows' last phase is done
+    {
+      const int b = tid / kIn, i = tid % kIn;  // 256 threads = kRows x kIn
+      s_x[b][i] = b < rows ? x[(base + b) * kIn + i] : 0.0f;
     }
-    const int o = n0 + r;
-    if (o < nout) {  // every lane reaches the next tile's MFMAs
-      const float bo = bf16_to_f32(bias[o]);
+    __syncthreads();
+    // rows past the batch hold zeros in every activation and delta
+    auto put = [&](float (*dst)[kLd], int rt, const f32x4_t& v) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int64_t b = b0 + 4 * q + j;
-        if (b < B) {
-          const float v = acc[j] + bo;
-          y[b * nout + o] = relu ? fmaxf(v, 0.0f) : v;
+        const int b = 16 * rt + 4 * q + j;
+        dst[b][n0 + r] = b < rows ? fmaxf(v[j], 0.0f) : 0.0f;
+      }
+    };
+#pragma unroll
+    for (int rt = 0; rt < kRows / 16; ++rt) {
+      f32x4_t acc = {bias1, bias1, bias1, bias1};
+#pragma unroll
+      for (int k0 = 0; k0 < kIn; k0 += 4)
+        acc = mfma4(s_x[16 * rt + r][k0 + q], s_w1[n0 + r][k0 + q], acc);
+      put(s_a1, rt, acc);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < kRows / 16; ++rt)
+      put(s_a2, rt, dot_rows(s_a1[16 * rt + r], s_w2[n0 + r], q, f32x4_t{bias2, bias2, bias2, bias2}));
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < kRows / 16; ++rt)
+      put(s_a3, rt, dot_rows(s_a2[16 * rt + r], s_w3[n0 + r], q, f32x4_t{bias3, bias3, bias3, bias3}));
+    __syncthreads();
+    if (w < kRows / 16) {  // outputs and loss: wavefront w takes rows [16 w, 16 w + 16)
+      f32x4_t acc = {bias4, bias4, bias4, bias4};
+#pragma unroll
+      for (int s = 0; s < 16; s += 4) {
+        const f32x4_t av = *(const f32x4_t*)(&s_a3[n0 + r][16 * q + s]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc = mfma4(av[j], r < kOut ? s_w4[r][16 * q + s + j] : 0.0f, acc);
+      }
+      if (r < kOut) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int b = n0 + 4 * q + j;
+          float dy = 0.0f;
+          if (b < rows) {
+            const int64_t e = (base + b) * kOut + r;
+            const float t = target[e], m = mask[e], yv = acc[j];
+            const float yc = fminf(yv, kMaxLogRate), lam = exp2f(yc);
+            dy = yv > kMaxLogRate ? 0.0f : m * (lam - t) * kLn2 / (float)B;
+            loss += m * (lam - t * yc * kLn2) / (float)B;
+          }
+          s_dy[b][r] = dy;
         }
       }
     }
-  }
-}
-
-// dx[b][i] = sum_o W[o][i] dy[b][o], times relu'(x) when the input came from
-// a ReLU (m = row, n = input, k = output).
-__global__ __launch_bounds__(256) void k_lin_bwd_data(const uint16_t* __restrict__ W,
-                                                      const float* __restrict__ dy,
-                                                      const float* __restrict__ xin, int B,
-                                                      int nin, int nout, int relu_in,
-                                                      float* __restrict__ dx) {
-  const int lane = (int)lane_id(), r = lane % 16, q = lane / 16;
-  const int64_t b0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / YGG_WAVE * 16;
-  if (b0 >= B) return;
-  for (int n0 = 0; n0 < nin; n0 += 16) {
-    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = 0; k0 < nout; k0 += 4) {
-      const int64_t b = b0 + r;
-      const int o = k0 + q, i = n0 + r;
-      const float av = (b < B && o < nout) ? dy[b * nout + o] : 0.0f;
-      const float bv = (o < nout && i < nin) ? bf16_to_f32(W[o * nin + i]) : 0.0f;
-      acc = mfma4(av, bv, acc);
-    }
-    const int i = n0 + r;
-    if (i < nin) {
+    __syncthreads();
+    // deltas of the third layer, gradients of the last
+    for (int e = tid; e < kRows * kH; e += 256) {
+      const int b = e / kH, i = e % kH;
+      float d = 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t b = b0 + 4 * q + j;
-        if (b < B) {
-          const int64_t e = b * nin + i;
-          dx[e] = (relu_in && !(xin[e] > 0.0f)) ? 0.0f : acc[j];
+      for (int o = 0; o < kOut; ++o) d += s_dy[b][o] * s_w4[o][i];
+      s_d[0][b][i] = s_a3[b][i] > 0.0f ? d : 0.0f;
+    }
+    if (tid < kOut * kH) {
+      const int o = tid / kH, i = tid % kH;
+#pragma unroll 8
+      for (int b = 0; b < kRows; ++b) g4 += s_dy[b][o] * s_a3[b][i];
+    } else if (tid < kOut * kH + kOut) {
+      for (int b = 0; b < kRows; ++b) gb += s_dy[b][tid - kOut * kH];
+    }
+    __syncthreads();
+    // weight gradients of a hidden layer (m = output, n = input, k = row),
+    // and its bias gradients in 64 threads of their own
+    auto weight_grads = [&](const float (*d)[kLd], const float (*a)[kLd], f32x4_t (&g)[4]) {
+#pragma unroll
+      for (int b0 = 0; b0 < kRows; b0 += 4) {
+        const float dv = d[b0 + q][n0 + r];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) g[t] = mfma4(dv, a[b0 + q][16 * t + r], g[t]);
+      }
+    };
+    auto bias_grads = [&](const float (*d)[kLd], int wave) {
+      if (w == wave)
+        for (int b = 0; b < kRows; ++b) gb += d[b][lane];
+    };
+    // deltas of the layer below: d W, where the ReLU passed
+    auto down = [&](const float (*d)[kLd], const float (*wt)[kLd], const float (*a)[kLd],
+                    float (*out)[kLd]) {
+#pragma unroll
+      for (int rt = 0; rt < kRows / 16; ++rt) {
+        const f32x4_t v = dot_cols(d[16 * rt + r], wt, n0 + r, q, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int b = 16 * rt + 4 * q + j;
+          out[b][n0 + r] = a[b][n0 + r] > 0.0f ? v[j] : 0.0f;
         }
       }
+    };
+    weight_grads(s_d[0], s_a2, g3);
+    bias_grads(s_d[0], 0);
+    down(s_d[0], s_w3, s_a2, s_d[1]);
+    __syncthreads();
+    weight_grads(s_d[1], s_a1, g2);
+    bias_grads(s_d[1], 1);
+    down(s_d[1], s_w2, s_a1, s_d[0]);
+    __syncthreads();
+#pragma unroll
+    for (int b0 = 0; b0 < kRows; b0 += 4)
+      g1 = mfma4(s_d[0][b0 + q][n0 + r], r < kIn ? s_x[b0 + q][r] : 0.0f, g1);
+    bias_grads(s_d[0], 2);
+  }
+
+  float* __restrict__ out = partial + (int64_t)blockIdx.x * kSlice;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = n0 + 4 * q + j;
+    if (r < kIn) out[kOffW1 + o * kIn + r] = g1[j];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      out[kOffW2 + o * kH + 16 * t + r] = g2[t][j];
+      out[kOffW3 + o * kH + 16 * t + r] = g3[t][j];
     }
   }
+  if (tid < kOut * kH) out[kOffW4 + tid] = g4;
+  // biases: wavefronts 0, 1, 2 hold those of layers 3, 2, 1, and the first
+  // kOut threads of wavefront 3 the last layer's
+  if (w < 3)
+    out[(w == 0 ? kOffB3 : (w == 1 ? kOffB2 : kOffB1)) + lane] = gb;
+  else if (lane < kOut)
+    out[kOffB4 + lane] = gb;
+  loss = wave_sum_f(loss);
+  if (lane == 0 && w < 2) s_loss[w] = loss;
+  __syncthreads();
+  if (tid == 0) out[kParams] = s_loss[0] + s_loss[1];
 }
 
-// Weight gradients, split over the batch: slice s of kGradSlice rows adds
-// into partial[s][m][n] = sum_b dy[b][m] xa[b][n] with xa = [x | 1] (the
-// column n = nin gives the bias gradient); m = output, n = input, k = row.
-// One wavefront per (16 x 16 tile, slice); Mp, Np are nout and nin + 1
-// rounded up to 16. The slices are summed in a fixed order afterwards, so
-// the gradients are deterministic.
-constexpr int kGradSlice = 256;
-
-__global__ __launch_bounds__(256) void k_lin_bwd_weight(const float* __restrict__ dy,
-                                                        const float* __restrict__ x, int B,
-                                                        int nin, int nout, int Mp, int Np,
-                                                        float* __restrict__ partial) {
-  const int lane = (int)lane_id(), r = lane % 16, q = lane / 16;
-  const int wave = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / YGG_WAVE);
-  const int tiles_n = Np / 16, tiles = (Mp / 16) * tiles_n;
-  const int slices = (B + kGradSlice - 1) / kGradSlice;
-  if (wave >= tiles * slices) return;
-  const int s = wave / tiles, t = wave % tiles;
-  const int m0 = (t / tiles_n) * 16, n0 = (t % tiles_n) * 16;
-  const int kb = s * kGradSlice, ke = min(B, kb + kGradSlice);
-  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int b0 = kb; b0 < ke; b0 += 4) {
-    const int b = b0 + q;
-    const int o = m0 + r, i = n0 + r;
-    const float av = (b < ke && o < nout) ? dy[(int64_t)b * nout + o] : 0.0f;
-    const float bv = b < ke ? (i < nin ? x[(int64_t)b * nin + i] : (i == nin ? 1.0f : 0.0f))
-                            : 0.0f;
-    acc = mfma4(av, bv, acc);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    partial[((int64_t)s * Mp + m0 + 4 * q + j) * Np + n0 + r] = acc[j];
-}
-
-// dW[o][i] and db[o] from the slices' partial sums, in slice order.
-__global__ void k_lin_grad_reduce(const float* __restrict__ partial, int slices, int Mp, int Np,
-                                  int nin, int nout, float* __restrict__ dW,
-                                  float* __restrict__ db) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nout * (nin + 1)) return;
-  const int o = e / (nin + 1), i = e % (nin + 1);
+// grads[i] = the sum of the slices' i-th entries (eight interleaved chains,
+// added in order), then the Adam step where lr > 0; entry kParams is the
+// loss. 32 consecutive entries and 8 chains to a workgroup.
+__global__ __launch_bounds__(256) void k_train_update(
+    const float* __restrict__ partial, int slices, float* __restrict__ grads,
+    float* __restrict__ loss_out, float* __restrict__ p, float* __restrict__ m,
+    float* __restrict__ v, uint16_t* __restrict__ pbf, float lr, float b1, float b2, float eps,
+    float c1, float c2) {
+  __shared__ float s_sum[8][32];
+  const int c = threadIdx.x / 32, i = blockIdx.x * 32 + threadIdx.x % 32;
   float acc = 0.0f;
-  for (int s = 0; s < slices; ++s) acc += partial[((int64_t)s * Mp + o) * Np + i];
-  if (i < nin)
-    dW[o * nin + i] = acc;
-  else
-    db[o] = acc;
-}
-
-// Masked mean squared error: dy = 2 (y - t) mask / B, loss accumulated.
-// Masked Poisson NLL with rate 2^y (y clamped at 30): per element
-// m (2^y - t y ln 2) / B, gradient m (2^y - t) ln 2 / B.
-constexpr float kLn2 = 0.69314718055994531f;
-constexpr float kMaxLogRate = 30.0f;
-
-__global__ void k_poisson(const float* __restrict__ y, const float* __restrict__ t,
-                          const float* __restrict__ mask, int B, float* __restrict__ dy,
-                          float* __restrict__ loss) {
-  int e = blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.0f;
-  if (e < B * kOut) {
-    float m = mask[e];
-    float yc = fminf(y[e], kMaxLogRate);
-    float lam = exp2f(yc);
-    dy[e] = y[e] > kMaxLogRate ? 0.0f : m * (lam - t[e]) * kLn2 / (float)B;
-    l = m * (lam - t[e] * yc * kLn2) / (float)B;
+  if (i <= kParams) {
+#pragma unroll 4
+    for (int s = c; s < slices; s += 8) acc += partial[(int64_t)s * kSlice + i];
   }
-  l = wave_sum_f(l);
-  if (lane_id() == 0 && l != 0.0f) atomicAdd(loss, l);
-}
-
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ pbf, int n, float lr,
-                       float b1, float b2, float eps, float c1, float c2) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float gi = g[i];
-  float mi = b1 * m[i] + (1.0f - b1) * gi;
-  float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+  s_sum[c][threadIdx.x % 32] = acc;
+  __syncthreads();
+  if (c || i > kParams) return;
+  float gi = acc;
+#pragma unroll
+  for (int k = 1; k < 8; ++k) gi += s_sum[k][threadIdx.x];
+  if (i == kParams) {
+    if (loss_out) *loss_out = gi;
+    return;
+  }
+  grads[i] = gi;
+  if (!(lr > 0.0f)) return;
+  const float mi = b1 * m[i] + (1.0f - b1) * gi;
+  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
-  float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  float np = p[i] - upd;
+  const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  const float np = p[i] - upd;
   p[i] = np;
   pbf[i] = f32_to_bf16(np);
 }
@@ -505,12 +602,15 @@ int ygg_mlp_forward(const uint16_t* params_bf16, const float* features, int64_t 
   return YGG_OK;
 }
 
-// One training step on a batch: forward, masked MSE, backward, Adam.
-// ws: float workspace of ygg_mlp_train_workspace_floats(B) entries.
-int64_t ygg_mlp_train_workspace_floats(int64_t B) {
-  const int64_t slices = (B + kGradSlice - 1) / kGradSlice;
-  return (int64_t)B * (3 * kH + kOut) * 2 + kParams + 16 + slices * kH * (kH + 16);
+// Workgroups of k_train_grads, and so slices of partial sums, for a batch.
+static int64_t train_slices(int64_t B) {
+  const int64_t s = (B + kRows - 1) / kRows;
+  return s < kTrainBlocks ? s : kTrainBlocks;
 }
+
+// One training step on a batch: forward, masked Poisson loss, backward, Adam.
+// ws: float workspace of ygg_mlp_train_workspace_floats(B) entries.
+int64_t ygg_mlp_train_workspace_floats(int64_t B) { return train_slices(B) * kSlice; }
 
 int ygg_mlp_train_step(float* params, uint16_t* params_bf16, float* adam_m, float* adam_v,
                        int64_t step, float lr, const float* x, const float* target,
@@ -518,62 +618,15 @@ int ygg_mlp_train_step(float* params, uint16_t* params_bf16, float* adam_m, floa
                        float* loss_out, void* stream) {
   if (B64 < 1 || !params || !grads || !ws) return YGG_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
-  const int B = (int)B64;
-  float* a1 = ws;
-  float* a2 = a1 + (int64_t)B * kH;
-  float* a3 = a2 + (int64_t)B * kH;
-  float* yo = a3 + (int64_t)B * kH;
-  float* d1 = yo + (int64_t)B * kOut;
-  float* d2 = d1 + (int64_t)B * kH;
-  float* d3 = d2 + (int64_t)B * kH;
-  float* dyo = d3 + (int64_t)B * kH;
-  float* partial = dyo + (int64_t)B * kOut;  // weight-gradient slices
-  const uint16_t* W = params_bf16;
-  auto g = [](int64_t n) { return dim3(grid_for(n, 256)); };
-  // one wavefront per 16 batch rows
-  const dim3 gr(grid_for(((int64_t)B + 15) / 16 * YGG_WAVE, 256));
-  hipLaunchKernelGGL(k_lin_fwd, gr, dim3(256), 0, st, W + kOffW1, W + kOffB1, x, B, kIn, kH, 1,
-                     a1);
-  hipLaunchKernelGGL(k_lin_fwd, gr, dim3(256), 0, st, W + kOffW2, W + kOffB2, a1, B, kH, kH, 1,
-                     a2);
-  hipLaunchKernelGGL(k_lin_fwd, gr, dim3(256), 0, st, W + kOffW3, W + kOffB3, a2, B, kH, kH, 1,
-                     a3);
-  hipLaunchKernelGGL(k_lin_fwd, gr, dim3(256), 0, st, W + kOffW4, W + kOffB4, a3, B, kH, kOut, 0,
-                     yo);
-  if (loss_out) hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, st, (uint32_t*)loss_out, 1);
-  hipLaunchKernelGGL(k_poisson, g((int64_t)B * kOut), dim3(256), 0, st, yo, target, mask, B,
-                     dyo, loss_out);
-  const int slices = (B + kGradSlice - 1) / kGradSlice;
-  auto weight_grads = [&](const float* dy, const float* xin, int nin, int nout, float* dW,
-                          float* db) {
-    const int Mp = (nout + 15) / 16 * 16, Np = (nin + 1 + 15) / 16 * 16;
-    const int64_t waves = (int64_t)(Mp / 16) * (Np / 16) * slices;
-    hipLaunchKernelGGL(k_lin_bwd_weight, dim3(grid_for(waves * YGG_WAVE, 256)), dim3(256), 0, st,
-                       dy, xin, B, nin, nout, Mp, Np, partial);
-    hipLaunchKernelGGL(k_lin_grad_reduce, g((int64_t)nout * (nin + 1)), dim3(256), 0, st,
-                       partial, slices, Mp, Np, nin, nout, dW, db);
-  };
-  // layer 4
-  weight_grads(dyo, a3, kH, kOut, grads + kOffW4, grads + kOffB4);
-  hipLaunchKernelGGL(k_lin_bwd_data, gr, dim3(256), 0, st, W + kOffW4, dyo, a3, B, kH, kOut, 1,
-                     d3);
-  // layer 3
-  weight_grads(d3, a2, kH, kH, grads + kOffW3, grads + kOffB3);
-  hipLaunchKernelGGL(k_lin_bwd_data, gr, dim3(256), 0, st, W + kOffW3, d3, a2, B, kH, kH, 1, d2);
-  // layer 2
-  weight_grads(d2, a1, kH, kH, grads + kOffW2, grads + kOffB2);
-  hipLaunchKernelGGL(k_lin_bwd_data, gr, dim3(256), 0, st, W + kOffW2, d2, a1, B, kH, kH, 1, d1);
-  // layer 1
-  weight_grads(d1, x, kIn, kH, grads + kOffW1, grads + kOffB1);
+  const int slices = (int)train_slices(B64);
+  hipLaunchKernelGGL(k_train_grads, dim3(slices), dim3(256), 0, st, params_bf16, x, target, mask,
+                     B64, ws);
+  const float b1 = 0.9f, b2 = 0.999f;
+  const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
+  hipLaunchKernelGGL(k_train_update, dim3((kParams + 1 + 31) / 32), dim3(256), 0, st, ws, slices,
+                     grads, loss_out, params, adam_m, adam_v, params_bf16, lr, b1, b2, 1e-8f, c1,
+                     c2);
   YGG_LAUNCH_CHECK();
-  if (lr > 0.0f) {
-    const float b1 = 0.9f, b2 = 0.999f;
-    float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
-    hipLaunchKernelGGL(k_adam, g(kParams), dim3(256), 0, st, params, grads, adam_m, adam_v,
-                       params_bf16, kParams, lr, b1, b2, 1e-8f, c1, c2);
-    YGG_LAUNCH_CHECK();
-  }
-  (void)yo;
   return YGG_OK;
 }
 
