@@ -616,6 +616,13 @@ int ygg_near_dense_from_list(int64_t num_leaves, const int64_t* row_offsets,
 int ygg_mlp_num_params(void);
 int ygg_mlp_forward(const uint16_t* params_bf16, const float* features, int64_t n,
                     float* outputs, void* stream);
+/* The same with feature 4 (the parent's far count) made from first_outputs,
+ * an earlier pass's outputs for the same nodes: scale_far * 2^y[parent[k]][0]
+ * (0 for parent[k] < 0) in place of what `features` hold; the features of
+ * ygg_mlp_features with the counts of ygg_mlp_far_counts give the same. */
+int ygg_mlp_forward_parent(const uint16_t* params_bf16, const float* features, int64_t n,
+                           const int32_t* parent, const float* first_outputs, float scale_far,
+                           float* outputs, void* stream);
 int64_t ygg_mlp_train_workspace_floats(int64_t batch);
 /* One Adam step (lr > 0) or gradient only (lr == 0) of the masked Poisson
  * negative log-likelihood (rate 2^y, target = count / per-output scale) on a

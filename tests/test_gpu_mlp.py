@@ -72,6 +72,33 @@ def test_mlp_gradients_at_row_block_edges(B):
     assert torch.equal(tr.gradients(*dev), g) and float(tr.loss) == loss
 
 
+@pytest.mark.parametrize("T", [1, 15, 17, 512 * 4 * 16 + 7])
+def test_mlp_forward_parent_matches_two_step_features(T):
+    """Feature 4 made inside the kernel against the same feature written by
+    ygg_mlp_far_counts and log2 here (a tile's edges, and more tiles than one
+    round of the grid). exp2/log2 differ between the two in their last bits:
+    1e-5 covers 2^-20 of a feature times the layers' gains."""
+    from yggdrax_amd import _lib, learned
+    lib = _lib.load()
+    model = learned.CapacityModel(learned.init_params(3))
+    x, _, _ = _batch(T, 1)
+    rng = np.random.default_rng(T)
+    x = torch.from_numpy(x).cuda()
+    parent = torch.from_numpy(rng.integers(-1, T, T).astype(np.int32)).cuda()
+    y0 = torch.from_numpy(rng.normal(0, 4, (T, 3)).astype(np.float32)).cuda()
+    y0[0, 0] = 40.0  # past the clamp of the log2 rate
+    st = _lib.stream_ptr(x.device)
+    y = torch.empty_like(y0)
+    _lib.check(lib.ygg_mlp_forward_parent(
+        model.device_weights(x.device).data_ptr(), x.data_ptr(), T, parent.data_ptr(),
+        y0.data_ptr(), 2.5, y.data_ptr(), st), "forward parent")
+    far = torch.empty(T, device=x.device)
+    _lib.check(lib.ygg_mlp_far_counts(y0.data_ptr(), T, 2.5, far.data_ptr(), st), "far counts")
+    up = parent.clamp(min=0).long()
+    x[:, 4] = torch.where(parent >= 0, torch.log2(1.0 + far[up].double()) / 16.0, 0.0).float()
+    torch.testing.assert_close(y, model.forward(x), rtol=1e-5, atol=1e-5)
+
+
 def test_mlp_training_reduces_loss():
     from yggdrax_amd import learned
     rng = np.random.default_rng(0)

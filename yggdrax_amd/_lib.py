@@ -179,6 +179,7 @@ _SIGS = {
                          [_P] * 2 + [_I64] + [_P] * 3),
     "ygg_mlp_num_params": (_INT, []),
     "ygg_mlp_forward": (_INT, [_P, _P, _I64, _P, _P]),
+    "ygg_mlp_forward_parent": (_INT, [_P, _P, _I64, _P, _P, _F, _P, _P]),
     "ygg_mlp_train_workspace_floats": (_I64, [_I64]),
     "ygg_mlp_train_step": (_INT, [_P, _P, _P, _P, _I64, _F, _P, _P, _P, _I64, _P, _P, _P, _P]),
     "ygg_mlp_params_to_bf16": (_INT, [_P, _P, _P]),

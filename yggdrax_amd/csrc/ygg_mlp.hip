@@ -37,146 +37,224 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 
 // ---- inference on the matrix cores --------------------------------------
 // Each wavefront runs 16 samples at a time through the four layers with
-// 16x16x16 bf16 MFMAs (fp32 accumulate). Operand layouts of
-// v_mfma_f32_16x16x16_bf16 on wave64 (lane l, j = 0..3):
-//   A[m][k]: lane l holds A[l % 16][4 (l / 16) + j]
-//   B[k][n]: lane l holds B[4 (l / 16) + j][l % 16]
-//   D[m][n]: lane l holds D[4 (l / 16) + j][l % 16]
+// 16x16x32 bf16 MFMAs (fp32 accumulate). Operand layouts of
+// v_mfma_f32_16x16x32_bf16 on wave64 (lane l, q = l / 16):
+//   A[m][k]: lane l holds A[l % 16][8 q + j],  j = 0..7
+//   B[k][n]: lane l holds B[8 q + j][l % 16],  j = 0..7
+//   D[m][n]: lane l holds D[4 q + j][l % 16],  j = 0..3
 // With A = a 16-output slice of W (m = output, k = input) and B = the
-// activations (k = input feature, n = sample), a layer's D tile t is, lane
-// for lane, the B operand of k-step t of the next layer: no data moves
-// between layers. The weights are exactly bf16; each fp32 activation is
-// split into bf16 hi + lo (split_bf16) and both halves are multiplied, so
-// the products keep ~2^-16 relative accuracy and the outputs match fp32
-// arithmetic to ~1e-5. Weight fragments live in registers for the whole
-// kernel.
-typedef short bf16x4_t __attribute__((ext_vector_type(4)));
-#ifndef MLP_INFER_BLOCKS
-#define MLP_INFER_BLOCKS 256
-#endif
+// activations (k = input feature, n = sample), the D tiles 2s and 2s + 1 of
+// a layer are, lane for lane, the B operand of k-step s of the next one if
+// slot (q, j) stands for input 16 (2s + j / 4) + 4 q + j % 4 in A as well:
+// no data moves between layers. The weights are exactly bf16; each fp32
+// activation is split into bf16 hi + lo (split_bf16) and both halves are
+// multiplied, so the products keep 2^-17 relative accuracy and the outputs
+// match fp32 arithmetic to ~1e-5. The first layer's eight inputs take one
+// k-step for both halves (slots q = 0 the hi, q = 1 the lo parts).
+//
+// Bound by the chain of splits and MFMAs of a tile (about 220 vector
+// instructions and 40 MFMAs): 0.83 us per tile and SIMD with two or three
+// wavefronts. Weight fragments live in registers for the whole kernel,
+// gathered once through LDS (from global memory the gather had taken 10 us of
+// every call), biases in LDS. 524287 nodes take 29 us, against 97 us for the
+// 16x16x16 form (80 MFMAs, rounding in integer arithmetic, one wavefront per
+// SIMD); with 2 wavefronts per SIMD 31 us, with 4 (spilling) 36 us.
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef f32x4_t __attribute__((aligned(4))) f32x4_u;
+constexpr int kInferBlocks = 768;
 
-// hi = v truncated to bf16, so v - hi is exact in fp32; lo = that remainder
-// rounded to nearest even. |v - hi - lo| <= 2^-9 |v - hi| < 2^-16 |v|.
-__device__ __forceinline__ void split_bf16(const f32x4_t& v, bf16x4_t& hi, bf16x4_t& lo) {
+// hi = v rounded to bf16, so v - hi is exact in fp32; lo = that remainder
+// rounded: |v - hi - lo| <= 2^-9 |v - hi| <= 2^-18 |v|. Values 2 e and
+// 2 e + 1 go to word e.
+__device__ __forceinline__ void split_bf16(float v0, float v1, uint32_t& hi, uint32_t& lo) {
+  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+  const pair_t h = {(__bf16)v0, (__bf16)v1};
+  hi = __builtin_bit_cast(uint32_t, h);
+  asm("" : "+v"(hi));  // else v0 is converted again for its own remainder
+  const pair_t r = {(__bf16)(v0 - __uint_as_float(hi << 16)),
+                    (__bf16)(v1 - __uint_as_float(hi & 0xFFFF0000u))};
+  lo = __builtin_bit_cast(uint32_t, r);
+}
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t __attribute__((aligned(2))) u32_2b_t;  // two bf16 weights, aligned as one
+
+__device__ __forceinline__ f32x4_t mfma32(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// max(v, 0), 0 for NaN, at most the largest bfloat16: one instruction, where
+// fmaxf takes two (it quiets its operand first).
+__device__ __forceinline__ float relu(float v) {
+  return __builtin_amdgcn_fmed3f(v, 0.0f, __uint_as_float(0x7F7F0000u));
+}
+
+// One hidden layer: acc (the previous layer's four D tiles) becomes this
+// layer's, through ReLU and the split. k-steps run outermost, so consecutive
+// MFMAs write different accumulators.
+__device__ __forceinline__ void split_relu(const f32x4_t (&acc)[4], u32x4_t (&hi)[2],
+                                           u32x4_t (&lo)[2]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t u = __float_as_uint(v[j]);
-    hi[j] = (short)(u >> 16);
-    lo[j] = (short)f32_to_bf16(v[j] - __uint_as_float(u & 0xFFFF0000u));
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f32x4_t& v = acc[2 * s + e / 2];
+      uint32_t h, l;
+      split_bf16(relu(v[2 * (e % 2)]), relu(v[2 * (e % 2) + 1]), h, l);
+      hi[s][e] = h;
+      lo[s][e] = l;
+    }
+}
+
+template <class Bias>
+__device__ __forceinline__ void hidden_layer(const u32x4_t (&a)[4][2], Bias bias,
+                                             f32x4_t (&acc)[4]) {
+  u32x4_t hi[2], lo[2];
+  split_relu(acc, hi, lo);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = bias(t);
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = mfma32(a[t][s], hi[s], acc[t]);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = mfma32(a[t][s], lo[s], acc[t]);
   }
 }
 
-__device__ __forceinline__ f32x4_t relu4(f32x4_t v) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = fmaxf(v[j], 0.0f);
-  return v;
+// Log-scaled far count of a parent node (feature 4) from its predicted
+// log2 rate.
+__device__ __forceinline__ float far_feature(float far) {
+  return log2f(1.0f + fmaxf(far, 0.0f)) / 16.0f;
 }
 
-__global__ __launch_bounds__(256) void k_mlp_infer(const uint16_t* __restrict__ wbf,
-                                                   const float* __restrict__ x, int64_t n,
-                                                   float* __restrict__ y) {
+constexpr float kLn2 = 0.69314718055994531f;
+constexpr float kMaxLogRate = 30.0f;
+
+// PARENT: feature 4 of node k is not read from x but made from y0, the first
+// pass's outputs, at the node's parent (0 for a root), as k_mlp_far_of and
+// k_mlp_features make it.
+template <bool PARENT>
+__global__ __launch_bounds__(256, 3) void k_mlp_infer(const uint16_t* __restrict__ wbf,
+                                                      const float* __restrict__ x, int64_t n,
+                                                      const int32_t* __restrict__ parent,
+                                                      const float* __restrict__ y0, float s0,
+                                                      float* __restrict__ y) {
   const unsigned l = lane_id();
   const int r = (int)(l % 16), q = (int)(l / 16);
-  auto w = [&](int off) { return (short)wbf[off]; };
-  auto wf = [&](int off) { return bf16_to_f32(wbf[off]); };
-  bf16x4_t a1[4], a2[4][4], a3[4][4], a4[4];
-  f32x4_t b1[4], b2[4], b3[4], b4;
+  // The weights pass through LDS: one coalesced read per workgroup, then each
+  // lane gathers its fragments there. Rows of 64 are kept at a pitch of 68.
+  constexpr int kPitch = kH + 4;
+  __shared__ __align__(16) uint16_t s_w1[kH * kIn], s_w2[kH * kPitch], s_w3[kH * kPitch],
+      s_w4[kOut * kPitch];
+  __shared__ __align__(16) float s_b[3][kH];
+  for (int e = threadIdx.x; e < kH * kH / 2; e += 256) {
+    const int at = 2 * e / kH * kPitch + 2 * e % kH;
+    *(uint32_t*)(s_w2 + at) = *(const u32_2b_t*)(wbf + kOffW2 + 2 * e);
+    *(uint32_t*)(s_w3 + at) = *(const u32_2b_t*)(wbf + kOffW3 + 2 * e);
+  }
+  {
+    const int e = threadIdx.x;  // 256 threads = kH * kIn / 2
+    *(uint32_t*)(s_w1 + 2 * e) = *(const u32_2b_t*)(wbf + kOffW1 + 2 * e);
+    if (e < kOut * kH) s_w4[e / kH * kPitch + e % kH] = wbf[kOffW4 + e];
+    if (e < kH) {
+      s_b[0][e] = bf16_to_f32(wbf[kOffB1 + e]);
+      s_b[1][e] = bf16_to_f32(wbf[kOffB2 + e]);
+      s_b[2][e] = bf16_to_f32(wbf[kOffB3 + e]);
+    }
+  }
+  f32x4_t b4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float w4 = bf16_to_f32(wbf[kOffB4 + min(4 * q + e, kOut - 1)]);
+    b4[e] = 4 * q + e < kOut ? w4 : 0.0f;
+  }
+  __syncthreads();
+  u32x4_t a1[4], a2[4][2], a3[4][2], a4[2];
+  // slots (q, 0..3) and (q, 4..7) of k-step s: inputs 32 s + 4 q and
+  // 32 s + 16 + 4 q, four each
+  auto frag = [&](const uint16_t* row, int s) {
+    const uint2 lo = *(const uint2*)(row + 32 * s + 4 * q);
+    const uint2 hi = *(const uint2*)(row + 32 * s + 16 + 4 * q);
+    return u32x4_t{lo.x, lo.y, hi.x, hi.y};
+  };
+  constexpr u32x4_t kZero = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
+    const u32x4_t w1 = *(const u32x4_t*)(s_w1 + (16 * t + r) * kIn);
+    a1[t] = q < 2 ? w1 : kZero;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = 4 * q + j;
-      a1[t][j] = k < kIn ? w(kOffW1 + (16 * t + r) * kIn + k) : (short)0;
-      b1[t][j] = wf(kOffB1 + 16 * t + k);
-      b2[t][j] = wf(kOffB2 + 16 * t + k);
-      b3[t][j] = wf(kOffB3 + 16 * t + k);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        a2[t][kk][j] = w(kOffW2 + (16 * t + r) * kH + 16 * kk + k);
-        a3[t][kk][j] = w(kOffW3 + (16 * t + r) * kH + 16 * kk + k);
-      }
+    for (int s = 0; s < 2; ++s) {
+      a2[t][s] = frag(s_w2 + (16 * t + r) * kPitch, s);
+      a3[t][s] = frag(s_w3 + (16 * t + r) * kPitch, s);
     }
   }
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a4[kk][j] = r < kOut ? w(kOffW4 + r * kH + 16 * kk + 4 * q + j) : (short)0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) b4[j] = 4 * q + j < kOut ? wf(kOffB4 + 4 * q + j) : 0.0f;
+  for (int s = 0; s < 2; ++s) {
+    const u32x4_t w4 = frag(s_w4 + min(r, kOut - 1) * kPitch, s);
+    a4[s] = r < kOut ? w4 : kZero;
+  }
+  // biases stay in LDS (one 16-byte read per output tile): in registers they
+  // would cost the third wavefront
+  auto bias = [&](int layer, int t) { return *(const f32x4_t*)(&s_b[layer][16 * t + 4 * q]); };
 
   // Wave-uniform loop over 16-sample tiles (every lane reaches every
-  // MFMA). At one wavefront per SIMD nothing else hides a load, so the next
-  // tile's features are loaded while this tile runs.
+  // MFMA); the next tile's features are loaded while this one runs, by
+  // unconditional loads (a lane past the last sample reads that one and
+  // writes nothing; conditional loads had been a branch each).
   const int64_t tiles = (n + 15) / 16;
   const int64_t nw = (int64_t)gridDim.x * (blockDim.x / YGG_WAVE);
+  struct In {
+    f32x4_u f[2];
+  };
   auto load_tile = [&](int64_t tl) {
-    f32x4_t v;
-    const int64_t sm = tl * 16 + r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = 4 * q + j;
-      v[j] = (sm < n && k < kIn) ? x[sm * kIn + k] : 0.0f;
+    int64_t sm = tl * 16 + r;
+    sm = sm < n ? sm : n - 1;
+    In v;
+    v.f[0] = *(const f32x4_u*)(x + sm * kIn);
+    v.f[1] = *(const f32x4_u*)(x + sm * kIn + 4);
+    if (PARENT) {
+      const int32_t p = parent[sm];
+      const float far = s0 * exp2f(fminf(y0[kOut * (int64_t)max(p, 0)], kMaxLogRate));
+      v.f[1][0] = p >= 0 ? far_feature(far) : 0.0f;
     }
     return v;
   };
   int64_t tile = (int64_t)blockIdx.x * (blockDim.x / YGG_WAVE) + threadIdx.x / YGG_WAVE;
-  f32x4_t in_next = load_tile(tile);
+  if (tile >= tiles) return;
+  In in_next = load_tile(tile);
   for (; tile < tiles; tile += nw) {
-    const int64_t smp = tile * 16 + r;
-    const bool ok = smp < n;
-    const f32x4_t in = in_next;
+    const In in = in_next;
     if (tile + nw < tiles) in_next = load_tile(tile + nw);
-    // Every activation tile is split once and feeds the four output tiles;
-    // k-steps run outermost, so consecutive MFMAs write different
-    // accumulators and pipeline.
-    bf16x4_t hi[4], lo[4];
-    f32x4_t acc[4];
-    split_bf16(in, hi[0], lo[0]);
+    u32x4_t b;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1[t], hi[0], b1[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1[t], lo[0], acc[t], 0, 0, 0);
+    for (int e = 0; e < 4; ++e) {
+      uint32_t hi, lo;
+      split_bf16(in.f[e / 2][2 * (e % 2)], in.f[e / 2][2 * (e % 2) + 1], hi, lo);
+      b[e] = q == 0 ? hi : (q == 1 ? lo : 0u);
     }
+    f32x4_t acc[4];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) split_bf16(relu4(acc[kk]), hi[kk], lo[kk]);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = b2[t];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2[t][kk], hi[kk], acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2[t][kk], lo[kk], acc[t], 0, 0, 0);
-      }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) split_bf16(relu4(acc[kk]), hi[kk], lo[kk]);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = b3[t];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a3[t][kk], hi[kk], acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a3[t][kk], lo[kk], acc[t], 0, 0, 0);
-      }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) split_bf16(relu4(acc[kk]), hi[kk], lo[kk]);
+    for (int t = 0; t < 4; ++t) acc[t] = mfma32(a1[t], b, bias(0, t));
+    hidden_layer(a2, [&](int t) { return bias(1, t); }, acc);
+    hidden_layer(a3, [&](int t) { return bias(2, t); }, acc);
+    u32x4_t hi[2], lo[2];
+    split_relu(acc, hi, lo);
     f32x4_t out = b4;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      out = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a4[kk], hi[kk], out, 0, 0, 0);
-      out = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a4[kk], lo[kk], out, 0, 0, 0);
+    for (int s = 0; s < 2; ++s) {
+      out = mfma32(a4[s], hi[s], out);
+      out = mfma32(a4[s], lo[s], out);
     }
-    if (q == 0 && ok) {
+    const int64_t smp = tile * 16 + r;
+    if (q == 0 && smp < n) {
 #pragma unroll
       for (int j = 0; j < kOut; ++j) y[smp * kOut + j] = out[j];
     }
   }
 }
-
-constexpr float kLn2 = 0.69314718055994531f;
-constexpr float kMaxLogRate = 30.0f;
 
 // ---- training: one kernel for a batch's gradients, one for the update ----
 // k_train_grads: a workgroup takes kRows batch rows at a time through the
@@ -475,7 +553,7 @@ __device__ __forceinline__ void node_features(int k, int NI, const int32_t* __re
   o[1] = log2f(cnt) / 24.0f;
   o[2] = log2f(maxext[k] / root_ext) / 32.0f + 1.0f;
   o[3] = log2f(radius[k] / root_rad) / 32.0f + 1.0f;
-  o[4] = log2f(1.0f + fmaxf(pf, 0.0f)) / 16.0f;
+  o[4] = far_feature(pf);
   o[5] = log2f(1.0f + sib) / 24.0f;
   float rel = (cnt / fmaxf(vol, 1e-30f)) / ((float)(ranges[1] + 1) / fmaxf(root_vol, 1e-30f));
   o[6] = fminf(fmaxf(log2f(fmaxf(rel, 1e-30f)) / 64.0f, -1.0f), 1.0f);
@@ -589,15 +667,30 @@ extern "C" {
 
 int ygg_mlp_num_params(void) { return kParams; }
 
+// 16-sample tiles, four wavefronts per workgroup, at most kInferBlocks
+// workgroups: three wavefronts per SIMD (the kernel's occupancy), each
+// gathering the weight fragments once and then looping over many tiles.
+static dim3 infer_grid(int64_t n) {
+  return dim3(grid_for((n + 15) / 16, 256 / YGG_WAVE, kInferBlocks));
+}
+
 int ygg_mlp_forward(const uint16_t* params_bf16, const float* features, int64_t n,
                     float* outputs, void* stream) {
   if (n < 0 || !params_bf16) return YGG_ERR_ARG;
   if (n == 0) return YGG_OK;
-  // 16-sample tiles, four wavefronts per workgroup, at most 256 workgroups:
-  // one wavefront per SIMD (the kernel's occupancy), each loading the weight
-  // fragments once and then looping over many tiles
-  hipLaunchKernelGGL(k_mlp_infer, dim3(grid_for((n + 15) / 16, 256 / YGG_WAVE, MLP_INFER_BLOCKS)),
-                     dim3(256), 0, (hipStream_t)stream, params_bf16, features, n, outputs);
+  hipLaunchKernelGGL(k_mlp_infer<false>, infer_grid(n), dim3(256), 0, (hipStream_t)stream,
+                     params_bf16, features, n, nullptr, nullptr, 0.0f, outputs);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
+int ygg_mlp_forward_parent(const uint16_t* params_bf16, const float* features, int64_t n,
+                           const int32_t* parent, const float* first_outputs, float scale_far,
+                           float* outputs, void* stream) {
+  if (n < 0 || !params_bf16 || !parent || !first_outputs) return YGG_ERR_ARG;
+  if (n == 0) return YGG_OK;
+  hipLaunchKernelGGL(k_mlp_infer<true>, infer_grid(n), dim3(256), 0, (hipStream_t)stream,
+                     params_bf16, features, n, parent, first_outputs, scale_far, outputs);
   YGG_LAUNCH_CHECK();
   return YGG_OK;
 }

@@ -132,11 +132,14 @@ class CapacityModel:
         lib = _lib.load()
         dt = device_topology(tree)
         dev = geom.center.device
-        y0 = self.forward(features(dt, geom, None))
-        pf = torch.empty(dt.num_nodes, dtype=torch.float32, device=dev)
-        _lib.check(lib.ygg_mlp_far_counts(y0.data_ptr(), dt.num_nodes, float(self.scale[0]),
-                                          pf.data_ptr(), _lib.stream_ptr(dev)), "far counts")
-        return self.forward(features(dt, geom, pf))
+        x = features(dt, geom, None)
+        y0 = self.forward(x)
+        y = torch.empty_like(y0)
+        _lib.check(lib.ygg_mlp_forward_parent(
+            self.device_weights(dev).data_ptr(), x.data_ptr(), x.shape[0], dt.parent.data_ptr(),
+            y0.data_ptr(), float(self.scale[0]), y.data_ptr(), _lib.stream_ptr(dev)),
+            "mlp forward parent")
+        return y
 
     def predict_totals(self, tree, geom) -> np.ndarray:
         """Uncalibrated sums of the predicted rates (far, near, queue)."""
