@@ -140,6 +140,41 @@ def test_radix_sort_every_digit_width(ygg, key_bytes, range_bits, n, digit_bits)
     assert np.array_equal(out, keys[perm])
 
 
+@pytest.mark.parametrize("key_bytes,begin,end", [(8, 0, 63), (8, 0, 64), (8, 3, 20), (4, 0, 8),
+                                                 (4, 0, 32), (4, 5, 18)])
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 4096, 4097, 12288, 12289, 12288 * 9 + 1,
+                               4096 * 150 + 77])
+def test_radix_sort_at_path_edges(ygg, key_bytes, begin, end, n):
+    """The sort of one workgroup (up to 1024, 4096 and 12288 pairs), the first
+    size past it, and sorts of some ten to a few hundred tiles, whose look-back
+    starts with every tile unresolved: numpy's stable order of the keys' bits
+    [begin, end), with given values and all-ones keys among them (equal to
+    the padding of a partial workgroup)."""
+    from yggdrax_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(n + end)
+    dt = np.uint64 if key_bytes == 8 else np.uint32
+    keys = rng.integers(0, 1 << (8 * key_bytes), n, dtype=np.uint64, endpoint=False).astype(dt) \
+        if key_bytes == 4 else rng.integers(0, np.iinfo(np.uint64).max, n, dtype=np.uint64,
+                                            endpoint=True)
+    keys[rng.random(n) < 0.2] = np.iinfo(dt).max
+    keys[rng.random(n) < 0.3] &= dt(0xFFF)
+    if end < 8 * key_bytes:  # no bits past the sorted range
+        keys &= dt((1 << end) - 1)
+    vals = rng.permutation(n).astype(np.int32)
+    kt = torch.from_numpy(keys.view(np.int64 if key_bytes == 8 else np.int32)).cuda()
+    vt = torch.from_numpy(vals).cuda()
+    ko, vo = torch.empty_like(kt), torch.empty_like(vt)
+    fn = lib.ygg_sort_pairs_u64 if key_bytes == 8 else lib.ygg_sort_pairs_u32
+    ws = _lib.workspace(lib.ygg_sort_workspace_bytes(n, key_bytes, begin, end, 0), kt.device)
+    _lib.check(fn(kt.data_ptr(), vt.data_ptr(), ko.data_ptr(), vo.data_ptr(), n, begin, end, 0,
+                  ws.data_ptr(), ws.numel(), _lib.stream_ptr(kt.device)), "sort")
+    part = (keys >> dt(begin)) & dt((1 << (end - begin)) - 1)
+    perm = np.argsort(part, kind="stable")
+    assert np.array_equal(vo.cpu().numpy(), vals[perm])
+    assert np.array_equal(ko.cpu().numpy().view(dt), keys[perm])
+
+
 def test_identical_points_stable(ygg):
     """tests/unit/test_tree.py:193-214: identical points keep input order."""
     pos = np.full((64, 3), 0.25, np.float32)

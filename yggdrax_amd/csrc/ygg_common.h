@@ -92,13 +92,27 @@ __device__ __forceinline__ unsigned mbcnt64(uint64_t mask) {
 // Lanes of `peers` whose BITS-bit digit equals this lane's (BITS ballots).
 template <int BITS>
 __device__ __forceinline__ uint64_t wave_match_bits(unsigned d, uint64_t peers) {
+  uint32_t lo = (uint32_t)peers, hi = (uint32_t)(peers >> 32);
+  // Each bit as 0 or ~0; peers & ~(ballot ^ bit) is then one three-operand
+  // logic instruction per half: four instructions per bit instead of the
+  // eight of selecting the ballot or its complement. All ballots come first,
+  // so that none is used right after its compare (two wait states). 2^24
+  // Morton codes: 1042 us, 1134 us before this and the wider look-back.
+  int m[BITS];
+  uint64_t bal[BITS];
 #pragma unroll
   for (int b = 0; b < BITS; ++b) {
-    bool bit = (d >> b) & 1u;
-    uint64_t bal = __ballot(bit);
-    peers &= bit ? bal : ~bal;
+    m[b] = __builtin_amdgcn_sbfe((int)d, b, 1);
+    asm("" : "+v"(m[b]));  // keeps the extracted bit as the ballot's operand
   }
-  return peers;
+#pragma unroll
+  for (int b = 0; b < BITS; ++b) bal[b] = __ballot(m[b] != 0);
+#pragma unroll
+  for (int b = 0; b < BITS; ++b) {
+    lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)lo, (int)(uint32_t)bal[b], m[b], 0x90);
+    hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)hi, (int)(uint32_t)(bal[b] >> 32), m[b], 0x90);
+  }
+  return ((uint64_t)hi << 32) | lo;
 }
 
 template <int BITS>

@@ -10,6 +10,7 @@
 // data but more look-back words per tile (2^bits per pass) and more LDS;
 // the width is a parameter so callers (and the autotuner) can pick the
 // cheapest pass count for a key range.
+#include <algorithm>
 #include <type_traits>
 
 #include "ygg_common.h"
@@ -33,7 +34,7 @@ constexpr int kWaves = kSortThreads / YGG_WAVE;  // 4
 // take 512 threads (8192 keys) to fit LDS.
 // 64-bit keys with 9-bit digits (the 63-bit Morton codes: 7 passes) take
 // 1024 threads of 12 keys: 12288-key tiles (runs of ~24 keys per digit) in
-// 150 KB of LDS; 2^24 clustered codes sort in 1.17 ms against 1.30 ms with
+// 150 KB of LDS; 2^24 uniform codes sort in 1.04 ms against 1.29 ms with
 // 8-bit digits on 4096-key tiles.
 template <typename K, int BITS>
 constexpr int sort_threads() {
@@ -45,9 +46,18 @@ constexpr int sort_items() {
   return (sizeof(K) == 8 && BITS == 9) ? 12 : 16;
 }
 constexpr int kSortItems = 16;
+// A sort whose 12288-key tiles leave most CUs idle takes smaller ones (64-bit
+// keys with 9-bit digits: the Morton codes). gfx950, 63-bit keys, 7 passes:
+//   keys       2e4   1e5   3e5   1e6   2e6   6e6   2^24
+//   512 x 4     59    75   110   206   345   716   2158 us
+//   512 x 8     70    82   105   166   248   509   1426 us
+//   1024 x 12  111   124   139   190   223   398   1041 us
+constexpr int kMidThreads = 512, kMidItems = 8, kLowItems = 4;
+constexpr int64_t kMidSort = 3 << 19, kLowSort = 3 << 16;
 constexpr uint32_t kFlagAgg = 1u << 30;
 constexpr uint32_t kFlagPre = 2u << 30;
 constexpr uint32_t kCountMask = (1u << 30) - 1u;
+constexpr int kLookback = 8;
 
 constexpr int passes_for(int range_bits, int bits) { return (range_bits + bits - 1) / bits; }
 
@@ -92,19 +102,21 @@ __global__ __launch_bounds__(256) void k_digit_hist(const K* __restrict__ keys, 
     if (h[i]) atomicAdd(&hist[i], h[i]);
 }
 
-// In-place exclusive scan of each pass's 2^BITS-bin histogram (one block per
-// pass; thread t owns bins [t * D, t * D + D)).
+// Exclusive scan of each pass's 2^BITS-bin histogram, in place where both
+// arguments are the same (one block per pass; thread t owns bins
+// [t * D, t * D + D)).
 template <int BITS>
-__global__ __launch_bounds__(256) void k_hist_scan(uint32_t* hist) {
+__global__ __launch_bounds__(256) void k_hist_scan(const uint32_t* hist_in, uint32_t* hist) {
   constexpr int kBins = 1 << BITS;
   constexpr int D = kBins / kSortThreads;
   __shared__ uint32_t wsum[kWaves];
+  const uint32_t* hin = hist_in + (int64_t)blockIdx.x * kBins;
   uint32_t* h = hist + (int64_t)blockIdx.x * kBins;
   unsigned v[D];
   unsigned t = 0;
 #pragma unroll
   for (int j = 0; j < D; ++j) {
-    v[j] = h[threadIdx.x * D + j];
+    v[j] = hin[threadIdx.x * D + j];
     t += v[j];
   }
   unsigned inc = wave_inclusive_sum(t);
@@ -189,6 +201,7 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(const K* __restrict__ keys
                                                   Emit em, int64_t n,
                                                   int shift, const uint32_t* __restrict__ hist_scan,
                                                   uint32_t* __restrict__ lookback,
+                                                  uint32_t* __restrict__ lookback_next,
                                                   uint32_t* __restrict__ tile_counter,
                                                   const int64_t* __restrict__ n_dev) {
   constexpr int kBins = 1 << BITS;
@@ -225,6 +238,10 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(const K* __restrict__ keys
   __syncthreads();
   const int64_t tile = s_tile;
   const int64_t base = tile * kTile;
+  // The passes take two look-back buffers in turn; this one clears its
+  // tile's words of the other for the next.
+  if (lookback_next)
+    for (int i = tid; i < kBins; i += THREADS) lookback_next[tile * kBins + i] = 0u;
   // A device-side count (n_dev) shortens the sort to its first *n_dev keys:
   // tiles past it exit at once (tiles are claimed in order, and a tile looks
   // back only at earlier ones).
@@ -282,17 +299,36 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(const K* __restrict__ keys
     const unsigned d = (unsigned)tid * D + j;
     unsigned e = 0;
     if (owner && tile > 0) {
+      // Look back: the tile before, then, as long as only tile counts and no
+      // prefix are found, up to kLookback earlier tiles with one round trip.
+      // In a sort of a few hundred tiles all of them start together, and a
+      // one-tile chain costs about half a round trip per tile: 2^20 codes
+      // sort in 164 us, against 176 us with windows of one (2^24: 1042
+      // against 1058 us).
       int64_t pt = tile - 1;
-      while (true) {
-        uint32_t v = atomic_load_agent(&lookback[pt * kBins + d]);
-        uint32_t f = v & ~kCountMask;
-        if (f == 0) {
-          __builtin_amdgcn_s_sleep(1);
-          continue;
+      int width = 1;
+      bool found = false;
+      while (!found) {
+        uint32_t v[kLookback];
+#pragma unroll
+        for (int q = 0; q < kLookback; ++q)
+          v[q] = q < width && pt - q >= 0 ? atomic_load_agent(&lookback[(pt - q) * kBins + d]) : 0u;
+        int used = 0;
+        bool open = true;
+#pragma unroll
+        for (int q = 0; q < kLookback; ++q) {
+          const uint32_t f = v[q] & ~kCountMask;
+          open = open && f != 0;  // not yet published (or past the window): resume here
+          if (open) {
+            e += v[q] & kCountMask;
+            ++used;
+            found = f == kFlagPre;
+            open = !found;
+          }
         }
-        e += v & kCountMask;
-        if (f == kFlagPre) break;
-        --pt;
+        if (used == 0) __builtin_amdgcn_s_sleep(1);
+        pt -= used;
+        width = kLookback;
       }
       atomic_store_agent(&lb[d], kFlagPre | (e + tot[j]));
     }
@@ -343,6 +379,112 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(const K* __restrict__ keys
   for (int p = tid; p < valid; p += THREADS) em.val((int64_t)s_global[s_dig[p]] + p, s_vb[p]);
 }
 
+// The whole sort of at most THREADS * ITEMS pairs in one workgroup: the
+// pairs stay in LDS from the first 8-bit digit to the last. Wavefront w ranks
+// the pairs [w * 64 * ITEMS, ...) of the current order with ballot matches and
+// its own digit counters, as a tile of k_onesweep does. Slots past n hold
+// all-ones keys, which a stable sort keeps behind every pair.
+// Bound by the chain of a pass (match, count, scan, exchange), 1.6 us at 512
+// pairs and 7 us at 12288. 512 63-bit keys sort in 13 us and 4000 in 25 us,
+// against 38 and 50 us through k_onesweep; from 8000 on the GPU times are the
+// same (57 us), but one launch takes the host 4 us and ten take it 28 us.
+template <typename K, int THREADS, int ITEMS>
+__global__ __launch_bounds__(THREADS) void k_small_sort(const K* __restrict__ keys_in,
+                                                        const uint32_t* __restrict__ vals_in,
+                                                        K* __restrict__ keys_out,
+                                                        uint32_t* __restrict__ vals_out, int n,
+                                                        int begin_bit, int end_bit) {
+  constexpr int kBins = 256, kW = THREADS / YGG_WAVE, kCap = THREADS * ITEMS;
+  static_assert(THREADS >= kBins, "one thread per digit");
+  __shared__ K s_key[kCap];
+  __shared__ uint32_t s_val[kCap];
+  __shared__ uint16_t s_hist[kW][kBins];
+  __shared__ uint32_t s_start[kBins];
+  __shared__ uint32_t s_wsum[kBins / YGG_WAVE];
+  const int tid = threadIdx.x, w = tid / YGG_WAVE;
+  const unsigned lane = lane_id();
+  const int first = w * YGG_WAVE * ITEMS + (int)lane;
+  K key[ITEMS];
+  uint32_t val[ITEMS], rank[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = first + k * YGG_WAVE;
+    key[k] = i < n ? keys_in[i] : (K)~(K)0;
+    val[k] = i < n ? (vals_in ? vals_in[i] : (uint32_t)i) : 0u;
+  }
+  for (int shift = begin_bit; shift < end_bit; shift += 8) {
+    const unsigned mask = end_bit - shift < 8 ? (1u << (end_bit - shift)) - 1u : 255u;
+    for (int i = tid; i < kW * kBins; i += THREADS) (&s_hist[0][0])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      const unsigned d = (unsigned)(key[k] >> shift) & mask;
+      const uint64_t peers = wave_match_bits<8>(d, ~0ull);
+      const unsigned below = mbcnt64(peers);
+      const unsigned before = s_hist[w][d];
+      rank[k] = before + below;
+      if (below == 0) s_hist[w][d] = (uint16_t)(before + (unsigned)__popcll(peers));
+    }
+    __syncthreads();
+    unsigned total = 0, inc = 0;
+    if (tid < kBins) {
+      for (int q = 0; q < kW; ++q) {
+        const unsigned c = s_hist[q][tid];
+        s_hist[q][tid] = (uint16_t)total;  // exclusive prefix over waves
+        total += c;
+      }
+      inc = wave_inclusive_sum(total);
+      if (lane == 63) s_wsum[w] = inc;
+    }
+    __syncthreads();
+    if (tid < kBins) {
+      unsigned run = inc - total;
+      for (int q = 0; q < w; ++q) run += s_wsum[q];
+      s_start[tid] = run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      const unsigned d = (unsigned)(key[k] >> shift) & mask;
+      const unsigned pos = s_start[d] + s_hist[w][d] + rank[k];
+      s_key[pos] = key[k];
+      s_val[pos] = val[k];
+    }
+    __syncthreads();
+    if (shift + 8 < end_bit) {
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        key[k] = s_key[first + k * YGG_WAVE];
+        val[k] = s_val[first + k * YGG_WAVE];
+      }
+    }
+  }
+  for (int i = tid; i < n; i += THREADS) {
+    keys_out[i] = s_key[i];
+    vals_out[i] = s_val[i];
+  }
+}
+
+// Largest sort that one workgroup takes (k_small_sort): 12288 64-bit keys and
+// their values fill 152 KB of LDS.
+constexpr int64_t kSmallSort = 12288;
+
+template <typename K>
+static int small_sort(const K* keys_in, const uint32_t* vals_in, K* keys_out, uint32_t* vals_out,
+                      int64_t n, int begin_bit, int end_bit, hipStream_t st) {
+  if (n <= 1024)
+    hipLaunchKernelGGL((k_small_sort<K, 256, 4>), dim3(1), dim3(256), 0, st, keys_in, vals_in,
+                       keys_out, vals_out, (int)n, begin_bit, end_bit);
+  else if (n <= 4096)
+    hipLaunchKernelGGL((k_small_sort<K, 1024, 4>), dim3(1), dim3(1024), 0, st, keys_in, vals_in,
+                       keys_out, vals_out, (int)n, begin_bit, end_bit);
+  else
+    hipLaunchKernelGGL((k_small_sort<K, 1024, 12>), dim3(1), dim3(1024), 0, st, keys_in, vals_in,
+                       keys_out, vals_out, (int)n, begin_bit, end_bit);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -369,7 +511,14 @@ int fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t st) {
   return YGG_OK;
 }
 
-static inline int64_t tile_keys(int key_bytes, int digit_bits) {
+// Whether a sort of n pairs takes a smaller tile than its kind's (64-bit
+// keys with 9-bit digits only).
+static inline bool mid_sort(int64_t n, int key_bytes, int digit_bits) {
+  return key_bytes == 8 && digit_bits == 9 && n <= kMidSort;
+}
+
+static inline int64_t tile_keys(int64_t n, int key_bytes, int digit_bits) {
+  if (mid_sort(n, key_bytes, digit_bits)) return kMidThreads * (n <= kLowSort ? kLowItems : kMidItems);
   const int threads =
       key_bytes == 4 ? (digit_bits == 9 || digit_bits == 10 ? 1024 : (digit_bits >= 11 ? 512 : 256))
                      : (digit_bits == 9 ? 1024 : 256);
@@ -377,7 +526,7 @@ static inline int64_t tile_keys(int key_bytes, int digit_bits) {
   return (int64_t)threads * items;
 }
 static inline int64_t num_tiles(int64_t n, int key_bytes, int digit_bits) {
-  const int64_t t = tile_keys(key_bytes, digit_bits);
+  const int64_t t = tile_keys(n, key_bytes, digit_bits);
   return (n + t - 1) / t;
 }
 
@@ -409,41 +558,43 @@ size_t sort_workspace_bytes(int64_t n, int key_bytes, int range_bits, int digit_
   a.take<char>((size_t)n * key_bytes);                              // alternate keys
   a.take<uint32_t>((size_t)n);                                      // alternate values
   a.take<uint32_t>((size_t)passes * bins);                          // histograms
-  a.take<uint32_t>((size_t)passes + (size_t)passes * t * bins);     // counters + look-back
+  // tile counters + look-back (two buffers in use; the narrower kinds keep
+  // room for every pass, as a workspace sized for one of them is also used
+  // for another)
+  const size_t buffers = mid_sort(n, key_bytes, digit_bits) ? 2 : (size_t)passes;
+  a.take<uint32_t>((size_t)passes + buffers * t * bins);
   return a.off;
 }
 
-template <typename K, int BITS, typename Last = EmitKV<K>>
+template <typename K, int BITS, typename Last = EmitKV<K>, int kThreads = sort_threads<K, BITS>(),
+          int kItems = sort_items<K, BITS>()>
 static int sort_pairs_bits(const K* keys_in, const uint32_t* vals_in, K* keys_out,
                            uint32_t* vals_out, int64_t n, int begin_bit, int end_bit, void* ws,
                            size_t ws_bytes, hipStream_t st, const uint32_t* hist_pre,
                            const Last* last = nullptr, const int64_t* n_dev = nullptr) {
   constexpr int kBins = 1 << BITS;
-  constexpr int kThreads = sort_threads<K, BITS>();
-  constexpr int kItems = sort_items<K, BITS>();
   const int passes = passes_for(end_bit - begin_bit, BITS);
   const int64_t tiles = num_tiles(n, (int)sizeof(K), BITS);
-  if (tile_keys((int)sizeof(K), BITS) != (int64_t)kThreads * kItems) return YGG_ERR_ARG;
+  if (tile_keys(n, (int)sizeof(K), BITS) != (int64_t)kThreads * kItems) return YGG_ERR_ARG;
   Arena a(ws, ws_bytes);
   K* kalt = (K*)a.take<char>((size_t)n * sizeof(K));
   uint32_t* valt = a.take<uint32_t>((size_t)n);
-  uint32_t* hist = a.take<uint32_t>((size_t)passes * kBins);
-  uint32_t* ctr = a.take<uint32_t>((size_t)passes + (size_t)passes * tiles * kBins);
-  if (!kalt || !valt || !hist || !ctr) return YGG_ERR_WORKSPACE;
-  uint32_t* lookback = ctr + passes;
-  int rc = fill_u32(ctr, 0u, (int64_t)passes + (int64_t)passes * tiles * kBins, st);
+  const size_t hist_words = (size_t)passes * kBins, ctr_words = (size_t)passes,
+               lb_words = (size_t)tiles * kBins;
+  uint32_t* hist = a.take<uint32_t>(hist_words + ctr_words + (passes > 1 ? 2 : 1) * lb_words);
+  if (!kalt || !valt || !hist) return YGG_ERR_WORKSPACE;
+  uint32_t* ctr = hist + hist_words;
+  uint32_t* lookback[2] = {ctr + ctr_words, ctr + ctr_words + lb_words};
+  // one fill: histograms, tile counters, the first pass's look-back words
+  int rc = fill_u32(hist, 0u, (int64_t)(hist_words + ctr_words + lb_words), st);
   if (rc) return rc;
-  if (hist_pre) {
-    rc = copy_u32(hist, hist_pre, (int64_t)passes * kBins, st);
-    if (rc) return rc;
-  } else {
-    rc = fill_u32(hist, 0u, (int64_t)passes * kBins, st);
-    if (rc) return rc;
+  if (!hist_pre) {
     hipLaunchKernelGGL((k_digit_hist<K, BITS>), dim3(grid_for(n, 256, 2048)), dim3(256), 0, st,
                        keys_in, n, begin_bit, end_bit, passes, hist, n_dev);
     YGG_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_hist_scan<BITS>, dim3(passes), dim3(256), 0, st, hist);
+  hipLaunchKernelGGL(k_hist_scan<BITS>, dim3(passes), dim3(256), 0, st, hist_pre ? hist_pre : hist,
+                     hist);
   YGG_LAUNCH_CHECK();
   const K* src_k = keys_in;
   const uint32_t* src_v = vals_in;
@@ -451,15 +602,16 @@ static int sort_pairs_bits(const K* keys_in, const uint32_t* vals_in, K* keys_ou
     bool to_out = ((passes - 1 - p) % 2) == 0;
     K* dk = to_out ? keys_out : kalt;
     uint32_t* dv = to_out ? vals_out : valt;
+    uint32_t* next = p + 1 < passes ? lookback[(p + 1) % 2] : nullptr;
     if (last && p == passes - 1) {
       hipLaunchKernelGGL((k_onesweep<K, BITS, kItems, kThreads, Last>), dim3((unsigned)tiles),
                          dim3(kThreads), 0, st, src_k, src_v, *last, n, begin_bit + BITS * p,
-                         hist + p * kBins, lookback + (int64_t)p * tiles * kBins, ctr + p, n_dev);
+                         hist + p * kBins, lookback[p % 2], next, ctr + p, n_dev);
     } else {
       hipLaunchKernelGGL((k_onesweep<K, BITS, kItems, kThreads, EmitKV<K>>), dim3((unsigned)tiles),
                          dim3(kThreads), 0, st, src_k, src_v, EmitKV<K>{dk, dv}, n,
-                         begin_bit + BITS * p, hist + p * kBins,
-                         lookback + (int64_t)p * tiles * kBins, ctr + p, n_dev);
+                         begin_bit + BITS * p, hist + p * kBins, lookback[p % 2], next, ctr + p,
+                         n_dev);
     }
     YGG_LAUNCH_CHECK();
     src_k = dk;
@@ -546,11 +698,31 @@ static int sort_pairs_impl(const K* keys_in, const uint32_t* vals_in, K* keys_ou
       end_bit > 8 * (int)sizeof(K))
     return YGG_ERR_ARG;
   if (digit_bits == 0) digit_bits = default_digit_bits((int)sizeof(K), end_bit - begin_bit);
+  if (digit_bits < 8 || digit_bits > kMaxDigitBits) return YGG_ERR_ARG;
+  if (ws_bytes < sort_workspace_bytes(n, (int)sizeof(K), end_bit - begin_bit, digit_bits))
+    return YGG_ERR_WORKSPACE;
+  if (n <= kSmallSort) {
+    // the bits that whole digits of the requested width cover, as the passes
+    // below take them (keys have no bits past end_bit by contract)
+    const int bits = passes_for(end_bit - begin_bit, digit_bits) * digit_bits;
+    const int end = std::min(begin_bit + bits, 8 * (int)sizeof(K));
+    return small_sort<K>(keys_in, vals_in, keys_out, vals_out, n, begin_bit, end, st);
+  }
   switch (digit_bits) {
     case 8:
       return sort_pairs_bits<K, 8>(keys_in, vals_in, keys_out, vals_out, n, begin_bit, end_bit,
                                    ws, ws_bytes, st, hist_pre);
     case 9:
+      if constexpr (sizeof(K) == 8) {
+        if (n <= kLowSort)
+          return sort_pairs_bits<K, 9, EmitKV<K>, kMidThreads, kLowItems>(
+              keys_in, vals_in, keys_out, vals_out, n, begin_bit, end_bit, ws, ws_bytes, st,
+              hist_pre);
+        if (n <= kMidSort)
+          return sort_pairs_bits<K, 9, EmitKV<K>, kMidThreads, kMidItems>(
+              keys_in, vals_in, keys_out, vals_out, n, begin_bit, end_bit, ws, ws_bytes, st,
+              hist_pre);
+      }
       return sort_pairs_bits<K, 9>(keys_in, vals_in, keys_out, vals_out, n, begin_bit, end_bit,
                                    ws, ws_bytes, st, hist_pre);
     case 10:
