@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void k_b_bounds(Seg sg, const float* __restric
 }
 
 // ---- Morton encode with per-system bounds + the code sort's histograms ----
-__global__ __launch_bounds__(256) void k_b_encode_hist(Seg sg, const float* __restrict__ pos,
+__global__ __launch_bounds__(kEncodeThreads) void k_b_encode_hist(Seg sg, const float* __restrict__ pos,
                                                        int64_t N, const float* __restrict__ b6,
                                                        uint64_t* __restrict__ codes,
                                                        uint32_t* __restrict__ hist) {
@@ -619,8 +619,8 @@ int ygg_batch_morton_sort(const YggBatch* b, const float* pos, const float* boun
   char* sws = a.take<char>(rest);
   if (!codes || !hist || !c1 || !i1 || !sk || !sk2 || !sws) return YGG_ERR_WORKSPACE;
   if ((rc = fill_u32(hist, 0u, kMortonHistWords, st))) return rc;
-  hipLaunchKernelGGL(k_b_encode_hist, dim3(grid_for(N, 256, 4096)), dim3(256), 0, st, sg, pos, N,
-                     bounds6, codes, hist);
+  hipLaunchKernelGGL(k_b_encode_hist, dim3(grid_for(N, kEncodeThreads, kEncodeBlocks)),
+                     dim3(kEncodeThreads), 0, st, sg, pos, N, bounds6, codes, hist);
   YGG_LAUNCH_CHECK();
   if ((rc = sort_pairs_u64(codes, nullptr, c1, i1, N, 0, kMortonEndBit, sws, rest, st, hist,
                             kMortonDigitBits))) return rc;

@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void k_encode(const float* __restrict__ pos, i
 }
 
 // Encode and count all eight 8-bit digit histograms of the codes.
-__global__ __launch_bounds__(256) void k_encode_hist(const float* __restrict__ pos, int64_t n,
+__global__ __launch_bounds__(kEncodeThreads) void k_encode_hist(const float* __restrict__ pos, int64_t n,
                                                      const float* __restrict__ b6,
                                                      uint64_t* __restrict__ codes,
                                                      uint32_t* __restrict__ hist) {
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void k_reorder(const float* __restrict__ pos,
 // Encode + digit histograms (as k_encode_hist) that also packs (x, y, z, m)
 // into one float4 per particle, so the later reorder gathers one 16-byte
 // record (one cache line) per particle instead of two.
-__global__ __launch_bounds__(256) void k_encode_hist_pack(const float* __restrict__ pos,
+__global__ __launch_bounds__(kEncodeThreads) void k_encode_hist_pack(const float* __restrict__ pos,
                                                           const float* __restrict__ mass,
                                                           int64_t n, const float* __restrict__ b6,
                                                           uint64_t* __restrict__ codes,
@@ -682,8 +682,8 @@ int ygg_morton_sort(const float* pos, int64_t n, const float* bounds6, uint64_t*
   if (!codes || !hist || !sws) return YGG_ERR_WORKSPACE;
   int rc = fill_u32(hist, 0u, kMortonHistWords, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_encode_hist, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, pos, n,
-                     bounds6, codes, hist);
+  hipLaunchKernelGGL(k_encode_hist, dim3(grid_for(n, kEncodeThreads, kEncodeBlocks)),
+                     dim3(kEncodeThreads), 0, st, pos, n, bounds6, codes, hist);
   YGG_LAUNCH_CHECK();
   return sort_pairs_u64(codes, nullptr, sorted_codes, perm, n, 0, kMortonEndBit, sws, rest, st, hist,
                         kMortonDigitBits);
@@ -744,8 +744,8 @@ static int morton_sort_pack(const float* pos, const float* mass, int64_t n, cons
   if (!packed || !codes || !hist || !sws) return YGG_ERR_WORKSPACE;
   int rc = fill_u32(hist, 0u, kMortonHistWords, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_encode_hist_pack, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, pos,
-                     mass, n, bounds6, codes, hist, packed);
+  hipLaunchKernelGGL(k_encode_hist_pack, dim3(grid_for(n, kEncodeThreads, kEncodeBlocks)),
+                     dim3(kEncodeThreads), 0, st, pos, mass, n, bounds6, codes, hist, packed);
   YGG_LAUNCH_CHECK();
   if ((rc = sort_pairs_u64(codes, nullptr, sorted_codes, perm, n, 0, kMortonEndBit, sws, rest, st, hist,
                         kMortonDigitBits)))

@@ -40,6 +40,14 @@ constexpr int kMortonPasses = (kMortonEndBit + kMortonDigitBits - 1) / kMortonDi
 constexpr int kMortonBins = 1 << kMortonDigitBits;
 constexpr int kMortonHistWords = kMortonPasses * kMortonBins;
 
+// Workgroups of the encode kernels: every workgroup ends by adding its
+// histogram words (up to 3584) to the same addresses, so few large ones: two
+// of 1024 threads per CU at most. 2^20 points take 21 us and 3e6 take 38 us,
+// against 87 and 89 us with up to 4096 workgroups of 256 (2^24: 173 against
+// 164 us).
+constexpr int kEncodeThreads = 1024;
+constexpr int kEncodeBlocks = 512;
+
 // Digit histograms of one code for every Morton sort pass: plain LDS
 // atomics for the low passes, ballot aggregation for the two top passes,
 // whose digits repeat within a cluster.
