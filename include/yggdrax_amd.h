@@ -491,7 +491,9 @@ typedef struct YggFlatWalkParams {
   uint64_t* gen_fill;         /* optional, emission walk only: [max_generations *
                                  YGG_WALK_GEN_RECORD_WORDS] per-generation records (entry counts
                                  far << 32 | near, and the stream offsets the generation starts
-                                 at), which make the walk resumable.
+                                 at), which make the walk resumable. (The upper half of the
+                                 records also holds words by which workgroups of one launch pass
+                                 small generations to each other.)
                                  Generation g writes after generations 0..g-1 and runs only if two
                                  entries per pair fit the remaining far and near capacity; if not,
                                  it writes nothing, flags[3] = g + 1, *num_generations = g, the

@@ -2,8 +2,10 @@
 profile (ygg_walk_flat's gen_pairs_hint): a profile only sizes the grids
 and the first batch of launches, so the lists stay those of the oracle
 with no profile, with the true profile, and with a profile that is far
-too small (every generation then runs on the 256-workgroup floor) or too
-short (generations past it launch from the bound alone)."""
+too small (one workgroup then runs every generation) or too short
+(generations past it launch from the bound alone), or names every third
+generation a large one (launches between generations that one launch runs
+together)."""
 
 from __future__ import annotations
 
@@ -33,7 +35,7 @@ def case():
     return ygg, tree, geom, rint, rnb
 
 
-@pytest.mark.parametrize("profile", ["none", "true", "tiny", "short"])
+@pytest.mark.parametrize("profile", ["none", "true", "tiny", "short", "mixed"])
 def test_walk_profile_keeps_the_lists(case, monkeypatch, profile):
     from yggdrax_amd import interactions as I
     ygg, tree, geom, rint, rnb = case
@@ -49,6 +51,9 @@ def test_walk_profile_keeps_the_lists(case, monkeypatch, profile):
         if profile == "tiny":
             for k in range(len(prof)):
                 arr[k] = 1
+        elif profile == "mixed":
+            for k in range(0, len(prof), 3):
+                arr[k] = 1 << 24
         elif profile == "short":
             for k in range(len(prof) // 3, len(prof)):
                 arr[k] = 0xFFFFFFFF

@@ -17,6 +17,8 @@
 #include "ygg_common.h"
 #include "ygg_walk.h"
 
+#include <algorithm>
+
 namespace ygg {
 
 constexpr int kFlatThreads = 256;
@@ -81,6 +83,452 @@ __device__ __forceinline__ unsigned long long wave_incl_u64(unsigned long long v
   return v;
 }
 
+// A workgroup's LDS for one chunk.
+//
+// Output staging. Each wavefront's outputs of one chunk occupy one
+// contiguous range of each stream (slots follow the block scan), so they
+// are gathered in LDS and written out by consecutive lanes. A pair yields
+// at most two far or two near entries: 2 * 64 * kFlatPer slots hold both
+// (far first, then near). Child pairs (up to four per pair) go through the
+// same buffer in rounds of kStage.
+// Writes that nobody reads (a pair with no output of that kind, a child
+// outside the current round) go to two spare slots past the range, so
+// every pair writes the same number of slots and the staging has no
+// per-pair branches.
+template <int kFlatPer, bool TAGS, int THREADS = kFlatThreads>
+struct WalkShared {
+  static constexpr int kStage = 2 * YGG_WAVE * kFlatPer;
+  unsigned long long wave[THREADS / YGG_WAVE];
+  unsigned long long base[3];
+  unsigned long long gbase[2];
+  int stop;
+  uint2 stage[THREADS / YGG_WAVE][kStage + 2];
+  int32_t tag[THREADS / YGG_WAVE][TAGS ? kStage : 1];
+};
+
+// How a chunk's workgroup works: one launch per generation (kLaunched), or
+// one of k_walk_persist's workgroups, beside others (kShared) or alone with
+// the whole generation (kAlone).
+enum WalkMode { kLaunched, kShared, kAlone };
+
+// A generation that one workgroup runs alone: its pairs lie in LDS (from_lds)
+// or in the queue, its children go to LDS where `fits` allows.
+struct AloneState {
+  uint64_t* pairs;  // LDS, THREADS * kFlatPer words
+  bool from_lds;
+  bool more;        // another generation of this launch may follow
+  unsigned long long bf, bn;  // stream offsets of the generation (the reserving threads)
+};
+
+// Evaluates pairs [chunk, chunk + THREADS * kFlatPer) of generation g and writes
+// their children and entries. In k_walk_persist the queues pass between
+// workgroups of the same launch, so their words go through agent-scope loads
+// and stores and have arrived when this returns; the generation's stream
+// offsets and the capacity check are taken here, beside the loads of the
+// pairs (false: the walk pauses at g and nothing was written). `children` is
+// the chunk's child count. Alone, nothing is reserved: counts and offsets are
+// this workgroup's own, and are stored for the generations after it.
+template <bool EMIT, int kFlatPer, bool TAGS, WalkMode MODE, int THREADS>
+__device__ __forceinline__ bool walk_chunk(const FlatArgs& a, const int g, const int64_t size,
+                                           const int64_t chunk,
+                                           WalkShared<kFlatPer, TAGS, THREADS>& sh,
+                                           const bool spread, unsigned long long& acc_f,
+                                           unsigned long long& acc_n, unsigned& children,
+                                           AloneState* alone = nullptr) {
+  constexpr bool PERSIST = MODE != kLaunched;
+  const uint64_t* __restrict__ wf_in = (g & 1) ? a.wf1 : a.wf0;
+  uint64_t* __restrict__ wf_out = (g & 1) ? a.wf0 : a.wf1;
+  const NodeRec* __restrict__ nodes = a.nodes;
+  const unsigned lane = lane_id();
+  const int w = threadIdx.x / YGG_WAVE;
+  constexpr int kStage = WalkShared<kFlatPer, TAGS>::kStage;
+  constexpr unsigned kDump = kStage;
+  // Two threads of different wavefronts reserve a chunk's output, so that
+  // their round trips overlap: one the children, the other the entries.
+  const bool for_children = threadIdx.x == 0, for_entries = threadIdx.x == YGG_WAVE;
+  unsigned long long rec_c = 0, rec_f = 0, rec_n = 0;  // generation g - 1's record (those two)
+  if (PERSIST && (for_children || for_entries) && g > 0 &&
+      !(MODE == kAlone && alone->from_lds)) {
+    const unsigned long long* r = a.gen_fill + (size_t)(g - 1) * kGenRecWords;
+    rec_c = atomic_load_agent(&r[0]);
+    rec_f = atomic_load_agent(&r[1]);
+    rec_n = atomic_load_agent(&r[2]);
+  }
+  // mode: 0 none, 1 accept, 2 near, 3 both-same, 4 both-cross, 5 split t, 6 split s
+  int mode[kFlatPer];
+  uint32_t pt[kFlatPer], ps[kFlatPer], x0[kFlatPer], x1[kFlatPer], x2[kFlatPer],
+      x3[kFlatPer];
+  unsigned nc = 0, nf = 0, nn = 0;
+  // Memory first, decisions after: every pair word of the chunk, then the
+  // node records of a group of four pairs, are loaded before any of them
+  // is used, so their latencies overlap instead of adding up pair by pair
+  // (a lane past the wavefront's end loads node 0 and decides nothing).
+  // Measured on the 2^24 clustered walk at 8 pairs per thread: 7.8 ms with
+  // the loads issued pair by pair, 6.9 ms with groups of two when the
+  // decisions branched per pair; with branch-free decisions 6.20 ms with
+  // groups of two, 6.13 ms with four (151 VGPRs, still 3 waves per SIMD)
+  // and 7.38 ms with eight (2 waves per SIMD).
+  constexpr uint64_t kNoPair = ~0ull;
+  uint64_t prw[kFlatPer];
+#pragma unroll
+  for (int k = 0; k < kFlatPer; ++k) {
+    const int64_t idx = chunk + k * THREADS + threadIdx.x;
+    if (MODE == kAlone && alone->from_lds)
+      prw[k] = idx < size ? alone->pairs[idx] : kNoPair;
+    else
+      prw[k] = idx < size ? (PERSIST ? atomic_load_agent(&wf_in[idx]) : wf_in[idx]) : kNoPair;
+  }
+  constexpr int kGroup = kFlatPer < 4 ? kFlatPer : 4;
+#pragma unroll
+  for (int k0 = 0; k0 < kFlatPer; k0 += kGroup) {
+  NodeRec rt[kGroup], rs[kGroup];
+#pragma unroll
+  for (int j = 0; j < kGroup; ++j) {
+    const uint64_t pr = prw[k0 + j];
+    const bool valid = pr != kNoPair;
+    rt[j] = nodes[valid ? (int32_t)(pr >> 32) : 0];
+    rs[j] = nodes[valid ? (int32_t)(uint32_t)pr : 0];
+  }
+#pragma unroll
+  for (int j = 0; j < kGroup; ++j) {
+    const int k = k0 + j;
+    mode[k] = 0;
+    const bool pvalid = prw[k] != kNoPair;
+    if (TAGS && !pvalid) continue;
+    const uint64_t pr = prw[k];
+    const int32_t t = (int32_t)(pr >> 32), s = (int32_t)(uint32_t)pr;
+    const NodeRec& nt = rt[j];
+    const NodeRec& ns = rs[j];
+    float dx = nt.cx - ns.cx, dy = nt.cy - ns.cy, dz = nt.cz - ns.cz;
+    float d2 = dx * dx;
+    d2 = d2 + dy * dy;
+    d2 = d2 + dz * dz;
+    const float et = nt.ext, es = ns.ext;
+    const bool diff = t != s;
+    bool ok;
+    if (a.mac_type == YGG_MAC_ENGBLOM) {
+      float rb = fmaxf(et, es), rs = fminf(et, es);
+      float lhs = rb + a.theta_root * rs;
+      ok = diff && d2 > 0.0f && (lhs * lhs <= a.theta_sq * d2);
+    } else {
+      float sum = et + es;
+      ok = diff && d2 > 0.0f && (sum * sum <= a.theta_sq * d2);
+    }
+    // internal nodes carry children (node ids of a forest are not
+    // split at num_internal)
+    const bool t_int = nt.left >= 0, s_int = ns.left >= 0;
+    if (a.node_hist && g == a.hist_gen && pvalid) atomicAdd(&a.node_hist[t], 1);
+    pt[k] = (uint32_t)t;
+    ps[k] = (uint32_t)s;
+    // accept / near rules (uniform per launch): the built-in MAC with
+    // near leaf pairs unless a policy descriptor says otherwise
+    bool acc = ok;
+    if (a.policy.accept == YGG_ACCEPT_DISTANCE)
+      acc = diff && d2 >= a.policy.accept_dist_sq;
+    else if (a.policy.accept == YGG_ACCEPT_DIFFERENT)
+      acc = diff;
+    else if (a.policy.accept == YGG_ACCEPT_NEVER)
+      acc = false;
+    const bool near_rule = a.policy.near == YGG_NEAR_LEAF_PAIRS;
+    const unsigned per_pair = !TAGS && a.pair_records ? 1u : 2u;  // stream slots
+    if (!TAGS) {
+      // Every field from selects, with no per-pair branch: accept (1),
+      // near (2) or a split (3 both of the same node, 4 both, 5 t only,
+      // 6 s only); nothing for a lane past the wavefront's end. On the
+      // 2^24 clustered walk the branching form took 6.88 ms, this one
+      // 6.21 ms (fewer exec-mask updates, 139 instead of 155 VGPRs).
+      const bool fa = pvalid && acc;
+      const bool fn = pvalid && !acc && near_rule && !t_int && !s_int && diff;
+      const bool same = !diff;
+      const bool split_t = t_int && (same || !s_int || et >= es);
+      const bool split_s = s_int && (same || !t_int || es > et);
+      const int ms = split_t && split_s ? (same ? 3 : 4) : (split_t ? 5 : (split_s ? 6 : 0));
+      const int m = fa ? 1 : (fn ? 2 : (pvalid ? ms : 0));
+      mode[k] = m;
+      x0[k] = (uint32_t)(fa ? nt.pad : (fn ? nt.leafpos : nt.left));
+      x1[k] = (uint32_t)(fa ? ns.pad : (fn ? ns.leafpos : nt.right));
+      x2[k] = (uint32_t)ns.left;
+      x3[k] = (uint32_t)ns.right;
+      nf += fa ? per_pair : 0u;
+      nn += fn ? per_pair : 0u;
+      nc += m == 3 ? 3u : (m == 4 ? 4u : (m >= 5 ? 2u : 0u));
+      continue;
+    }
+    if (acc) {
+      mode[k] = 1;
+      x0[k] = (uint32_t)nt.pad;  // level-major rank of t
+      x1[k] = (uint32_t)ns.pad;
+      if (TAGS) {  // directed tags: (t <- s) and (s <- t)
+        x2[k] = (uint32_t)desc_tag(a.policy, d2, et, es, t);
+        x3[k] = (uint32_t)desc_tag(a.policy, d2, es, et, s);
+      }
+      nf += 2;
+    } else if (near_rule && !t_int && !s_int && diff) {
+      mode[k] = 2;
+      x0[k] = (uint32_t)nt.leafpos;
+      x1[k] = (uint32_t)ns.leafpos;
+      nn += 2;
+    } else {
+      const bool same = !diff;
+      const bool split_t = t_int && (same || !s_int || et >= es);
+      const bool split_s = s_int && (same || !t_int || es > et);
+      x0[k] = (uint32_t)nt.left;
+      x1[k] = (uint32_t)nt.right;
+      x2[k] = (uint32_t)ns.left;
+      x3[k] = (uint32_t)ns.right;
+      if (split_t && split_s) {
+        mode[k] = same ? 3 : 4;
+        nc += same ? 3 : 4;
+      } else if (split_t) {
+        mode[k] = 5;
+        nc += 2;
+      } else if (split_s) {
+        mode[k] = 6;
+        nc += 2;
+      }
+    }
+  }
+  }
+  // Block exclusive scan of (children, far, near) packed in 21-bit fields.
+  const unsigned long long packed =
+      (unsigned long long)nc | ((unsigned long long)nf << 21) | ((unsigned long long)nn << 42);
+  const unsigned long long incl = wave_incl_u64(packed);
+  if (lane == 63) sh.wave[w] = incl;
+  __syncthreads();
+  unsigned long long wbase = 0, btot = 0;
+#pragma unroll
+  for (int q = 0; q < THREADS / YGG_WAVE; ++q) {
+    if (q < w) wbase += sh.wave[q];
+    btot += sh.wave[q];
+  }
+  const unsigned long long mask = (1ull << 21) - 1;
+  if (for_children || for_entries) {
+    const unsigned long long tc = btot & mask, tf = (btot >> 21) & mask,
+                             tn = (btot >> 42) & mask;
+    unsigned long long bf = 0, bn = 0;  // stream offsets of the generation
+    bool go = true;
+    if (PERSIST) {
+      const bool known = MODE == kAlone && alone->from_lds;
+      bf = known ? alone->bf : rec_f + (rec_c >> 32);
+      bn = known ? alone->bn : rec_n + (rec_c & 0xFFFFFFFFull);
+      const int64_t worst = a.pair_records ? size : 2 * size;
+      go = (int64_t)bf + worst <= a.far_cap && (int64_t)bn + worst <= a.near_cap;
+      if (MODE == kAlone && go) {
+        alone->bf = bf + tf;
+        alone->bn = bn + tn;
+      }
+    } else if (EMIT && a.gen_fill) {
+      bf = sh.gbase[0];
+      bn = sh.gbase[1];
+    }
+    unsigned long long* rec = a.gen_fill ? a.gen_fill + (size_t)g * kGenRecWords : nullptr;
+    if (for_children) {
+      if (PERSIST) {
+        sh.stop = !go;
+        if (!go) atomicMax(&a.flags[3], (uint32_t)(g + 1));
+      }
+      if (MODE == kAlone) {
+        if (go) atomic_store_agent(&a.gen_sizes[g + 1], (uint32_t)tc);
+        sh.base[0] = 0;
+      } else {
+        sh.base[0] = go && tc ? atomicAdd(&a.gen_sizes[g + 1], (uint32_t)tc) : 0;
+      }
+    } else if (go) {
+      if (PERSIST && chunk == 0) {
+        atomic_store_agent(&rec[1], bf);
+        atomic_store_agent(&rec[2], bn);
+      }
+      if (MODE == kAlone) {
+        atomic_store_agent(&rec[0], (tf << 32) | tn);
+        sh.base[1] = bf;
+        sh.base[2] = bn;
+      } else if (spread) {
+        acc_f += tf;
+        acc_n += tn;
+        sh.base[1] = sh.base[2] = 0;
+      } else if (EMIT && a.gen_fill) {
+        // this generation's far (high) and near (low 32 bits) counts in one
+        // reservation; they stay below 2 * queue_cap < 2^32
+        const unsigned long long add = (tf << 32) | tn;
+        const unsigned long long old = add ? atomicAdd(&rec[0], add) : 0ull;
+        sh.base[1] = bf + (old >> 32);
+        sh.base[2] = bn + (old & 0xFFFFFFFFull);
+      } else if (EMIT) {
+        // far (high 32 bits) and near (low 32 bits) running totals in one
+        // reservation; a field that would pass 2^32 marks the walk as
+        // overflowed (its result is discarded)
+        const unsigned long long add = (tf << 32) | tn;
+        const unsigned long long old = add ? atomicAdd(&a.counters[0], add) : 0ull;
+        sh.base[1] = old >> 32;
+        sh.base[2] = old & 0xFFFFFFFFull;
+        if ((old >> 32) + tf > 0xFFFFFFFFull || (old & 0xFFFFFFFFull) + tn > 0xFFFFFFFFull)
+          atomicOr(&a.flags[1], 1u);
+      } else {
+        sh.base[1] = tf ? atomicAdd(&a.counters[0], tf) : 0;
+        sh.base[2] = tn ? atomicAdd(&a.counters[1], tn) : 0;
+      }
+    }
+  }
+  __syncthreads();
+  if (PERSIST && sh.stop) return false;
+  children = (unsigned)(btot & mask);
+  const unsigned long long ex = wbase + incl - packed;
+  // wavefront-local offsets of this lane's far and near entries
+  const unsigned long long lex = incl - packed;
+  const unsigned wave_nf = (unsigned)((sh.wave[w] >> 21) & mask);
+  unsigned lf = (unsigned)((lex >> 21) & mask);
+  unsigned ln = wave_nf + (unsigned)((lex >> 42) & mask);
+  bool qover = false, fover = false, nover = false;
+  const bool records = !TAGS && a.pair_records;
+  const unsigned per_pair = records ? 1u : 2u;
+#pragma unroll
+  for (int k = 0; k < kFlatPer; ++k) {
+    const int m = mode[k];
+    const bool isf = m == 1, isn = m == 2;
+    if (EMIT && !TAGS) {
+      // entries (t's row key, s) and (s's row key, t), or the record
+      // (t, s) with the second store going to the spare slot
+      const unsigned dst = isf ? lf : (isn ? ln : kDump);
+      sh.stage[w][dst] = make_uint2(records ? pt[k] : x0[k], ps[k]);
+      sh.stage[w][records ? kDump + 1 : dst + 1] = make_uint2(x1[k], pt[k]);
+    } else if (EMIT) {
+      if (isf) {
+        sh.stage[w][lf] = make_uint2(x0[k], ps[k]);
+        sh.stage[w][lf + 1] = make_uint2(x1[k], pt[k]);
+        sh.tag[w][lf] = (int32_t)x2[k];
+        sh.tag[w][lf + 1] = (int32_t)x3[k];
+      } else if (isn) {
+        sh.stage[w][ln] = make_uint2(x0[k], ps[k]);
+        sh.stage[w][ln + 1] = make_uint2(x1[k], pt[k]);
+      }
+    }
+    lf += isf ? per_pair : 0u;
+    ln += isn ? per_pair : 0u;
+  }
+  if (EMIT) {
+    __syncthreads();  // staged entries visible to the whole wavefront
+    const unsigned wave_nn = (unsigned)((sh.wave[w] >> 42) & mask);
+    const unsigned long long wex = wbase;  // block-exclusive prefix of this wavefront
+    const int64_t fbase = (int64_t)sh.base[1] + (int64_t)((wex >> 21) & mask);
+    const int64_t nbase = (int64_t)sh.base[2] + (int64_t)((wex >> 42) & mask);
+    // The streams are read only after the walk, by the row lists: written
+    // non-temporally they leave L2 and the Infinity Cache to the node
+    // records every generation gathers (2^24 clustered emission walk:
+    // 5.69 -> 5.56 ms).
+    for (unsigned j = lane; j < wave_nf; j += YGG_WAVE) {
+      const int64_t slot = fbase + j;
+      if (slot < a.far_cap) {
+        const uint2 e = sh.stage[w][j];
+        __builtin_nontemporal_store(e.x, &a.far_keys[slot]);
+        __builtin_nontemporal_store(e.y, &a.far_vals[slot]);
+        if (TAGS) __builtin_nontemporal_store(sh.tag[w][j], &a.far_tags[slot]);
+      } else {
+        fover = true;
+      }
+    }
+    for (unsigned j = lane; j < wave_nn; j += YGG_WAVE) {
+      const int64_t slot = nbase + j;
+      if (slot < a.near_cap) {
+        const uint2 e = sh.stage[w][wave_nf + j];
+        __builtin_nontemporal_store(e.x, &a.near_keys[slot]);
+        __builtin_nontemporal_store(e.y, &a.near_vals[slot]);
+      } else {
+        nover = true;
+      }
+    }
+  }
+  // Children that fit one chunk of the same workgroup stay in LDS (the pairs
+  // of this one are in registers since before the scan's barrier).
+  const bool in_lds = MODE == kAlone && alone->more &&
+                      children <= (unsigned)(THREADS * kFlatPer) &&
+                      (int64_t)children <= a.queue_cap;
+  if (in_lds) {
+    unsigned lc = (unsigned)(wbase & mask) + (unsigned)(lex & mask);
+#pragma unroll
+    for (int k = 0; k < kFlatPer; ++k) {
+      const int m = mode[k];
+      if (m < 3) continue;
+      auto put = [&](uint32_t t, uint32_t s) {
+        alone->pairs[lc++] = ((uint64_t)min(t, s) << 32) | max(t, s);
+      };
+      put(m == 6 ? pt[k] : x0[k], m == 3 ? x0[k] : (m == 5 ? ps[k] : x2[k]));
+      put(m == 6 ? pt[k] : (m == 5 ? x1[k] : x0[k]), m == 3 ? x1[k] : (m == 5 ? ps[k] : x3[k]));
+      if (m == 3) put(x1[k], x1[k]);
+      if (m == 4) {
+        put(x1[k], x2[k]);
+        put(x1[k], x3[k]);
+      }
+    }
+  } else {
+    // Child pairs, in rounds of kStage slots of the wavefront's range; the
+    // round count is the largest over the block's wavefronts so every thread
+    // reaches the same barriers.
+    unsigned max_nc = 0;
+#pragma unroll
+    for (int q = 0; q < THREADS / YGG_WAVE; ++q)
+      max_nc = max(max_nc, (unsigned)(sh.wave[q] & mask));
+    const unsigned wave_nc = (unsigned)(sh.wave[w] & mask);
+    const int64_t cbase = (int64_t)sh.base[0] + (int64_t)(wbase & mask);
+    const unsigned lc0 = (unsigned)(lex & mask);
+    for (unsigned r0 = 0; r0 < max_nc; r0 += kStage) {
+      if (EMIT || r0 > 0) __syncthreads();  // previous use of sh.stage finished
+      unsigned lc = lc0;
+#pragma unroll
+      for (int k = 0; k < kFlatPer; ++k) {
+        const int m = mode[k];
+        // children (a_j, b_j): mode 3 (t,t) split, 4 cross split,
+        // 5 split t only, 6 split s only
+        const uint32_t a0 = m == 6 ? pt[k] : x0[k];
+        const uint32_t b0 = m == 3 ? x0[k] : (m == 5 ? ps[k] : x2[k]);
+        const uint32_t a1 = m == 6 ? pt[k] : (m == 5 ? x1[k] : x0[k]);
+        const uint32_t b1 = m == 3 ? x1[k] : (m == 5 ? ps[k] : x3[k]);
+        const uint32_t a2 = x1[k];
+        const uint32_t b2 = m == 3 ? x1[k] : x2[k];
+        const uint32_t a3 = x1[k], b3 = x3[k];
+        const unsigned cnt = m < 3 ? 0u : (m == 3 ? 3u : (m == 4 ? 4u : 2u));
+        // a slot outside this round's window (the offset wraps when
+        // lc < r0), or past the pair's children, is the dump slot
+        unsigned o = lc - r0;
+        sh.stage[w][cnt && o < (unsigned)kStage ? o : kDump] = make_uint2(min(a0, b0), max(a0, b0));
+        o = lc + 1 - r0;
+        sh.stage[w][cnt && o < (unsigned)kStage ? o : kDump] = make_uint2(min(a1, b1), max(a1, b1));
+        o = lc + 2 - r0;
+        sh.stage[w][cnt > 2 && o < (unsigned)kStage ? o : kDump] =
+            make_uint2(min(a2, b2), max(a2, b2));
+        o = lc + 3 - r0;
+        sh.stage[w][cnt > 3 && o < (unsigned)kStage ? o : kDump] =
+            make_uint2(min(a3, b3), max(a3, b3));
+        lc += cnt;
+      }
+      __syncthreads();
+      // Children [r0, end) of the wavefront's; none where another wavefront
+      // needs the round. (Written as a count of children left, 0 below r0,
+      // the compiler dropped the comparison and took the wrapped count.)
+      const unsigned end = min(wave_nc, r0 + (unsigned)kStage);
+      for (unsigned j = r0 + lane; j < end; j += YGG_WAVE) {
+        const int64_t slot = cbase + j;
+        if (slot < a.queue_cap) {
+          const uint2 e = sh.stage[w][j - r0];
+          const uint64_t word = ((uint64_t)e.x << 32) | e.y;
+          if (PERSIST)
+            atomic_store_agent(&wf_out[slot], word);
+          else
+            wf_out[slot] = word;
+        } else {
+          qover = true;
+        }
+      }
+    }
+  }
+  if (qover) atomicOr(&a.flags[0], 1u);
+  if (fover) atomicOr(&a.flags[1], 1u);
+  if (nover) atomicOr(&a.flags[2], 1u);
+  // this wavefront's queue words have arrived (in LDS they need not be waited for)
+  if (PERSIST && !in_lds) __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();  // every wavefront's; and sh is free again
+  return true;
+}
+
 template <bool EMIT, int kFlatPer, bool TAGS = false>
 __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
   static_assert(!TAGS || EMIT, "tags are written by the emission walk");
@@ -107,7 +555,7 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
   // record's offsets plus its final counts, the same in every workgroup;
   // workgroup 0 stores them in record g, also when it has no chunk) and the
   // capacity check that pauses the walk before anything is written.
-  __shared__ unsigned long long s_gbase[2];
+  __shared__ WalkShared<kFlatPer, TAGS> sh;
   if (EMIT && a.gen_fill) {
     if (c_first >= c_end && blockIdx.x != 0) return;
     if (threadIdx.x == 0) {
@@ -118,8 +566,8 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
         bf = r[1] + (c >> 32);
         bn = r[2] + (c & 0xFFFFFFFFull);
       }
-      s_gbase[0] = bf;
-      s_gbase[1] = bn;
+      sh.gbase[0] = bf;
+      sh.gbase[1] = bn;
       if (blockIdx.x == 0) {
         a.gen_fill[(size_t)g * kGenRecWords + 1] = bf;
         a.gen_fill[(size_t)g * kGenRecWords + 2] = bn;
@@ -128,345 +576,183 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
     __syncthreads();
     if (c_first >= c_end) return;
     const int64_t worst = a.pair_records ? size : 2 * size;
-    if ((int64_t)s_gbase[0] + worst > a.far_cap || (int64_t)s_gbase[1] + worst > a.near_cap) {
+    if ((int64_t)sh.gbase[0] + worst > a.far_cap || (int64_t)sh.gbase[1] + worst > a.near_cap) {
       if (threadIdx.x == 0) atomicMax(&a.flags[3], (uint32_t)(g + 1));
       return;
     }
   }
   if (c_first >= c_end) return;
-  const uint64_t* __restrict__ wf_in = (g & 1) ? a.wf1 : a.wf0;
-  uint64_t* __restrict__ wf_out = (g & 1) ? a.wf0 : a.wf1;
-  const NodeRec* __restrict__ nodes = a.nodes;
-  const unsigned lane = lane_id();
-  const int w = threadIdx.x / YGG_WAVE;
-  __shared__ unsigned long long s_wave[kFlatThreads / YGG_WAVE];
-  __shared__ unsigned long long s_base[3];
   // counting walk with spread counters: this workgroup's far/near totals,
   // added to one lane at the end instead of one reservation per chunk
   const bool spread = !EMIT && a.spread != nullptr;
   unsigned long long acc_f = 0, acc_n = 0;
-  // Output staging. Each wavefront's outputs of one chunk occupy one
-  // contiguous range of each stream (slots follow the block scan), so they
-  // are gathered in LDS and written out by consecutive lanes. A pair yields
-  // at most two far or two near entries: 2 * 64 * kFlatPer slots hold both
-  // (far first, then near). Child pairs (up to four per pair) go through the
-  // same buffer in rounds of kStage.
-  // Writes that nobody reads (a pair with no output of that kind, a child
-  // outside the current round) go to two spare slots past the range, so
-  // every pair writes the same number of slots and the staging has no
-  // per-pair branches.
-  constexpr int kStage = 2 * YGG_WAVE * kFlatPer;
-  constexpr unsigned kDump = kStage;
-  __shared__ uint2 s_stage[kFlatThreads / YGG_WAVE][kStage + 2];
-  __shared__ int32_t s_tag[kFlatThreads / YGG_WAVE][TAGS ? 2 * YGG_WAVE * kFlatPer : 1];
-
-  for (int64_t ci = c_first; ci < c_end; ci += c_step) {
-    const int64_t chunk = ci * kFlatChunk;
-    // mode: 0 none, 1 accept, 2 near, 3 both-same, 4 both-cross, 5 split t, 6 split s
-    int mode[kFlatPer];
-    uint32_t pt[kFlatPer], ps[kFlatPer], x0[kFlatPer], x1[kFlatPer], x2[kFlatPer],
-        x3[kFlatPer];
-    unsigned nc = 0, nf = 0, nn = 0;
-    // Memory first, decisions after: every pair word of the chunk, then the
-    // node records of a group of four pairs, are loaded before any of them
-    // is used, so their latencies overlap instead of adding up pair by pair
-    // (a lane past the wavefront's end loads node 0 and decides nothing).
-    // Measured on the 2^24 clustered walk at 8 pairs per thread: 7.8 ms with
-    // the loads issued pair by pair, 6.9 ms with groups of two when the
-    // decisions branched per pair; with branch-free decisions 6.20 ms with
-    // groups of two, 6.13 ms with four (151 VGPRs, still 3 waves per SIMD)
-    // and 7.38 ms with eight (2 waves per SIMD).
-    constexpr uint64_t kNoPair = ~0ull;
-    uint64_t prw[kFlatPer];
-#pragma unroll
-    for (int k = 0; k < kFlatPer; ++k) {
-      const int64_t idx = chunk + k * kFlatThreads + threadIdx.x;
-      prw[k] = idx < size ? wf_in[idx] : kNoPair;
-    }
-    constexpr int kGroup = kFlatPer < 4 ? kFlatPer : 4;
-#pragma unroll
-    for (int k0 = 0; k0 < kFlatPer; k0 += kGroup) {
-    NodeRec rt[kGroup], rs[kGroup];
-#pragma unroll
-    for (int j = 0; j < kGroup; ++j) {
-      const uint64_t pr = prw[k0 + j];
-      const bool valid = pr != kNoPair;
-      rt[j] = nodes[valid ? (int32_t)(pr >> 32) : 0];
-      rs[j] = nodes[valid ? (int32_t)(uint32_t)pr : 0];
-    }
-#pragma unroll
-    for (int j = 0; j < kGroup; ++j) {
-      const int k = k0 + j;
-      mode[k] = 0;
-      const bool pvalid = prw[k] != kNoPair;
-      if (TAGS && !pvalid) continue;
-      const uint64_t pr = prw[k];
-      const int32_t t = (int32_t)(pr >> 32), s = (int32_t)(uint32_t)pr;
-      const NodeRec& nt = rt[j];
-      const NodeRec& ns = rs[j];
-      float dx = nt.cx - ns.cx, dy = nt.cy - ns.cy, dz = nt.cz - ns.cz;
-      float d2 = dx * dx;
-      d2 = d2 + dy * dy;
-      d2 = d2 + dz * dz;
-      const float et = nt.ext, es = ns.ext;
-      const bool diff = t != s;
-      bool ok;
-      if (a.mac_type == YGG_MAC_ENGBLOM) {
-        float rb = fmaxf(et, es), rs = fminf(et, es);
-        float lhs = rb + a.theta_root * rs;
-        ok = diff && d2 > 0.0f && (lhs * lhs <= a.theta_sq * d2);
-      } else {
-        float sum = et + es;
-        ok = diff && d2 > 0.0f && (sum * sum <= a.theta_sq * d2);
-      }
-      // internal nodes carry children (node ids of a forest are not
-      // split at num_internal)
-      const bool t_int = nt.left >= 0, s_int = ns.left >= 0;
-      if (a.node_hist && g == a.hist_gen && pvalid) atomicAdd(&a.node_hist[t], 1);
-      pt[k] = (uint32_t)t;
-      ps[k] = (uint32_t)s;
-      // accept / near rules (uniform per launch): the built-in MAC with
-      // near leaf pairs unless a policy descriptor says otherwise
-      bool acc = ok;
-      if (a.policy.accept == YGG_ACCEPT_DISTANCE)
-        acc = diff && d2 >= a.policy.accept_dist_sq;
-      else if (a.policy.accept == YGG_ACCEPT_DIFFERENT)
-        acc = diff;
-      else if (a.policy.accept == YGG_ACCEPT_NEVER)
-        acc = false;
-      const bool near_rule = a.policy.near == YGG_NEAR_LEAF_PAIRS;
-      const unsigned per_pair = !TAGS && a.pair_records ? 1u : 2u;  // stream slots
-      if (!TAGS) {
-        // Every field from selects, with no per-pair branch: accept (1),
-        // near (2) or a split (3 both of the same node, 4 both, 5 t only,
-        // 6 s only); nothing for a lane past the wavefront's end. On the
-        // 2^24 clustered walk the branching form took 6.88 ms, this one
-        // 6.21 ms (fewer exec-mask updates, 139 instead of 155 VGPRs).
-        const bool fa = pvalid && acc;
-        const bool fn = pvalid && !acc && near_rule && !t_int && !s_int && diff;
-        const bool same = !diff;
-        const bool split_t = t_int && (same || !s_int || et >= es);
-        const bool split_s = s_int && (same || !t_int || es > et);
-        const int ms = split_t && split_s ? (same ? 3 : 4) : (split_t ? 5 : (split_s ? 6 : 0));
-        const int m = fa ? 1 : (fn ? 2 : (pvalid ? ms : 0));
-        mode[k] = m;
-        x0[k] = (uint32_t)(fa ? nt.pad : (fn ? nt.leafpos : nt.left));
-        x1[k] = (uint32_t)(fa ? ns.pad : (fn ? ns.leafpos : nt.right));
-        x2[k] = (uint32_t)ns.left;
-        x3[k] = (uint32_t)ns.right;
-        nf += fa ? per_pair : 0u;
-        nn += fn ? per_pair : 0u;
-        nc += m == 3 ? 3u : (m == 4 ? 4u : (m >= 5 ? 2u : 0u));
-        continue;
-      }
-      if (acc) {
-        mode[k] = 1;
-        x0[k] = (uint32_t)nt.pad;  // level-major rank of t
-        x1[k] = (uint32_t)ns.pad;
-        if (TAGS) {  // directed tags: (t <- s) and (s <- t)
-          x2[k] = (uint32_t)desc_tag(a.policy, d2, et, es, t);
-          x3[k] = (uint32_t)desc_tag(a.policy, d2, es, et, s);
-        }
-        nf += 2;
-      } else if (near_rule && !t_int && !s_int && diff) {
-        mode[k] = 2;
-        x0[k] = (uint32_t)nt.leafpos;
-        x1[k] = (uint32_t)ns.leafpos;
-        nn += 2;
-      } else {
-        const bool same = !diff;
-        const bool split_t = t_int && (same || !s_int || et >= es);
-        const bool split_s = s_int && (same || !t_int || es > et);
-        x0[k] = (uint32_t)nt.left;
-        x1[k] = (uint32_t)nt.right;
-        x2[k] = (uint32_t)ns.left;
-        x3[k] = (uint32_t)ns.right;
-        if (split_t && split_s) {
-          mode[k] = same ? 3 : 4;
-          nc += same ? 3 : 4;
-        } else if (split_t) {
-          mode[k] = 5;
-          nc += 2;
-        } else if (split_s) {
-          mode[k] = 6;
-          nc += 2;
-        }
-      }
-    }
-    }
-    // Block exclusive scan of (children, far, near) packed in 21-bit fields.
-    const unsigned long long packed =
-        (unsigned long long)nc | ((unsigned long long)nf << 21) | ((unsigned long long)nn << 42);
-    const unsigned long long incl = wave_incl_u64(packed);
-    if (lane == 63) s_wave[w] = incl;
-    __syncthreads();
-    unsigned long long wbase = 0, btot = 0;
-#pragma unroll
-    for (int q = 0; q < kFlatThreads / YGG_WAVE; ++q) {
-      if (q < w) wbase += s_wave[q];
-      btot += s_wave[q];
-    }
-    const unsigned long long mask = (1ull << 21) - 1;
-    if (threadIdx.x == 0) {
-      const unsigned long long tc = btot & mask, tf = (btot >> 21) & mask,
-                               tn = (btot >> 42) & mask;
-      s_base[0] = tc ? atomicAdd(&a.gen_sizes[g + 1], (uint32_t)tc) : 0;
-      if (spread) {
-        acc_f += tf;
-        acc_n += tn;
-        s_base[1] = s_base[2] = 0;
-      } else if (EMIT && a.gen_fill) {
-        // this generation's far (high) and near (low 32 bits) counts in one
-        // reservation; they stay below 2 * queue_cap < 2^32
-        const unsigned long long add = (tf << 32) | tn;
-        const unsigned long long old =
-            add ? atomicAdd(&a.gen_fill[(size_t)g * kGenRecWords], add) : 0ull;
-        s_base[1] = s_gbase[0] + (old >> 32);
-        s_base[2] = s_gbase[1] + (old & 0xFFFFFFFFull);
-      } else if (EMIT) {
-        // far (high 32 bits) and near (low 32 bits) running totals in one
-        // reservation; a field that would pass 2^32 marks the walk as
-        // overflowed (its result is discarded)
-        const unsigned long long add = (tf << 32) | tn;
-        const unsigned long long old = add ? atomicAdd(&a.counters[0], add) : 0ull;
-        s_base[1] = old >> 32;
-        s_base[2] = old & 0xFFFFFFFFull;
-        if ((old >> 32) + tf > 0xFFFFFFFFull || (old & 0xFFFFFFFFull) + tn > 0xFFFFFFFFull)
-          atomicOr(&a.flags[1], 1u);
-      } else {
-        s_base[1] = tf ? atomicAdd(&a.counters[0], tf) : 0;
-        s_base[2] = tn ? atomicAdd(&a.counters[1], tn) : 0;
-      }
-    }
-    __syncthreads();
-    const unsigned long long ex = wbase + incl - packed;
-    // wavefront-local offsets of this lane's far and near entries
-    const unsigned long long lex = incl - packed;
-    const unsigned wave_nf = (unsigned)((s_wave[w] >> 21) & mask);
-    unsigned lf = (unsigned)((lex >> 21) & mask);
-    unsigned ln = wave_nf + (unsigned)((lex >> 42) & mask);
-    bool qover = false, fover = false, nover = false;
-    const bool records = !TAGS && a.pair_records;
-    const unsigned per_pair = records ? 1u : 2u;
-#pragma unroll
-    for (int k = 0; k < kFlatPer; ++k) {
-      const int m = mode[k];
-      const bool isf = m == 1, isn = m == 2;
-      if (EMIT && !TAGS) {
-        // entries (t's row key, s) and (s's row key, t), or the record
-        // (t, s) with the second store going to the spare slot
-        const unsigned dst = isf ? lf : (isn ? ln : kDump);
-        s_stage[w][dst] = make_uint2(records ? pt[k] : x0[k], ps[k]);
-        s_stage[w][records ? kDump + 1 : dst + 1] = make_uint2(x1[k], pt[k]);
-      } else if (EMIT) {
-        if (isf) {
-          s_stage[w][lf] = make_uint2(x0[k], ps[k]);
-          s_stage[w][lf + 1] = make_uint2(x1[k], pt[k]);
-          s_tag[w][lf] = (int32_t)x2[k];
-          s_tag[w][lf + 1] = (int32_t)x3[k];
-        } else if (isn) {
-          s_stage[w][ln] = make_uint2(x0[k], ps[k]);
-          s_stage[w][ln + 1] = make_uint2(x1[k], pt[k]);
-        }
-      }
-      lf += isf ? per_pair : 0u;
-      ln += isn ? per_pair : 0u;
-    }
-    if (EMIT) {
-      __syncthreads();  // staged entries visible to the whole wavefront
-      const unsigned wave_nn = (unsigned)((s_wave[w] >> 42) & mask);
-      const unsigned long long wex = wbase;  // block-exclusive prefix of this wavefront
-      const int64_t fbase = (int64_t)s_base[1] + (int64_t)((wex >> 21) & mask);
-      const int64_t nbase = (int64_t)s_base[2] + (int64_t)((wex >> 42) & mask);
-      // The streams are read only after the walk, by the row lists: written
-      // non-temporally they leave L2 and the Infinity Cache to the node
-      // records every generation gathers (2^24 clustered emission walk:
-      // 5.69 -> 5.56 ms).
-      for (unsigned j = lane; j < wave_nf; j += YGG_WAVE) {
-        const int64_t slot = fbase + j;
-        if (slot < a.far_cap) {
-          const uint2 e = s_stage[w][j];
-          __builtin_nontemporal_store(e.x, &a.far_keys[slot]);
-          __builtin_nontemporal_store(e.y, &a.far_vals[slot]);
-          if (TAGS) __builtin_nontemporal_store(s_tag[w][j], &a.far_tags[slot]);
-        } else {
-          fover = true;
-        }
-      }
-      for (unsigned j = lane; j < wave_nn; j += YGG_WAVE) {
-        const int64_t slot = nbase + j;
-        if (slot < a.near_cap) {
-          const uint2 e = s_stage[w][wave_nf + j];
-          __builtin_nontemporal_store(e.x, &a.near_keys[slot]);
-          __builtin_nontemporal_store(e.y, &a.near_vals[slot]);
-        } else {
-          nover = true;
-        }
-      }
-    }
-    // Child pairs, in rounds of kStage slots of the wavefront's range; the
-    // round count is the largest over the block's wavefronts so every thread
-    // reaches the same barriers.
-    {
-      unsigned max_nc = 0;
-#pragma unroll
-      for (int q = 0; q < kFlatThreads / YGG_WAVE; ++q)
-        max_nc = max(max_nc, (unsigned)(s_wave[q] & mask));
-      const unsigned wave_nc = (unsigned)(s_wave[w] & mask);
-      const int64_t cbase = (int64_t)s_base[0] + (int64_t)(wbase & mask);
-      const unsigned lc0 = (unsigned)(lex & mask);
-      for (unsigned r0 = 0; r0 < max_nc; r0 += kStage) {
-        if (EMIT || r0 > 0) __syncthreads();  // previous use of s_stage finished
-        unsigned lc = lc0;
-#pragma unroll
-        for (int k = 0; k < kFlatPer; ++k) {
-          const int m = mode[k];
-          // children (a_j, b_j): mode 3 (t,t) split, 4 cross split,
-          // 5 split t only, 6 split s only
-          const uint32_t a0 = m == 6 ? pt[k] : x0[k];
-          const uint32_t b0 = m == 3 ? x0[k] : (m == 5 ? ps[k] : x2[k]);
-          const uint32_t a1 = m == 6 ? pt[k] : (m == 5 ? x1[k] : x0[k]);
-          const uint32_t b1 = m == 3 ? x1[k] : (m == 5 ? ps[k] : x3[k]);
-          const uint32_t a2 = x1[k];
-          const uint32_t b2 = m == 3 ? x1[k] : x2[k];
-          const uint32_t a3 = x1[k], b3 = x3[k];
-          const unsigned cnt = m < 3 ? 0u : (m == 3 ? 3u : (m == 4 ? 4u : 2u));
-          // a slot outside this round's window (the offset wraps when
-          // lc < r0), or past the pair's children, is the dump slot
-          unsigned o = lc - r0;
-          s_stage[w][cnt && o < (unsigned)kStage ? o : kDump] = make_uint2(min(a0, b0), max(a0, b0));
-          o = lc + 1 - r0;
-          s_stage[w][cnt && o < (unsigned)kStage ? o : kDump] = make_uint2(min(a1, b1), max(a1, b1));
-          o = lc + 2 - r0;
-          s_stage[w][cnt > 2 && o < (unsigned)kStage ? o : kDump] =
-              make_uint2(min(a2, b2), max(a2, b2));
-          o = lc + 3 - r0;
-          s_stage[w][cnt > 3 && o < (unsigned)kStage ? o : kDump] =
-              make_uint2(min(a3, b3), max(a3, b3));
-          lc += cnt;
-        }
-        __syncthreads();
-        const unsigned n_r = wave_nc > r0 ? min(wave_nc - r0, (unsigned)kStage) : 0u;
-        for (unsigned j = lane; j < n_r; j += YGG_WAVE) {
-          const int64_t slot = cbase + r0 + j;
-          if (slot < a.queue_cap) {
-            const uint2 e = s_stage[w][j];
-            wf_out[slot] = ((uint64_t)e.x << 32) | e.y;
-          } else {
-            qover = true;
-          }
-        }
-      }
-    }
-    if (qover) atomicOr(&a.flags[0], 1u);
-    if (fover) atomicOr(&a.flags[1], 1u);
-    if (nover) atomicOr(&a.flags[2], 1u);
-    __syncthreads();  // s_wave / s_base / s_stage reuse
-  }
-  if (spread && threadIdx.x == 0 && (acc_f | acc_n)) {
+  unsigned children = 0;
+  for (int64_t ci = c_first; ci < c_end; ci += c_step)
+    walk_chunk<EMIT, kFlatPer, TAGS, kLaunched, kFlatThreads>(a, g, size, ci * kFlatChunk, sh, spread, acc_f, acc_n,
+                                            children);
+  if (spread && threadIdx.x == YGG_WAVE && (acc_f | acc_n)) {
     const int lane_id = (int)(blockIdx.x % (unsigned)a.spread_lanes);
     if (acc_f) atomicAdd(&a.spread[2 * lane_id], acc_f);
     if (acc_n) atomicAdd(&a.spread[2 * lane_id + 1], acc_n);
+  }
+}
+
+// Generations [lo, hi) of a resumable emission walk in one launch. A
+// generation of up to 10^5 pairs costs a launch its own dependent chain
+// (11 us for one pair, 14 us for 128 K pairs, instruction fetch and the
+// launch gap included), so a small walk spends all of its 15 to 50
+// generations there, and a large one half; here only the chain is left.
+//
+// A generation of at most one chunk is run by one workgroup alone, with
+// those that follow it while they fit: pairs in LDS, nothing reserved.
+// Larger ones are shared, as follows.
+//
+// No workgroup waits for another that may not be running: chunks of kChunk
+// pairs are claimed by ticket, and a generation is over when all its chunks
+// are done, whoever ran them. The workgroup that adds the last done chunk
+// knows the children's total and publishes the next generation; the others
+// wait for that word. A claimed chunk belongs to a running workgroup, so
+// every wait ends; one that starts late finds no tickets and catches up. The
+// tickets of a generation are claimed before its size is known, while
+// waiting.
+//
+// Between workgroups (on XCDs with an L2 each) only agent-scope words pass:
+// queue words, records, done counts and the published size. Each wavefront
+// waits for its stores before the workgroup releases its done chunk.
+//
+// Measured (kernel time of all generations): 1 K pairs in 14 generations 50
+// against 113 us of launches, 120 K in 25 165 against 250 us, 1 M in 47 394
+// to 431 against 548 us. Each release writes the XCD's L2 back, so few large
+// workgroups: with 256 threads (512-pair chunks) the last takes 913 us.
+//
+// Record g + half of gen_fill (g < half = max_generations / 2) holds
+// generation g's sync words: tickets (3), done chunks << 36 | children so far
+// (4), and what is published of it (5): kPublished | size, kPublished | kJump |
+// generation (go on there), or kPublished | kStopped.
+constexpr unsigned long long kPublished = 1ull << 63, kStopped = 1ull << 62, kJump = 1ull << 61;
+constexpr int kTicketWord = 3, kDoneWord = 4, kReadyWord = 5;
+constexpr int kSpinLimit = 1 << 20;  // about a second
+constexpr int kPersistThreads = 1024, kPersistPer = 2;
+constexpr int kPersistChunk = kPersistThreads * kPersistPer;
+
+template <bool TAGS>
+__global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, int half, int lo, int hi) {
+  if (atomic_load_agent(&a.flags[0]) | atomic_load_agent(&a.flags[1]) |
+      atomic_load_agent(&a.flags[2]) | atomic_load_agent(&a.flags[3]))
+    return;
+  __shared__ WalkShared<kPersistPer, TAGS, kPersistThreads> sh;
+  __shared__ uint64_t s_pairs[kPersistChunk];
+  // slot g % 2: a wavefront may still read the last generation's
+  __shared__ unsigned long long s_ready[2], s_ticket[2];
+  unsigned long long acc_f = 0, acc_n = 0;
+  int g = lo;
+  while (g < hi) {
+    unsigned long long* sync = a.gen_fill + (size_t)(half + g) * kGenRecWords;
+    if (threadIdx.x == 0) {
+      const unsigned long long ticket = atomicAdd(&sync[kTicketWord], 1ull);
+      unsigned long long v = 0;
+      if (g == lo) {
+        v = kPublished | atomic_load_agent(&a.gen_sizes[g]);
+      } else {
+        for (int spin = 0; spin < kSpinLimit; ++spin) {
+          v = atomic_load_agent(&sync[kReadyWord]);
+          if (v & kPublished) break;
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (!(v & kPublished)) {  // not reached: the walk counts as overflowed
+          atomicOr(&a.flags[0], 1u);
+          v = kPublished | kStopped;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      s_ready[g & 1] = v;
+      s_ticket[g & 1] = ticket;
+    }
+    __syncthreads();
+    const unsigned long long ready = s_ready[g & 1];
+    if (ready & kStopped) return;
+    if (ready & kJump) {  // generations that one workgroup has run alone
+      g = (int)(ready & 0xFFFFFFFFull);
+      __syncthreads();  // slots of the same parity
+      continue;
+    }
+    const int64_t size = (int64_t)(ready & 0xFFFFFFFFull);
+    if (size == 0) return;
+    const unsigned long long nchunks =
+        (unsigned long long)((size + kPersistChunk - 1) / kPersistChunk);
+    unsigned long long t = s_ticket[g & 1];
+    if (nchunks == 1 && t == 0) {
+      // This workgroup has the generation to itself, and keeps the ones that
+      // follow as long as their pairs fit one chunk.
+      AloneState al = {s_pairs, false, false, 0, 0};
+      int64_t n = size;
+      const int wait_g = g + 1;  // where the others wait
+      auto publish = [&](int k, unsigned long long v) {
+        atomic_store_agent(&a.gen_fill[(size_t)(half + k) * kGenRecWords + kReadyWord],
+                           kPublished | v);
+      };
+      while (true) {
+        unsigned children = 0;
+        al.more = g + 1 < hi;
+        const bool go = walk_chunk<true, kPersistPer, TAGS, kAlone, kPersistThreads>(
+            a, g, n, 0, sh, false, acc_f, acc_n, children, &al);
+        const bool over = (int64_t)children > a.queue_cap;
+        if (go && al.more && !over && children > 0 && children <= (unsigned)kPersistChunk) {
+          al.from_lds = true;
+          n = children;
+          ++g;
+          continue;
+        }
+        // the last generation run alone: over to everybody
+        if (!go && al.from_lds) {  // a paused walk resumes from the queue
+          uint64_t* q = (g & 1) ? a.wf1 : a.wf0;
+          for (int i = threadIdx.x; i < (int)n; i += kPersistThreads) q[i] = s_pairs[i];
+        }
+        if (threadIdx.x == 0) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+          __builtin_amdgcn_s_waitcnt(0);  // the write-back has completed
+          if (over) atomicOr(&a.flags[0], 1u);
+          const bool on = go && !over && al.more;
+          if (on) publish(g + 1, children);
+          if (wait_g < hi && !(on && wait_g == g + 1))
+            publish(wait_g, on ? kJump | (unsigned)(g + 1) : kStopped);
+        }
+        if (!go || over) return;
+        break;
+      }
+      ++g;
+      __syncthreads();  // slots of the same parity
+      continue;
+    }
+    while (t < nchunks) {
+      unsigned children = 0;
+      const bool go = walk_chunk<true, kPersistPer, TAGS, kShared, kPersistThreads>(
+          a, g, size, (int64_t)t * kPersistChunk, sh, false, acc_f, acc_n, children);
+      unsigned long long* next = sync + kGenRecWords;
+      if (!go) {  // the same in every workgroup with a chunk; the others hear it here
+        if (threadIdx.x == 0 && g + 1 < hi)
+          atomic_store_agent(&next[kReadyWord], kPublished | kStopped);
+        return;
+      }
+      if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __builtin_amdgcn_s_waitcnt(0);  // the write-back has completed
+        const unsigned long long mine = (1ull << 36) | children;
+        const unsigned long long sum = atomicAdd(&sync[kDoneWord], mine) + mine;
+        if (sum >> 36 == nchunks) {
+          const unsigned long long total = sum & ((1ull << 36) - 1);
+          if (g + 1 < hi)
+            atomic_store_agent(&next[kReadyWord],
+                               kPublished | ((int64_t)total > a.queue_cap ? kStopped : total));
+          s_ticket[g & 1] = nchunks;  // none is left
+        } else {
+          s_ticket[g & 1] = atomicAdd(&sync[kTicketWord], 1ull);
+        }
+      }
+      __syncthreads();
+      t = s_ticket[g & 1];
+    }
+    ++g;
   }
 }
 
@@ -840,6 +1126,31 @@ static int gen_blocks(int k, int64_t roots, int64_t queue_cap, int per, int bloc
   return nb < blocks ? (int)(nb > 0 ? nb : 1) : blocks;
 }
 
+// Whether generation k goes to k_walk_persist: by the hint where there is
+// one, else by the bound roots * 4^k and, for small trees, always. Up to
+// kPersistPairs (32 workgroups) a generation takes 5 to 9 us there, against
+// 12 us and a launch; past that the releases outgrow the launch.
+constexpr int64_t kPersistPairs = 65536;
+constexpr int32_t kPersistNodes = 1 << 14;
+constexpr int kPersistBlocks = 64;
+static bool persist_gen(int k, int64_t roots, int32_t num_nodes, const uint32_t* hint) {
+  if (hint && hint[k] != 0xFFFFFFFFu) return hint[k] <= kPersistPairs;
+  int64_t bound = roots;
+  for (int i = 0; i < k && bound <= kPersistPairs; ++i) bound *= 4;
+  return bound <= kPersistPairs || num_nodes <= kPersistNodes;
+}
+
+// Workgroups for generations [lo, hi): 1.5x the chunks of the largest as
+// hinted, or kPersistBlocks where a size is unknown.
+static int persist_blocks(int lo, int hi, const uint32_t* hint) {
+  int64_t most = 1;
+  for (int k = lo; k < hi; ++k) {
+    if (!hint || hint[k] == 0xFFFFFFFFu) return kPersistBlocks;
+    most = std::max<int64_t>(most, ((int64_t)hint[k] * 3 / 2 + kPersistChunk - 1) / kPersistChunk);
+  }
+  return (int)std::min<int64_t>(most, kPersistBlocks);
+}
+
 static hipEvent_t g_flat_events[2 * 1025];
 static int g_flat_events_ready = 0;
 
@@ -900,7 +1211,25 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
   if (batch < 2) batch = 2;
   while (true) {
     int end = g + batch < G ? g + batch : G;
+    const int half = G / 2;
+    const bool persist = a.gen_fill && !gen_ms && g0 == 0 && a.xcd_groups <= 1;
     for (int k = g; k < end; ++k) {
+      if (persist && k < half && persist_gen(k, a.num_roots, p->num_nodes, p->gen_pairs_hint)) {
+        int hi = k + 1;
+        while (hi < end && hi < half &&
+               persist_gen(hi, a.num_roots, p->num_nodes, p->gen_pairs_hint))
+          ++hi;
+        const int blocks = persist_blocks(k, hi, p->gen_pairs_hint);
+        if (hi == end && hi < half) hi = end = half;  // however many are left
+        if (a.far_tags)
+          hipLaunchKernelGGL(k_walk_persist<true>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
+                             half, k, hi);
+        else
+          hipLaunchKernelGGL(k_walk_persist<false>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
+                             half, k, hi);
+        k = hi - 1;
+        continue;
+      }
       if (gen_ms) YGG_CHECK(hipEventRecord(g_flat_events[2 * k], st));
       launch_flat(a, k, p->emit != 0, p->pairs_per_thread,
                   gen_blocks(k, a.num_roots, a.queue_cap, p->pairs_per_thread, blocks,
