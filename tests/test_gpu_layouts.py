@@ -70,6 +70,51 @@ def test_dense_interactions_match_oracle(ygg, name):
     assert np.array_equal(_bits(gd), _bits(od))
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("lens", [[3, 0, 1], [1, 0, 1], [5, 2, 2], [1023, 7, 0], [1024, 1, 1024],
+                                  [1500, 1025, 3]])
+def test_dense_kernel_row_lengths(ygg, lens, shift):
+    """Slot lengths around a thread's four elements and a workgroup's 1024,
+    with aligned output buffers (wide stores) and with buffers one element off
+    (narrow ones), against the slots filled here; the arithmetic is one
+    float32 subtraction, so bit for bit."""
+    from yggdrax_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(len(lens) + lens[0])
+    T, K = len(lens) * 2, max(1, max(lens))
+    counts = np.array(lens + lens[::-1], np.int64)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    src = rng.integers(0, T, max(1, off[-1]))
+    loff = np.array([0, 1, T], np.int32)      # two levels: one node, then the others
+    nbl = rng.permutation(T).astype(np.int32)
+    c = rng.normal(size=(T, 3)).astype(np.float32)
+    width, slots = T - 1, 2 * (T - 1)
+    want = {"s": np.full((slots, K), -1), "m": np.zeros((slots, K), bool),
+            "d": np.zeros((slots, K, 3), np.float32), "c": np.zeros(slots, np.int64)}
+    for level in (0, 1):
+        for k, node in enumerate(nbl[loff[level]:loff[level + 1]]):
+            row, n = level * width + k, counts[node]
+            want["c"][row] = n
+            want["s"][row, :n] = src[off[node]:off[node + 1]]
+            want["m"][row, :n] = True
+            want["d"][row, :n] = c[node] - c[src[off[node]:off[node + 1]]]
+    dev = [torch.from_numpy(a).cuda() for a in (off, counts, src, nbl, loff, c)]
+    n = slots * K
+    out = [torch.full((size + shift,), 77, dtype=t, device="cuda")[shift:] for size, t in
+           ((n, torch.int64), (3 * n, torch.float32), (n, torch.uint8), (slots, torch.int64))]
+    err = torch.empty(1, dtype=torch.int32, device="cuda")
+    _lib.check(lib.ygg_dense_interactions(
+        dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(), 1, T, int(off[-1]),
+        dev[3].data_ptr(), dev[4].data_ptr(), 2, width, K, dev[5].data_ptr(),
+        *(t.data_ptr() for t in out), err.data_ptr(), _lib.stream_ptr(err.device)), "dense")
+    s, d, m, cnt = (parity.np_(t) for t in out)
+    assert int(err) == 0
+    assert np.array_equal(s.reshape(slots, K), want["s"])
+    assert np.array_equal(m.reshape(slots, K).astype(bool), want["m"])
+    assert np.array_equal(_bits(d.reshape(slots, K, 3)), _bits(want["d"]))
+    assert np.array_equal(cnt, want["c"])
+
+
 def _grouped_np(g):
     return {f: parity.np_(getattr(g, f)) for f in g._fields}
 

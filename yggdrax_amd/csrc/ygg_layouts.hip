@@ -12,53 +12,148 @@
 namespace ygg {
 namespace {
 
-// One thread per (slot, entry): consecutive threads write consecutive
-// entries of one slot, so every output stream is written coalesced and the
-// slot's CSR row is read once per wavefront. A CSR row reaching outside the
-// num_far sources, or a source outside [0, num_nodes), is written as
-// padding and raises *err (checked by the caller after the launch).
-template <typename IdxT>
-__global__ void k_dense_m2l(const IdxT* __restrict__ offsets, const IdxT* __restrict__ counts,
-                            const IdxT* __restrict__ sources, int64_t num_nodes, int64_t num_far,
-                            const int32_t* __restrict__ nbl, const int32_t* __restrict__ loff,
-                            int num_levels, int64_t max_nodes, int64_t K,
-                            const float* __restrict__ center, IdxT* __restrict__ out_src,
-                            float* __restrict__ out_disp, uint8_t* __restrict__ out_mask,
-                            IdxT* __restrict__ out_counts, int32_t* __restrict__ err) {
+// A CSR row reaching outside the num_far sources, or a source outside
+// [0, num_nodes), is written as padding and raises *err (checked by the
+// caller after the launch).
+// Elements of the [num_levels][max_nodes][K] buffers, four consecutive ones
+// per thread and 1024 per workgroup and step: a workgroup divides once, its
+// threads step on from there, and with aligned buffers (VEC) whole spans go
+// out as 16-byte stores over contiguous runs, past the caches (nothing here
+// reads them again). Bound by the writes, 21 bytes per element: 2.16 GB (2^18
+// Plummer points, leaf 32) in 360 us, 6.0 TB/s where a plain fill reaches
+// 6.9; 491 us with one element per thread (two 64-bit divisions each), 469 us
+// with four per thread and stores of a thread's own, 565 us through LDS with
+// cached stores.
+constexpr int kDensePer = 4, kDenseThreads = 256, kDenseSpan = kDensePer * kDenseThreads;
+
+template <typename IdxT, bool VEC>
+__global__ __launch_bounds__(kDenseThreads) void k_dense_m2l(
+    const IdxT* __restrict__ offsets, const IdxT* __restrict__ counts,
+    const IdxT* __restrict__ sources, int64_t num_nodes, int64_t num_far,
+    const int32_t* __restrict__ nbl, const int32_t* __restrict__ loff, int num_levels,
+    int64_t max_nodes, int64_t K, const float* __restrict__ center, IdxT* __restrict__ out_src,
+    float* __restrict__ out_disp, uint8_t* __restrict__ out_mask, IdxT* __restrict__ out_counts,
+    int32_t* __restrict__ err) {
+  __shared__ __align__(16) IdxT s_src[VEC ? kDenseSpan : 1];
+  __shared__ __align__(16) float s_disp[VEC ? 3 * kDenseSpan : 1];
   const int64_t total = (int64_t)num_levels * max_nodes * K;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t slot = e / K;
-    const int64_t j = e - slot * K;
-    const int l = (int)(slot / max_nodes);
-    const int64_t s = slot - (int64_t)l * max_nodes;
-    const int64_t lc = (int64_t)loff[l + 1] - loff[l];
-    const int64_t node = s < lc ? (int64_t)nbl[loff[l] + s] : -1;
-    int64_t cnt = node >= 0 ? (int64_t)counts[node] : 0;
-    bool bad = cnt < 0;
-    if (bad) cnt = 0;
-    bool valid = j < cnt;
-    int64_t src = -1;
-    if (valid) {
-      const int64_t at = (int64_t)offsets[node] + j;
-      if (at < 0 || at >= num_far) {
-        bad = true;
-      } else {
-        src = (int64_t)sources[at];
-        if (src < 0 || src >= num_nodes) bad = true;
+  for (int64_t base = (int64_t)blockIdx.x * kDenseSpan; base < total;
+       base += (int64_t)gridDim.x * kDenseSpan) {
+    // uniform: the span's first slot, its level and place in it
+    const int64_t slot0 = base / K;
+    const int64_t l0 = slot0 / max_nodes;
+    const int64_t e0 = base + (int64_t)threadIdx.x * kDensePer;
+    if (e0 >= total) continue;
+    int64_t j = base - slot0 * K + (int64_t)threadIdx.x * kDensePer;
+    int64_t slot = slot0;
+    if (K >= kDenseSpan) {
+      if (j >= K) {  // at most one slot ends inside the span
+        j -= K;
+        ++slot;
       }
-      if (bad) {
-        valid = false;
-        src = -1;
+    } else {
+      const uint32_t q = (uint32_t)j / (uint32_t)K;
+      slot += q;
+      j -= (int64_t)q * K;
+    }
+    int64_t s = slot - l0 * max_nodes;
+    int l = (int)l0;
+    int64_t node = -1, cnt = 0, off = 0;
+    float tc[3] = {0.0f, 0.0f, 0.0f};
+    bool bad = false;
+    auto enter_slot = [&]() {
+      while (s >= max_nodes) {
+        s -= max_nodes;
+        ++l;
+      }
+      const int64_t lc = (int64_t)loff[l + 1] - loff[l];
+      node = s < lc ? (int64_t)nbl[loff[l] + s] : -1;
+      cnt = node >= 0 ? (int64_t)counts[node] : 0;
+      if (cnt < 0) {
+        bad = true;
+        cnt = 0;
+      }
+      if (j < cnt) {
+        off = (int64_t)offsets[node];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) tc[d] = center[3 * node + d];
+      }
+    };
+    enter_slot();
+    IdxT src[kDensePer];
+    float disp[3 * kDensePer];
+    uint32_t mask = 0;
+    const int64_t left = total - e0;
+#pragma unroll
+    for (int k = 0; k < kDensePer; ++k) {
+      src[k] = (IdxT)-1;
+      disp[3 * k] = disp[3 * k + 1] = disp[3 * k + 2] = 0.0f;
+      if (k < left) {
+        if (j == K) {
+          j = 0;
+          ++slot;
+          ++s;
+          enter_slot();
+        }
+        if (j < cnt) {
+          const int64_t at = off + j;
+          int64_t v = -1;
+          if (at >= 0 && at < num_far) v = (int64_t)sources[at];
+          if (v < 0 || v >= num_nodes) {
+            bad = true;
+          } else {
+            src[k] = (IdxT)v;
+            mask |= 1u << (8 * k);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) disp[3 * k + d] = tc[d] - center[3 * v + d];
+          }
+        }
+        if (j == 0) out_counts[slot] = (IdxT)cnt;
+        ++j;
       }
     }
     if (bad) *err = 1;
-    out_src[e] = (IdxT)src;
-    out_mask[e] = valid ? 1 : 0;
+    if (VEC && base + kDenseSpan <= total) {
+      // uniform: a whole span; sources and displacements change hands in LDS
+      // so that each wide store of a wavefront covers one run of memory
+      *(uint32_t*)(out_mask + e0) = mask;
+      const bool any = __syncthreads_or((int)mask);
+      if (any) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-      out_disp[3 * e + d] = valid ? center[3 * node + d] - center[3 * src + d] : 0.0f;
-    if (j == 0) out_counts[slot] = (IdxT)cnt;
+        for (int k = 0; k < kDensePer; ++k) {
+          s_src[threadIdx.x * kDensePer + k] = src[k];
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            s_disp[(threadIdx.x * kDensePer + k) * 3 + d] = disp[3 * k + d];
+        }
+        __syncthreads();
+      }
+      constexpr int kSrcWords = kDenseSpan * (int)sizeof(IdxT) / 16, kDispWords = kDenseSpan * 12 / 16;
+      typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+      const u32x4 ones = {~0u, ~0u, ~0u, ~0u}, zeros = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int k = 0; k < kSrcWords / kDenseThreads; ++k) {
+        const int i = k * kDenseThreads + (int)threadIdx.x;
+        __builtin_nontemporal_store(any ? ((const u32x4*)s_src)[i] : ones,
+                                    &((u32x4*)(out_src + base))[i]);
+      }
+#pragma unroll
+      for (int k = 0; k < kDispWords / kDenseThreads; ++k) {
+        const int i = k * kDenseThreads + (int)threadIdx.x;
+        __builtin_nontemporal_store(any ? ((const u32x4*)s_disp)[i] : zeros,
+                                    &((u32x4*)(out_disp + 3 * base))[i]);
+      }
+      if (any) __syncthreads();  // before the next span's values
+    } else {
+#pragma unroll
+      for (int k = 0; k < kDensePer; ++k) {
+        if (k >= left) break;
+        out_src[e0 + k] = src[k];
+        out_mask[e0 + k] = (uint8_t)(mask >> (8 * k));
+#pragma unroll
+        for (int d = 0; d < 3; ++d) out_disp[3 * (e0 + k) + d] = disp[3 * k + d];
+      }
+    }
   }
 }
 
@@ -442,19 +537,23 @@ int ygg_dense_interactions(const void* offsets, const void* counts, const void* 
   int rc;
   if ((rc = fill_u32((uint32_t*)error_flag, 0u, 1, st))) return rc;
   const int64_t total = (int64_t)num_levels * max_nodes * max_interactions;
-  dim3 g(grid_for(total, 256));
+  const dim3 g(grid_for(total, kDenseSpan));
+  // wide stores need 16-byte aligned sources and displacements, a 4-byte
+  // aligned mask
+  const bool vec = (((uintptr_t)out_sources | (uintptr_t)out_displacements) & 15) == 0 &&
+                   ((uintptr_t)out_mask & 3) == 0;
+  auto launch = [&](auto kernel, auto idx) {
+    using IdxT = decltype(idx);
+    hipLaunchKernelGGL(kernel, g, dim3(kDenseThreads), 0, st, (const IdxT*)offsets,
+                       (const IdxT*)counts, (const IdxT*)sources, num_nodes, num_far,
+                       nodes_by_level, level_offsets, num_levels, max_nodes, max_interactions,
+                       center, (IdxT*)out_sources, out_displacements, out_mask,
+                       (IdxT*)out_counts, error_flag);
+  };
   if (idx_i64)
-    hipLaunchKernelGGL(k_dense_m2l<int64_t>, g, dim3(256), 0, st, (const int64_t*)offsets,
-                       (const int64_t*)counts, (const int64_t*)sources, num_nodes, num_far,
-                       nodes_by_level, level_offsets, num_levels, max_nodes, max_interactions,
-                       center, (int64_t*)out_sources, out_displacements, out_mask,
-                       (int64_t*)out_counts, error_flag);
+    vec ? launch(k_dense_m2l<int64_t, true>, int64_t()) : launch(k_dense_m2l<int64_t, false>, int64_t());
   else
-    hipLaunchKernelGGL(k_dense_m2l<int32_t>, g, dim3(256), 0, st, (const int32_t*)offsets,
-                       (const int32_t*)counts, (const int32_t*)sources, num_nodes, num_far,
-                       nodes_by_level, level_offsets, num_levels, max_nodes, max_interactions,
-                       center, (int32_t*)out_sources, out_displacements, out_mask,
-                       (int32_t*)out_counts, error_flag);
+    vec ? launch(k_dense_m2l<int32_t, true>, int32_t()) : launch(k_dense_m2l<int32_t, false>, int32_t());
   YGG_LAUNCH_CHECK();
   return YGG_OK;
 }

@@ -39,7 +39,7 @@ def densify_interactions(tree, geometry: TreeGeometry,
     False and zeros. ``max_interactions`` is max(1, max count)."""
     topology = resolve_tree_topology(tree)
     require_fmm_core_topology(topology)
-    level_geometry = geometry_to_level_major(topology, geometry)
+    level_geometry = geometry_to_level_major(tree, geometry)
     dt = device_topology(tree)
     num_levels, max_nodes = (int(s) for s in level_geometry.node_indices.shape)
     dev = geometry.center.device
