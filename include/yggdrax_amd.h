@@ -219,15 +219,16 @@ int ygg_geometry(const float* pos_sorted, const float* particle_radius,
                  float* center, float* half_extent, float* radius, float* max_extent, void* ws,
                  size_t ws_bytes, void* stream);
 
+/* Nodes of each level (level_offsets [num_levels + 1]) and *out_widest, the
+ * largest of the counts and 1; out_counts is int64 if out_i64, else int32. */
+int ygg_level_counts(const int32_t* level_offsets, int32_t num_levels, void* out_counts,
+                     int out_i64, int32_t* out_widest, void* stream);
+
 /* Particle-order leaf table of a radix tree (_resolve_leaf_ordering,
  * yggdrax/_interactions_impl.py:1071-1103 without octree metadata). */
 int ygg_radix_leaf_order(int64_t num_leaves, int32_t* leaf_indices, int32_t* leaf_position,
                          void* stream);
 
-/* geometry_to_level_major (yggdrax/_geometry_impl.py:342-433): padded
- * [num_levels][max_nodes] level-major copies of the node geometry; slot j of
- * level l holds node nodes_by_level[level_offsets[l] + j] while j is below
- * the level's count, else zeros and node index -1. */
 int ygg_geometry_level_major(const float* center, const float* half_extent, const float* radius,
                              const float* max_extent, const int32_t* nodes_by_level,
                              const int32_t* level_offsets, int32_t num_levels, int64_t max_nodes,

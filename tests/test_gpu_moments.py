@@ -134,3 +134,39 @@ def test_mass_moments_large_root_total(ygg):
     com = (w / float(mm.mass[root])).cpu().numpy()
     got = parity.np_(mm.center_of_mass[root]).astype(np.float64)
     assert np.all(np.abs(got - com) <= 4 * np.spacing(np.abs(com).astype(np.float32)))
+
+
+@pytest.mark.parametrize("leaf,n", [(1, 700), (3, 1539), (8, 4097), (9, 4612), (17, 9001),
+                                    (33, 1), (64, 65), (65, 33_281), (1000, 5001),
+                                    (1025, 40_001)])
+def test_node_data_at_path_edges(ygg, leaf, n):
+    """Leaves of every lane grouping, with a remainder of four in the last;
+    segment trees of 1, 512 and more than 512 leaves; the level counts."""
+    g = torch.Generator().manual_seed(leaf * n)
+    pos = torch.randn(n, 3, generator=g).cuda()
+    mass = (torch.rand(n, generator=g) + 0.5).cuda()
+    tree, ps, ms, _ = ygg.build_tree(pos, mass, return_reordered=True, leaf_size=leaf)
+    rad = torch.rand(n, generator=g).cuda()
+    first, last = parity.np_(tree.node_ranges).astype(np.int64).T
+    for r in (None, rad):
+        geom = ygg.compute_tree_geometry(tree, ps, particle_radius=r)
+        lo = hi = parity.np_(ps)
+        if r is not None:
+            lo, hi = lo - parity.np_(r)[:, None], hi + parity.np_(r)[:, None]
+        lo = np.stack([lo[a:b + 1].min(0) for a, b in zip(first, last)])
+        hi = np.stack([hi[a:b + 1].max(0) for a, b in zip(first, last)])
+        assert np.array_equal(parity.np_(geom.center), np.float32(0.5) * (lo + hi))
+        assert np.array_equal(parity.np_(geom.half_extent),
+                              np.maximum(np.float32(0.5) * (hi - lo), np.float32(1e-6)))
+    lm = ygg.geometry_to_level_major(tree, geom)
+    want = np.bincount(parity.np_(tree.node_level).astype(np.int64), minlength=tree.num_levels)
+    assert np.array_equal(parity.np_(lm.level_counts), want)
+    assert lm.centers.shape == (tree.num_levels, max(int(want.max()), 1), 3)
+    mm = tm.compute_tree_mass_moments(tree, ps, ms)
+    m64 = parity.np_(ms).astype(np.float64)
+    p32 = parity.np_(ms)[:, None] * parity.np_(ps)
+    exp = {"mass": np.array([m64[a:b + 1].sum() for a, b in zip(first, last)], np.float32)}
+    exp["center_of_mass"] = (np.stack([p32[a:b + 1].astype(np.float64).sum(0)
+                                       for a, b in zip(first, last)]).astype(np.float32)
+                             / exp["mass"][:, None])
+    _check(mm, exp, (leaf, n))

@@ -147,6 +147,7 @@ _SIGS = {
     "ygg_octree_meta_workspace_bytes": (_SZ, [_I64]),
     "ygg_octree_meta": (_INT, [_P, _P, _I64, ctypes.POINTER(OctreeMetaPtrs), _P, _SZ, _P]),
     "ygg_geometry_workspace_bytes": (_SZ, [_I64]),
+    "ygg_level_counts": (_INT, [_P, _I32, _P, _INT, _P, _P]),
     "ygg_geometry_level_major": (_INT, [_P] * 6 + [_I32, _I64] + [_P] * 5 + [_INT, _P]),
     "ygg_dense_interactions": (_INT, [_P] * 3 + [_INT, _I64, _I64] + [_P] * 2 +
                                [_I32, _I64, _I64] + [_P] * 7),

@@ -86,8 +86,12 @@ def geometry_to_level_major(tree, geometry: TreeGeometry) -> LevelMajorTreeGeome
     if tuple(geometry.center.shape) != (dt.num_nodes, 3):
         raise ValueError(f"geometry.center must have shape ({dt.num_nodes}, 3)")
     off = dt.level_offsets[: num_levels + 1].to(torch.int32).contiguous()
-    counts = (off[1:] - off[:-1]).to(INDEX_DTYPE)
-    max_nodes = int(torch.clamp(counts, min=1).max())
+    counts = torch.empty(num_levels, dtype=INDEX_DTYPE, device=dev)
+    widest = torch.empty(1, dtype=torch.int32, device=dev)
+    _lib.check(lib.ygg_level_counts(
+        off.data_ptr(), num_levels, counts.data_ptr(), int(INDEX_DTYPE == torch.int64),
+        widest.data_ptr(), _lib.stream_ptr(dev)), "level counts")
+    max_nodes = int(widest)
     f32 = dict(dtype=torch.float32, device=dev)
     centers = torch.empty((num_levels, max_nodes, 3), **f32)
     halves = torch.empty((num_levels, max_nodes, 3), **f32)
