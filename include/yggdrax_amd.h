@@ -603,6 +603,21 @@ int ygg_near_lists_sort(const uint32_t* keys, const uint32_t* vals, int64_t n,
                         const int64_t* row_sub, const int32_t* leaf_nodes, int out_i64,
                         uint32_t* key_scratch, int64_t* row_offsets, void* neighbors,
                         void* counts, void* offsets, void* ws, size_t ws_bytes, void* stream);
+/* The small tables that go with a tree's lists, in one launch (all index
+ * outputs int64 if out_i64, else int32): out_leaves [L] = leaf_indices,
+ * out_particle_order [L] = num_internal + i, out_to_native [L] with
+ * out_to_native[leaf_indices[i] - num_internal] = i, out_block_offsets
+ * [L + 1] = 0; unless out_level_offsets is null, out_level_offsets
+ * [num_levels + 1] = far_offsets[level_offsets[i]]; unless out_longest is
+ * null, out_longest [longest_rows][2], whose column maxima are the longest row
+ * of far_offsets [L + num_internal + 1] and of near_offsets [L + 1]. */
+int ygg_list_tables(int64_t num_leaves, int64_t num_internal, const int32_t* leaf_indices,
+                    const int32_t* level_offsets, int32_t num_levels, const int64_t* far_offsets,
+                    const int64_t* near_offsets, int out_i64, void* out_leaves,
+                    void* out_particle_order, void* out_to_native, void* out_block_offsets,
+                    void* out_level_offsets, int64_t* out_longest, int32_t longest_rows,
+                    void* stream);
+
 /* The dense -1 padded [L][max_count] neighbour leaf rows from a near list
  * (neighbors int64 if out_i64, else int32). */
 int ygg_near_dense_from_list(int64_t num_leaves, const int64_t* row_offsets,

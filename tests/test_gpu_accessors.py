@@ -72,3 +72,28 @@ def test_traversal_diagnostics_lines(system, capsys, monkeypatch):
     monkeypatch.setattr(I, "_TRAVERSAL_DIAGNOSTICS", False)
     ygg.build_interactions_and_neighbors(tree, geom, theta=0.6, mac_type="dehnen")
     assert "[yggdrax.traversal]" not in capsys.readouterr().out
+
+
+@pytest.mark.parametrize("n,leaf", [(5, 8), (511 * 8, 8), (8193, 32), (20_000, 1)])
+def test_list_tables_against_tensor_formulas(n, leaf):
+    """One leaf, as many rows as threads of a workgroup less one, and rows for
+    the whole grid: the tables and the longest rows."""
+    import yggdrax_amd as ygg
+    from yggdrax_amd.interactions import _list_tables
+    from yggdrax_amd.tree import device_topology
+    pos = torch.from_numpy(inputs.uniform_cube(n, n)[0]).cuda()
+    dt = device_topology(ygg.build_octree(pos, torch.ones(n, device="cuda"), leaf_size=leaf))
+    T, L = dt.num_nodes, dt.num_leaves
+    far = torch.randint(0, 90, (T,), generator=torch.Generator().manual_seed(n)).cuda()
+    near = torch.randint(0, 90, (L,), generator=torch.Generator().manual_seed(L)).cuda()
+    far_off, near_off = (torch.cat([c.new_zeros(1), c.cumsum(0)]) for c in (far, near))
+    t = _list_tables(dt, far_off, near_off, True)
+    rows = torch.arange(L, device="cuda")
+    assert torch.equal(t.leaf_indices, dt.leaf_indices.to(t.leaf_indices.dtype))
+    assert torch.equal(t.particle_order.long(), rows + T - L)
+    assert torch.equal(t.to_native[dt.leaf_indices.long() - (T - L)].long(), rows)
+    assert t.block_offsets.numel() == L + 1 and not t.block_offsets.any()
+    assert torch.equal(t.level_offsets.long(),
+                       far_off[dt.level_offsets[:int(dt.num_levels) + 1].long()])
+    assert t.longest.amax(0).tolist() == [int(far.max()), int(near.max())]
+    assert _list_tables(dt).level_offsets is None

@@ -130,6 +130,7 @@ _SIGS = {
     "ygg_near_lists_sort_workspace_bytes": (_SZ, [_I64, _INT, _INT]),
     "ygg_near_lists_sort": (_INT, [_P, _P, _I64, _P, _I64, _INT, _INT, _P, _P, _INT, _P, _P,
                                    _P, _P, _P, _P, _SZ, _P]),
+    "ygg_list_tables": (_INT, [_I64, _I64, _P, _P, _I32, _P, _P, _INT] + [_P] * 6 + [_I32, _P]),
     "ygg_near_dense_from_list": (_INT, [_I64, _P, _P, _P, _I64, _INT, _P, _P]),
     "ygg_target_block_offsets_workspace_bytes": (_SZ, [_I64]),
     "ygg_target_block_offsets": (_INT, [_I64, _P, _I64, _P, _P, _SZ, _P]),

@@ -29,7 +29,7 @@ from . import _lib
 from .dtypes import INDEX_DTYPE
 from .geometry import TreeGeometry
 from .interactions import (FLAT_GRID_BLOCKS, MAC_TYPES, NodeInteractionList, NodeNeighborList,
-                           _WalkContext, _ladder, _leaf_tables, _run_walk_flat)
+                           _WalkContext, _ladder, _list_tables, _run_walk_flat)
 from .tree import _assemble_tree, _ptrs, build_octree, build_tree
 
 
@@ -412,8 +412,7 @@ class _ForestContext(_WalkContext):
             ctypes.c_float(float(dehnen_radius_scale)).value, self.nodes.data_ptr(),
             self.roots.data_ptr(), self.stream), "batch walk nodes")
         self.host_status = torch.zeros(MAX_GENERATIONS + 16, dtype=torch.int32, pin_memory=True)
-        self.gen_sizes = torch.empty(MAX_GENERATIONS + 1, dtype=torch.int32, device=self.dev)
-        self.flags = torch.empty(4, dtype=torch.int32, device=self.dev)
+        self._alloc_status()
         self.decisions = torch.empty(3, dtype=torch.int64, device=self.dev)
         self.timing = WALK_TIMING["enabled"]
         max_levels = int(trees.scalars[:, 0].max())
@@ -474,7 +473,7 @@ class BatchedLists:
         idx = INDEX_DTYPE
         dev = self.neighbors.device
         L = l1 - l0
-        leaf_indices, po, p2n = _leaf_tables(dt)
+        leaf_indices, po, p2n, block_offsets = _list_tables(dt)[:4]
         nbrs = NodeNeighborList(
             offsets=no, neighbors=self.neighbors[nbase:nend], leaf_indices=leaf_indices,
             counts=self.near_counts[l0:l1], particle_order_leaf_indices=po,
@@ -483,7 +482,7 @@ class BatchedLists:
             target_block_leaf_ids=torch.zeros(0, dtype=idx, device=dev),
             target_block_source_leaf_ids=torch.zeros((0, 0), dtype=idx, device=dev),
             target_block_valid_mask=torch.zeros((0, 0), dtype=torch.bool, device=dev),
-            target_block_offsets=torch.zeros(L + 1, dtype=idx, device=dev), target_block_size=0)
+            target_block_offsets=block_offsets, target_block_size=0)
         return inter, nbrs
 
 

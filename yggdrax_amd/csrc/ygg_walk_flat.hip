@@ -967,6 +967,53 @@ __global__ __launch_bounds__(256) void k_near_dense_from_list(
   }
 }
 
+// The small tables of a pair of lists in one launch: the leaves in list order,
+// in particle order, and the inverse of the two; zeroed target-block offsets;
+// the far offsets of the levels; and, per workgroup, the longest far and near
+// row. Every one of them is an elementwise or reducing launch of 6 to 8 us of
+// host time otherwise, 16 of them behind each walk
+// (with the status words in one copy, a step at 512 points 1310 -> 1240 us, at
+// 100 003 points 1671 -> 1639 us).
+template <typename IdxT>
+__global__ __launch_bounds__(256) void k_list_tables(
+    int64_t L, int64_t NI, const int32_t* __restrict__ leaf_indices, IdxT* __restrict__ leaves,
+    IdxT* __restrict__ particle_order, IdxT* __restrict__ to_native,
+    IdxT* __restrict__ block_offsets, const int32_t* __restrict__ level_nodes, int levels1,
+    const int64_t* __restrict__ far_off, IdxT* __restrict__ level_off, int64_t T,
+    const int64_t* __restrict__ near_off, int64_t* __restrict__ longest) {
+  const int64_t first = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = first; i <= L; i += step) {
+    block_offsets[i] = (IdxT)0;
+    if (i == L) break;
+    const int64_t node = leaf_indices[i];
+    leaves[i] = (IdxT)node;
+    particle_order[i] = (IdxT)(NI + i);
+    if (node >= NI && node < NI + L) to_native[node - NI] = (IdxT)i;
+  }
+  for (int64_t i = first; i < levels1; i += step) level_off[i] = (IdxT)far_off[level_nodes[i]];
+  if (!longest) return;
+  int64_t mf = 0, mn = 0;
+  for (int64_t i = first; i < T; i += step) mf = max(mf, far_off[i + 1] - far_off[i]);
+  for (int64_t i = first; i < L; i += step) mn = max(mn, near_off[i + 1] - near_off[i]);
+#pragma unroll
+  for (int o = YGG_WAVE / 2; o > 0; o >>= 1) {
+    mf = max(mf, (int64_t)__shfl_xor((long long)mf, o, YGG_WAVE));
+    mn = max(mn, (int64_t)__shfl_xor((long long)mn, o, YGG_WAVE));
+  }
+  __shared__ int64_t s_f[4], s_n[4];
+  const int w = threadIdx.x / YGG_WAVE;
+  if (lane_id() == 0) {
+    s_f[w] = mf;
+    s_n[w] = mn;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    longest[2 * blockIdx.x] = max(max(s_f[0], s_f[1]), max(s_f[2], s_f[3]));
+    longest[2 * blockIdx.x + 1] = max(max(s_n[0], s_n[1]), max(s_n[2], s_n[3]));
+  }
+}
+
 // ---- batched (forest) lists -> per-system lists ---------------------------------
 // Per far entry, the target's system (largest s with node_off(s) <= t) by a
 // binary search over the node offsets, staged in LDS (seg_stage).
@@ -1242,13 +1289,20 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
     // every batch lets the batch's one copy carry them to the host.
     if (a.gen_fill) hipLaunchKernelGGL(k_unpack_totals, dim3(1), dim3(64), 0, st, a, G);
     YGG_LAUNCH_CHECK();
-    YGG_CHECK(hipMemcpyAsync(host_status, p->gen_sizes, sizeof(uint32_t) * (G + 1),
+    // device words that lie as host_status does take one copy instead of three
+    // (5 us each)
+    const bool one_copy = a.gen_fill && p->flags == p->gen_sizes + G + 1 &&
+                          (const void*)a.counters == (const void*)(p->gen_sizes + G + 5);
+    YGG_CHECK(hipMemcpyAsync(host_status, p->gen_sizes,
+                             sizeof(uint32_t) * (one_copy ? G + 9 : G + 1),
                              hipMemcpyDeviceToHost, st));
-    YGG_CHECK(hipMemcpyAsync(host_status + G + 1, p->flags, sizeof(uint32_t) * 4,
-                             hipMemcpyDeviceToHost, st));
-    if (a.gen_fill)
-      YGG_CHECK(hipMemcpyAsync(host_status + G + 5, a.counters, sizeof(uint64_t) * 2,
+    if (!one_copy) {
+      YGG_CHECK(hipMemcpyAsync(host_status + G + 1, p->flags, sizeof(uint32_t) * 4,
                                hipMemcpyDeviceToHost, st));
+      if (a.gen_fill)
+        YGG_CHECK(hipMemcpyAsync(host_status + G + 5, a.counters, sizeof(uint64_t) * 2,
+                                 hipMemcpyDeviceToHost, st));
+    }
     YGG_CHECK(hipStreamSynchronize(st));
     const uint32_t* fl = host_status + G + 1;
     int done = -1;
@@ -1576,6 +1630,38 @@ int ygg_near_lists_sort(const uint32_t* keys, const uint32_t* vals, int64_t n,
   else
     hipLaunchKernelGGL(k_near_rows<int32_t>, gr, dim3(256), 0, st, L, row_offsets,
                        (int32_t*)counts, (int32_t*)offsets);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
+int ygg_list_tables(int64_t num_leaves, int64_t num_internal, const int32_t* leaf_indices,
+                    const int32_t* level_offsets, int32_t num_levels, const int64_t* far_offsets,
+                    const int64_t* near_offsets, int out_i64, void* out_leaves,
+                    void* out_particle_order, void* out_to_native, void* out_block_offsets,
+                    void* out_level_offsets, int64_t* out_longest, int32_t longest_rows,
+                    void* stream) {
+  if (num_leaves < 0 || num_internal < 0 || !out_block_offsets) return YGG_ERR_ARG;
+  if (num_leaves > 0 && (!leaf_indices || !out_leaves || !out_particle_order || !out_to_native))
+    return YGG_ERR_ARG;
+  if (out_level_offsets && (!level_offsets || !far_offsets || num_levels < 0)) return YGG_ERR_ARG;
+  if (out_longest && (!far_offsets || !near_offsets || longest_rows < 1)) return YGG_ERR_ARG;
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t T = num_internal + num_leaves;
+  const int levels1 = out_level_offsets ? num_levels + 1 : 0;
+  const dim3 g(out_longest ? (unsigned)longest_rows
+                           : (unsigned)grid_for(std::max<int64_t>(num_leaves, levels1) + 1, 256));
+  if (out_i64)
+    hipLaunchKernelGGL(k_list_tables<int64_t>, g, dim3(256), 0, st, num_leaves, num_internal,
+                       leaf_indices, (int64_t*)out_leaves, (int64_t*)out_particle_order,
+                       (int64_t*)out_to_native, (int64_t*)out_block_offsets, level_offsets,
+                       levels1, far_offsets, (int64_t*)out_level_offsets, T, near_offsets,
+                       out_longest);
+  else
+    hipLaunchKernelGGL(k_list_tables<int32_t>, g, dim3(256), 0, st, num_leaves, num_internal,
+                       leaf_indices, (int32_t*)out_leaves, (int32_t*)out_particle_order,
+                       (int32_t*)out_to_native, (int32_t*)out_block_offsets, level_offsets,
+                       levels1, far_offsets, (int32_t*)out_level_offsets, T, near_offsets,
+                       out_longest);
   YGG_LAUNCH_CHECK();
   return YGG_OK;
 }

@@ -388,8 +388,7 @@ class _WalkContext:
             ctypes.c_float(float(dehnen_radius_scale)).value, self.nodes.data_ptr(),
             self.stream), "walk_prepare_nodes")
         self.host_status = torch.zeros(MAX_GENERATIONS + 16, dtype=torch.int32, pin_memory=True)
-        self.gen_sizes = torch.empty(MAX_GENERATIONS + 1, dtype=torch.int32, device=self.dev)
-        self.flags = torch.empty(4, dtype=torch.int32, device=self.dev)
+        self._alloc_status()
         self.decisions = torch.empty(3, dtype=torch.int64, device=self.dev)
         self.timing = WALK_TIMING["enabled"]
         self.gen_hint = int(1.5 * max(1, dt.num_levels)) + 4
@@ -398,6 +397,14 @@ class _WalkContext:
         self.grid_blocks = FLAT_GRID_BLOCKS
         self.pairs_per_thread = WALK_PAIRS_PER_THREAD
         self.kernel_log = WALK_TIMING["log"]
+
+    def _alloc_status(self):
+        # the walk's device words in host_status order, from the second word
+        # on so that the two 64-bit totals are aligned: one copy reads them
+        words = torch.empty(MAX_GENERATIONS + 10, dtype=torch.int32, device=self.dev)
+        self.gen_sizes = words[1:MAX_GENERATIONS + 2]
+        self.flags = words[MAX_GENERATIONS + 2:MAX_GENERATIONS + 6]
+        self.counters = words[MAX_GENERATIONS + 6:].view(torch.int64)
 
     def run_flat(self, *, emit: bool, queue_cap: int, far_cap: int = 0, near_cap: int = 0,
                  gen_hint: int = 0, hist_gen: int = -1, node_hist=None, grid_blocks: int = 0,
@@ -421,7 +428,6 @@ class _WalkContext:
         # generation 0 holds every root pair, so the queue holds at least those
         Q = max(4, int(queue_cap), 0 if roots is None else int(roots.numel()))
         wf = torch.empty((2, Q), dtype=torch.int64, device=dev)
-        counters = torch.empty(2, dtype=torch.int64, device=dev)
         # the counting walk adds its totals into spread lanes instead of
         # reserving per chunk on two contended addresses
         spread = None if emit else torch.empty(2 * SPREAD_LANES, dtype=torch.int64, device=dev)
@@ -448,7 +454,7 @@ class _WalkContext:
         p.nodes = self.nodes.data_ptr()
         p.wf0, p.wf1 = wf[0].data_ptr(), wf[1].data_ptr()
         p.gen_sizes, p.flags = self.gen_sizes.data_ptr(), self.flags.data_ptr()
-        p.counters = counters.data_ptr()
+        p.counters = self.counters.data_ptr()
         p.far_keys, p.far_vals = _lib.ptr(fk), _lib.ptr(fv)
         p.near_keys, p.near_vals = _lib.ptr(nk), _lib.ptr(nv)
         p.hist_gen, p.node_hist = int(hist_gen), _lib.ptr(node_hist)
@@ -753,7 +759,7 @@ class _FlatResult(NamedTuple):
     stats: dict
     # the list outputs, when the sorts wrote them directly (fused last pass)
     inter: Optional["NodeInteractionList"] = None
-    near: Optional[tuple] = None       # (neighbors, counts, offsets)
+    near: Optional[tuple] = None       # (neighbors, counts, offsets, _ListTables)
 
 
 def row_lists_digit_bits(end_bit: int, n: int) -> int:
@@ -766,14 +772,15 @@ def row_lists_digit_bits(end_bit: int, n: int) -> int:
     return autotune.sort_digit_bits(4, end_bit, n) if n else 8
 
 
-def _fused_lists(em: dict, dt: DeviceTopology):
+def _fused_lists(em: dict, dt: DeviceTopology, longest: bool = False):
     """Far and near row lists in the reference's layouts, grouped by row
     by ygg_far_lists_sort / ygg_near_lists_sort (bucketing kernels, or the
     row-key sort whose last pass writes the lists). The near lists, the
     longer of the two, are launched first on the current stream; the far
     lists follow on a side stream, ordered after the walk only. Returns the
-    NodeInteractionList, the near (neighbors, counts, offsets) and both
-    int64 row offset arrays."""
+    NodeInteractionList, the near (neighbors, counts, offsets, _ListTables,
+    these with the `longest` rows if asked for) and both int64 row offset
+    arrays."""
     lib = _lib.load()
     dev = dt.parent.device
     idx = INDEX_DTYPE
@@ -828,13 +835,13 @@ def _fused_lists(em: dict, dt: DeviceTopology):
     main.wait_stream(side)
     for t in (sources, targets, levels, counts, counts32, node_off, far_off, fsorted, fws):
         t.record_stream(main)
-    nl = int(dt.num_levels)
-    level_offsets = far_off[dt.level_offsets[: nl + 1].long()].to(idx)
+    tables = _list_tables(dt, far_off, near_off, longest)
+    level_offsets = tables.level_offsets
     if nf == 0:
         node_off = torch.zeros(T + 1, dtype=idx, device=dev)
-        level_offsets = torch.zeros(nl + 1, dtype=idx, device=dev)
+        level_offsets = torch.zeros_like(level_offsets)
     inter = NodeInteractionList(node_off, sources, targets, counts, level_offsets, levels)
-    return inter, (neighbors, ncounts, noff), fsorted, far_off, near_off
+    return inter, (neighbors, ncounts, noff, tables), fsorted, far_off, near_off
 
 
 def _sort_entries(keys, vals, n, rows, exact_keys=False):
@@ -1029,18 +1036,21 @@ def _run_walk_flat(ctx: _WalkContext, dt: DeviceTopology, lad: _Ladder,
                     f"total_far_pairs={nf} total_near_pairs={nn} hinted={hinted} "
                     f"stream_growths={em.get('stream_growths', 0)}")
     inter = near = None
+    want_max = need_max or strict_int32 or not lad.use_count
     if callable(fused_lists):  # the caller's own list layout (batched mode)
         inter, near, fk, far_off, near_off = fused_lists(em)
         fv = nv = None
     elif fused_lists:
-        inter, near, fk, far_off, near_off = _fused_lists(em, dt)
+        inter, near, fk, far_off, near_off = _fused_lists(em, dt, want_max)
         fv = nv = None
     else:
         (fk, fv, far_off), (_, nv, near_off) = _sort_far_and_near(
             em["far_keys"], em["far_vals"], nf, T, em["near_keys"], em["near_vals"], nn, L)
     _record_stage("dual_split_shared_combined_fill", t_stage, ctx.dev)
     max_far = max_near = None
-    if need_max or strict_int32 or not lad.use_count:
+    if want_max and near is not None and isinstance(near[-1], _ListTables):
+        max_far, max_near = (max(c) for c in zip(*near[-1].longest.tolist()))
+    elif want_max:
         mx = torch.stack([torch.diff(far_off).max(), torch.diff(near_off).max()]).tolist()
         max_far, max_near = int(mx[0]), int(mx[1])
     stats = dict(peak=em["peak"], gen_sizes=em["gen_sizes"], decisions=em["decisions"],
@@ -1068,7 +1078,7 @@ def _flat_outputs(fr: _FlatResult, dt: DeviceTopology, topo, neighbor_positions:
     i64 = int(idx == torch.int64)
     st = _lib.stream_ptr(dev)
     if fr.inter is not None:
-        neighbors, ncounts, noff = fr.near
+        neighbors, ncounts, noff, tables = fr.near
         maxc = fr.stats["max_near"] if neighbor_positions else 0
         nlp = torch.empty((L, maxc), dtype=idx, device=dev)
         if maxc > 0:
@@ -1076,7 +1086,7 @@ def _flat_outputs(fr: _FlatResult, dt: DeviceTopology, topo, neighbor_positions:
                                                     neighbors.data_ptr(),
                                                     dt.leaf_position.data_ptr(), maxc, i64,
                                                     nlp.data_ptr(), st), "near dense")
-        leaf_indices, po, p2n = _leaf_tables(dt)
+        leaf_indices, po, p2n, block_offsets = tables[:4]
         return fr.inter, _with_target_blocks(NodeNeighborList(
             offsets=noff, neighbors=neighbors, leaf_indices=leaf_indices, counts=ncounts,
             particle_order_leaf_indices=po, particle_order_to_native_leaf=p2n,
@@ -1084,7 +1094,7 @@ def _flat_outputs(fr: _FlatResult, dt: DeviceTopology, topo, neighbor_positions:
             target_block_leaf_ids=torch.zeros(0, dtype=idx, device=dev),
             target_block_source_leaf_ids=torch.zeros((0, 0), dtype=idx, device=dev),
             target_block_valid_mask=torch.zeros((0, 0), dtype=torch.bool, device=dev),
-            target_block_offsets=torch.zeros(L + 1, dtype=idx, device=dev),
+            target_block_offsets=block_offsets,
             target_block_size=0), dt)
     nf = fr.stats["far_total"]
     nn = fr.stats["near_total"]
@@ -1100,11 +1110,6 @@ def _flat_outputs(fr: _FlatResult, dt: DeviceTopology, topo, neighbor_positions:
         targets.data_ptr(), levels.data_ptr(), counts.data_ptr(), node_off.data_ptr(),
         counts32.data_ptr(), st), "far lists")
     nl = int(topo.num_levels)
-    level_offsets = fr.far_off[dt.level_offsets[: nl + 1].long()].to(idx)
-    if nf == 0:
-        node_off = torch.zeros(T + 1, dtype=idx, device=dev)
-        level_offsets = torch.zeros(nl + 1, dtype=idx, device=dev)
-    inter = NodeInteractionList(node_off, sources, targets, counts, level_offsets, levels)
     maxc = fr.stats["max_near"] if neighbor_positions else 0
     neighbors = torch.empty(nn, dtype=idx, device=dev)
     nlp = torch.empty((L, maxc), dtype=idx, device=dev)
@@ -1114,14 +1119,18 @@ def _flat_outputs(fr: _FlatResult, dt: DeviceTopology, topo, neighbor_positions:
         L, fr.near_off.data_ptr(), fr.near_vals.data_ptr(), dt.leaf_position.data_ptr(), maxc,
         i64, neighbors.data_ptr(), nlp.data_ptr() if maxc > 0 else None, ncounts.data_ptr(),
         noff.data_ptr(), st), "near lists")
-    leaf_indices, po, p2n = _leaf_tables(dt)
+    leaf_indices, po, p2n, block_offsets, level_offsets, _ = _list_tables(dt, fr.far_off)
+    if nf == 0:
+        node_off = torch.zeros(T + 1, dtype=idx, device=dev)
+        level_offsets = torch.zeros(nl + 1, dtype=idx, device=dev)
+    inter = NodeInteractionList(node_off, sources, targets, counts, level_offsets, levels)
     nbrs = NodeNeighborList(
         offsets=noff, neighbors=neighbors, leaf_indices=leaf_indices, counts=ncounts,
         particle_order_leaf_indices=po, particle_order_to_native_leaf=p2n,
         neighbor_leaf_positions=nlp, target_block_leaf_ids=torch.zeros(0, dtype=idx, device=dev),
         target_block_source_leaf_ids=torch.zeros((0, 0), dtype=idx, device=dev),
         target_block_valid_mask=torch.zeros((0, 0), dtype=torch.bool, device=dev),
-        target_block_offsets=torch.zeros(L + 1, dtype=idx, device=dev), target_block_size=0)
+        target_block_offsets=block_offsets, target_block_size=0)
     return inter, _with_target_blocks(nbrs, dt)
 
 
@@ -1235,15 +1244,39 @@ def _to_interactions(raw: _RawWalk, dt: DeviceTopology, topo) -> NodeInteraction
     return NodeInteractionList(offsets, sources, targets, counts_out, level_offsets, levels)
 
 
-def _leaf_tables(dt: DeviceTopology):
+class _ListTables(NamedTuple):
+    leaf_indices: torch.Tensor
+    particle_order: torch.Tensor       # the leaves by particle order
+    to_native: torch.Tensor            # row of each of them in leaf_indices
+    block_offsets: torch.Tensor        # zeros [L + 1]
+    level_offsets: Optional[torch.Tensor]  # far offsets of the levels
+    longest: Optional[torch.Tensor]    # [k, 2]: column maxima are the longest rows
+
+
+def _list_tables(dt: DeviceTopology, far_off: Optional[torch.Tensor] = None,
+                 near_off: Optional[torch.Tensor] = None, longest: bool = False) -> _ListTables:
+    """The small tables that go with a tree's lists, by one kernel
+    (ygg_list_tables)."""
+    lib = _lib.load()
     dev = dt.parent.device
     idx = INDEX_DTYPE
     L, NI = dt.num_leaves, dt.num_internal
-    po = torch.arange(NI, NI + L, dtype=idx, device=dev)
-    p2n = torch.empty(L, dtype=idx, device=dev)
-    native = dt.leaf_indices.long() - NI
-    p2n[native] = torch.arange(L, dtype=idx, device=dev)
-    return dt.leaf_indices.to(idx), po, p2n
+    leaves = dt.leaf_indices.to(torch.int32).contiguous()
+    outs = [torch.empty(L, dtype=idx, device=dev) for _ in range(3)]
+    outs.append(torch.empty(L + 1, dtype=idx, device=dev))
+    nl = int(dt.num_levels)
+    level_off = levels = rows = None
+    if far_off is not None:
+        levels = dt.level_offsets[: nl + 1]
+        level_off = torch.empty(levels.numel(), dtype=idx, device=dev)
+    if longest:
+        rows = torch.empty((min(64, (L + NI) // 256 + 1), 2), dtype=torch.int64, device=dev)
+    _lib.check(lib.ygg_list_tables(
+        L, NI, leaves.data_ptr(), _lib.ptr(levels), level_off.numel() - 1 if levels is not None
+        else 0, _lib.ptr(far_off), _lib.ptr(near_off), int(idx == torch.int64),
+        *[t.data_ptr() for t in outs], _lib.ptr(level_off), _lib.ptr(rows),
+        rows.shape[0] if longest else 0, _lib.stream_ptr(dev)), "list tables")
+    return _ListTables(*outs, level_off, rows)
 
 
 def _target_block_size() -> int:
@@ -1300,7 +1333,7 @@ def _to_neighbors(raw: Optional[_RawWalk], dt: DeviceTopology) -> NodeNeighborLi
     dev = dt.parent.device
     idx = INDEX_DTYPE
     L = dt.num_leaves
-    leaf_indices, po, p2n = _leaf_tables(dt)
+    leaf_indices, po, p2n, block_offsets = _list_tables(dt)[:4]
     if raw is None:
         counts = torch.zeros(L, dtype=torch.int32, device=dev)
     else:
@@ -1324,7 +1357,7 @@ def _to_neighbors(raw: Optional[_RawWalk], dt: DeviceTopology) -> NodeNeighborLi
         target_block_leaf_ids=torch.zeros(0, dtype=idx, device=dev),
         target_block_source_leaf_ids=torch.zeros((0, 0), dtype=idx, device=dev),
         target_block_valid_mask=torch.zeros((0, 0), dtype=torch.bool, device=dev),
-        target_block_offsets=torch.zeros(L + 1, dtype=idx, device=dev), target_block_size=0), dt)
+        target_block_offsets=block_offsets, target_block_size=0), dt)
 
 
 def _node_order_rows(values_lm: torch.Tensor, inter: NodeInteractionList,
