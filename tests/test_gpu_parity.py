@@ -308,3 +308,41 @@ def test_geometry_to_level_major_matches_oracle(ygg, name):
         got, exp = parity.np_(getattr(lm, f)), np.asarray(rl[f])
         assert got.shape == exp.shape, f
         assert np.array_equal(got, exp.astype(got.dtype)), f
+
+
+def _paired_points(n, seed):
+    """Every second point a copy of its neighbour or a few last bits off, and a
+    geometric chain towards a corner (cells of every depth)."""
+    pos, mass = inputs.uniform_cube(n, seed)
+    pos[1::2] = pos[: n // 2 * 2: 2]
+    pos[1::4] += np.float32(2e-6)
+    k = np.arange(min(n // 4, 60))
+    pos[2 * k] = (np.float32(0.9) * np.float32(0.75) ** k[:, None]).astype(np.float32)
+    return pos, mass
+
+
+@pytest.mark.parametrize("points", [inputs.uniform_cube, _paired_points])
+@pytest.mark.parametrize("n,leaf", [(2, 1), (65, 32), (512, 1), (513, 1), (1535, 3), (2048, 1),
+                                    (2049, 1)])
+def test_build_at_workgroup_edges(ygg, points, n, leaf):
+    """Trees of 3 nodes, of the most nodes that 256 and 1024 threads hold (L =
+    512, 2048), and one leaf more; cells of every depth and duplicate codes."""
+    pos, mass = points(n, 17 + n)
+    for octree in (False, True):
+        ref = (oracle.build_octree if octree else oracle.build_tree)(pos, mass, leaf_size=leaf)
+        tree = (ygg.build_octree if octree else ygg.build_tree)(
+            torch.from_numpy(pos).cuda(), torch.from_numpy(mass).cuda(), leaf_size=leaf)
+        print(f"[parity] {points.__name__} n={n} leaf={leaf} octree={octree}", flush=True)
+        parity.assert_topology_equal(tree, ref, octree=octree)
+
+
+@pytest.mark.parametrize("n", [1, 4095, 4097, 16384, 16385])
+def test_scan_at_path_edges(ygg, n):
+    from yggdrax_amd.interactions import _scan
+    g = torch.Generator().manual_seed(n)
+    counts = torch.randint(0, 1 << 30, (n + 3,), generator=g, dtype=torch.int32).cuda()
+    order = torch.randperm(n + 3, generator=g)[:n].to(torch.int32).cuda()
+    for c, gather in ((counts[:n].contiguous(), None), (counts, order)):
+        want = (c if gather is None else c[gather.long()]).long().cumsum(0)
+        got = _scan(c, gather)
+        assert int(got[0]) == 0 and torch.equal(got[1:], want)

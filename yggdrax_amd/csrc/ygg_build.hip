@@ -283,8 +283,10 @@ __global__ __launch_bounds__(256) void k_scatter_sorted(const float* __restrict_
 // ---- Karras radix build (_tree_impl.py:1117-1270) ---------------------------
 __global__ __launch_bounds__(256) void k_leaves(const uint64_t* __restrict__ sc, int64_t n,
                                                 int64_t leaf, int L, uint64_t* __restrict__ lc,
-                                                int32_t* __restrict__ ranges) {
+                                                int32_t* __restrict__ ranges,
+                                                int32_t* __restrict__ scal) {
   int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < 8) scal[j] = 0;
   if (j >= L) return;
   int64_t s = (int64_t)j * leaf;
   int64_t e = min(s + leaf, n);
@@ -416,8 +418,10 @@ __global__ __launch_bounds__(256) void k_pd_finish(const int64_t* __restrict__ d
 
 // ---- explicit octree metadata (octree.py:168-550) ---------------------------
 __global__ void k_oct_resolve(const uint64_t* __restrict__ sc, const int32_t* __restrict__ ranges,
-                              int L, uint64_t* __restrict__ rc, int32_t* __restrict__ rd) {
+                              int L, uint64_t* __restrict__ rc, int32_t* __restrict__ rd,
+                              int32_t* __restrict__ scal) {
   int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < 4) scal[j] = 0;
   if (j >= L) return;
   int64_t node = (int64_t)(L - 1) + j;
   uint64_t f = sc[ranges[2 * node]], l = sc[ranges[2 * node + 1]];
@@ -609,22 +613,372 @@ __global__ void k_radix_to_oct(const uint64_t* __restrict__ sc, const int32_t* _
   if (k >= NI) leaf_key[k - NI] = (uint32_t)pos;
 }
 
-__global__ void k_leaf_order(const uint32_t* __restrict__ native, int NI, int L, int T,
+// leaf_indices[k] = node of native leaf k (NI + k without an order), and the
+// inverse leaf_position, -1 at internal nodes.
+__global__ void k_leaf_order(const uint32_t* __restrict__ native, int NI, int L,
                              int32_t* __restrict__ leaf_indices,
                              int32_t* __restrict__ leaf_position) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < T) leaf_position[k] = -1;
-  (void)L;
-}
-
-__global__ void k_leaf_order2(const uint32_t* __restrict__ native, int NI, int L,
-                              int32_t* __restrict__ leaf_indices,
-                              int32_t* __restrict__ leaf_position) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < NI) leaf_position[k] = -1;
   if (k >= L) return;
-  int32_t node = NI + (native ? (int32_t)native[k] : k);
+  const int32_t node = NI + (native ? (int32_t)native[k] : k);
   leaf_indices[k] = node;
   leaf_position[node] = k;
+}
+
+// ---- small trees: the whole build in one workgroup ---------------------------
+// Trees of fewer nodes than the workgroup holds (four per thread) are bound by
+// launches: 9 for the radix build and 21 for the octree, of 4 us each for the
+// host, with 2 to 6 us of work on a few CUs behind each. One workgroup runs the
+// same steps with barriers between them and keeps codes, addresses and parent
+// links in LDS, where the searches and parent walks are short chains: a step at 512 points
+// 1240 -> 1078 us, at 10 007 points 1206 -> 1151 us.
+constexpr int kSmallItems = 4;
+constexpr int kSmallNodes = 1024 * kSmallItems;
+
+// Radix build of L >= 2 leaves, 2 L - 1 < THREADS * kSmallItems nodes
+// (k_leaves, k_karras, k_levels_walk, k_level_offsets and the sort by level).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_radix_small(const uint64_t* __restrict__ sc,
+                                                         int64_t n, int64_t leaf, int L,
+                                                         YggRadixTopology o) {
+  constexpr int kItems = kSmallItems, kCap = THREADS * kItems, kW = THREADS / YGG_WAVE;
+  __shared__ uint64_t s_code[kCap / 2];
+  __shared__ uint32_t s_par[kCap];
+  __shared__ uint32_t s_lev[64];
+  __shared__ uint16_t s_hist[kW][256];
+  __shared__ uint32_t s_start[256], s_wsum[4];
+  __shared__ int s_maxd, s_roots;
+  __shared__ unsigned s_deep, s_bad;
+  const int tid = threadIdx.x, NI = L - 1, T = 2 * L - 1;
+  if (tid == 0) {
+    s_maxd = 0;
+    s_roots = 0;
+    s_deep = 0;
+    s_bad = 0;
+  }
+  if (tid < 64) s_lev[tid] = 0;
+  for (int k = tid; k < T; k += THREADS) s_par[k] = 0;
+  for (int j = tid; j < L; j += THREADS) {
+    const int64_t s = (int64_t)j * leaf, e = min(s + leaf, n);
+    const uint64_t c = sc[s];
+    s_code[j] = c;
+    o.leaf_codes[j] = c;
+    o.node_ranges[2 * (NI + j)] = (int32_t)s;
+    o.node_ranges[2 * (NI + j) + 1] = (int32_t)(e - 1);
+  }
+  __syncthreads();
+  for (int i = tid; i < NI; i += THREADS)
+    karras_node(s_code, L, n, leaf, i, o.left_child, o.right_child, o.left_is_leaf,
+                o.right_is_leaf, o.node_ranges, s_par);
+  __syncthreads();
+  const int first = (tid / YGG_WAVE) * YGG_WAVE * kItems + (int)lane_id();
+  uint32_t level[kItems];
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    level[q] = 255u;  // slots past the last node stay behind it
+    if (k >= T) continue;
+    const int32_t p = dec_parent(s_par[k]);
+    int d = 0;
+    bool deep = false;
+    for (int32_t a = p; a >= 0; a = dec_parent(s_par[a])) {
+      ++d;
+      if (d > 255) {
+        deep = true;
+        break;
+      }
+    }
+    o.parent[k] = p;
+    o.node_level[k] = d;
+    level[q] = (uint32_t)d;
+    if (deep) s_deep = 1u;
+    if (d < 64) atomicAdd(&s_lev[d], 1u);
+    atomicMax(&s_maxd, d);
+    if (p < 0) atomicAdd(&s_roots, 1);
+    if (k < NI && (dec_parent(s_par[o.left_child[k]]) != k ||
+                   dec_parent(s_par[o.right_child[k]]) != k))
+      s_bad = 1u;
+  }
+  unsigned pos[kItems];
+  block_digit_positions<THREADS, kItems>(level, 0, 255u, s_hist, s_start, s_wsum, pos);
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    if (k < T) o.nodes_by_level[pos[q]] = k;
+  }
+  if (tid < 64) {  // the first wavefront; the barriers above order s_lev
+    const unsigned inc = wave_inclusive_sum(s_lev[tid]);
+    o.level_offsets[tid + 1] = (int32_t)inc;
+    if (tid == 0) {
+      o.level_offsets[0] = 0;
+      o.scalars[0] = s_maxd + 1 > 64 ? 64 : s_maxd + 1;
+      o.scalars[1] = s_maxd;
+      o.scalars[2] = (int32_t)s_deep;
+      o.scalars[3] = (int32_t)s_bad;
+      o.scalars[4] = s_roots;
+      o.scalars[5] = 0;
+      o.scalars[6] = 0;
+      o.scalars[7] = 0;
+    }
+  }
+}
+
+// Octree metadata of L leaves, 2 L - 1 < THREADS * kSmallItems nodes: the
+// steps of ygg_octree_meta in their order.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_octree_small(const uint64_t* __restrict__ sc,
+                                                          const int32_t* __restrict__ ranges,
+                                                          int L, YggOctreeMeta o) {
+  constexpr int kItems = kSmallItems, kCap = THREADS * kItems, kW = THREADS / YGG_WAVE;
+  constexpr int kLeaves = kCap / 2;
+  __shared__ uint64_t s_rc[kLeaves];  // resolved leaf codes and depths
+  __shared__ int32_t s_rd[kLeaves];
+  __shared__ uint64_t s_addr[kCap];   // cell addresses: sorted, then the distinct ones
+  __shared__ uint32_t s_val[kCap];
+  __shared__ uint64_t s_code[kCap];   // of the distinct cells
+  __shared__ int32_t s_dep[kCap];
+  __shared__ uint16_t s_hist[kW][256];
+  __shared__ uint32_t s_start[256], s_wsum[4], s_count[kW], s_lev[64];
+  __shared__ int s_maxd;
+  const int tid = threadIdx.x, w = tid / YGG_WAVE;
+  const unsigned lane = lane_id();
+  const int NI = L - 1, M = 2 * L - 1;
+  const int first = w * YGG_WAVE * kItems + (int)lane;
+  if (tid < 64) s_lev[tid] = 0;
+  if (tid == 0) s_maxd = 0;
+  __syncthreads();
+  for (int j = tid; j < L; j += THREADS) {
+    const uint64_t f = sc[ranges[2 * (NI + j)]], l = sc[ranges[2 * (NI + j) + 1]];
+    const int d = common_depth(f, l);
+    s_rd[j] = d;
+    s_rc[j] = prefix_code(f, d);
+  }
+  for (int i = tid; i < 8 * M; i += THREADS) o.oct_children[i] = -1;
+  __syncthreads();
+  // candidate cells by address (at depth d below 2^(3 d + 1))
+  uint64_t key[kItems];
+  uint32_t val[kItems];
+  unsigned pos[kItems];
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    key[q] = ~0ull;  // slots past the last stay behind it
+    val[q] = (uint32_t)k;
+    if (k < M) {
+      uint64_t c;
+      int d;
+      candidate(s_rc, s_rd, L, k, &c, &d);
+      key[q] = oct_address(c, d);
+      atomicMax(&s_maxd, d);
+    }
+  }
+  __syncthreads();
+  const int bits = min(3 * s_maxd + 1, 64);
+  for (int shift = 0; shift < bits; shift += 8) {
+    block_digit_positions<THREADS, kItems>(key, shift, 255u, s_hist, s_start, s_wsum, pos);
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+      s_addr[pos[q]] = key[q];
+      s_val[pos[q]] = val[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+      key[q] = s_addr[first + q * YGG_WAVE];
+      val[q] = s_val[first + q * YGG_WAVE];
+    }
+  }
+  // the distinct ones, the first candidate of each
+  bool lead[kItems];
+  unsigned before[kItems], mine = 0;
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    lead[q] = k < M && (k == 0 || s_addr[k - 1] != key[q]);
+    const uint64_t b = __ballot(lead[q]);
+    before[q] = mine + mbcnt64(b);
+    mine += (unsigned)__popcll(b);
+  }
+  if (lane == 0) s_count[w] = mine;
+  __syncthreads();
+  int cells = 0, base = 0;
+#pragma unroll
+  for (int q = 0; q < kW; ++q) {
+    if (q < w) base += (int)s_count[q];
+    cells += (int)s_count[q];
+  }
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    if (lead[q]) {
+      const int u = base + (int)before[q];
+      uint64_t c;
+      int d;
+      candidate(s_rc, s_rd, L, (int)val[q], &c, &d);
+      s_addr[u] = key[q];
+      s_code[u] = c;
+      s_dep[u] = d;
+    }
+    if (k >= cells && k < M) {
+      s_addr[k] = ~0ull;
+      s_code[k] = 0;
+      s_dep[k] = -1;
+    }
+  }
+  __syncthreads();
+  uint32_t lkey[kItems];
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    lkey[q] = 255u;
+    if (k >= M) continue;
+    const bool v = k < cells;
+    const uint64_t c = s_code[k];
+    const int d = s_dep[k];
+    o.oct_node_codes[k] = c;
+    o.oct_node_depths[k] = d;
+    o.oct_valid_mask[k] = v;
+    int32_t r0 = 0, r1 = -1;
+    if (v) {
+      const uint64_t bs = 63ull - 3ull * (uint64_t)max(d, 0);
+      const uint64_t endc = c | ((1ull << (bs < 62ull ? bs : 62ull)) - 1ull);
+      const int f = min(max(fixed_round_search(s_rc, L, c, true), 0), L - 1);
+      const int l = min(max(fixed_round_search(s_rc, L, endc, false) - 1, 0), L - 1);
+      r0 = ranges[2 * (NI + f)];
+      r1 = ranges[2 * (NI + l) + 1];
+      atomicAdd(&s_lev[min(max(d, 0), 21)], 1u);
+    }
+    o.oct_node_ranges[2 * k] = r0;
+    o.oct_node_ranges[2 * k + 1] = r1;
+    lkey[q] = v ? (uint32_t)d : 22u;
+  }
+  block_digit_positions<THREADS, kItems>(lkey, 0, 255u, s_hist, s_start, s_wsum, pos);
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    if (k < M) o.oct_nodes_by_level[pos[q]] = k;
+  }
+  if (w == 0) {
+    const unsigned inc = wave_inclusive_sum(lane < 22 ? s_lev[lane] : 0u);
+    if (lane < 22) o.oct_level_offsets[lane + 1] = (int32_t)inc;
+    if (lane == 0) {
+      o.oct_level_offsets[0] = 0;
+      o.scalars[0] = s_maxd + 1;
+      o.scalars[1] = cells;
+      o.scalars[3] = s_maxd;
+    }
+  }
+  // parents: the nearest ancestor cell that is there
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    if (k >= M) continue;
+    int32_t par = -1;
+    if (k < cells) {
+      const int d = s_dep[k];
+      const uint64_t c = s_code[k];
+      for (int up = 1; up <= 21 && up <= d; ++up) {
+        const uint64_t pa = oct_address(prefix_code(c, d - up), d - up);
+        const int at = fixed_round_search(s_addr, M, pa, true);
+        if (s_addr[min(at, M - 1)] == pa) {
+          par = at;
+          break;
+        }
+      }
+      if (par >= 0) atomicMax(&o.oct_children[(int64_t)par * 8 + octant_at_depth(c, d)], k);
+    }
+    o.oct_parent[k] = par;
+  }
+  __syncthreads();
+  mine = 0;
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    int cnt = 0;
+    if (k < M) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const int32_t child = __hip_atomic_load(&o.oct_children[(int64_t)k * 8 + c],
+                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool m = k < cells && child >= 0;
+        o.oct_child_mask[(int64_t)k * 8 + c] = m;
+        cnt += m;
+      }
+      o.oct_child_counts[k] = cnt;
+    }
+    lead[q] = k < cells && cnt == 0;
+    if (k < M) o.oct_leaf_mask[k] = lead[q];
+    const uint64_t b = __ballot(lead[q]);
+    before[q] = mine + mbcnt64(b);
+    mine += (unsigned)__popcll(b);
+  }
+  if (lane == 0) s_count[w] = mine;
+  __syncthreads();
+  int leaves = 0;
+  base = 0;
+#pragma unroll
+  for (int q = 0; q < kW; ++q) {
+    if (q < w) base += (int)s_count[q];
+    leaves += (int)s_count[q];
+  }
+  if (tid == 0) o.scalars[2] = leaves;
+#pragma unroll
+  for (int q = 0; q < kItems; ++q) {
+    const int k = first + q * YGG_WAVE;
+    if (lead[q]) o.oct_leaf_nodes[base + (int)before[q]] = k;
+    if (k >= leaves && k < M) o.oct_leaf_nodes[k] = -1;
+    if (k >= M) continue;
+    // radix node k's cell
+    int d;
+    uint64_t c;
+    if (k >= NI) {
+      d = s_rd[k - NI];
+      c = s_rc[k - NI];
+    } else {
+      const uint64_t f = sc[ranges[2 * k]], l = sc[ranges[2 * k + 1]];
+      d = common_depth(f, l);
+      c = prefix_code(f, d);
+      o.leaf_position[k] = -1;
+    }
+    const int at = fixed_round_search(s_addr, M, oct_address(c, d), true);
+    o.radix_node_to_oct[k] = at;
+    if (k >= NI) s_val[k - NI] = (uint32_t)at;
+  }
+  __syncthreads();
+  // leaves by cell
+  constexpr int kHalf = kItems / 2;
+  const int hfirst = w * YGG_WAVE * kHalf + (int)lane;
+  uint32_t hk[kHalf], hv[kHalf];
+  unsigned hp[kHalf];
+#pragma unroll
+  for (int q = 0; q < kHalf; ++q) {
+    const int i = hfirst + q * YGG_WAVE;
+    hk[q] = i < L ? s_val[i] : ~0u;
+    hv[q] = (uint32_t)i;
+  }
+  for (int shift = 0; shift < 16; shift += 8) {  // addresses' places are below 2^12
+    block_digit_positions<THREADS, kHalf>(hk, shift, 255u, s_hist, s_start, s_wsum, hp);
+#pragma unroll
+    for (int q = 0; q < kHalf; ++q) {
+      s_val[hp[q]] = hk[q];
+      s_val[kLeaves + hp[q]] = hv[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kHalf; ++q) {
+      hk[q] = s_val[hfirst + q * YGG_WAVE];
+      hv[q] = s_val[kLeaves + hfirst + q * YGG_WAVE];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kHalf; ++q) {
+    const int i = hfirst + q * YGG_WAVE;
+    if (i >= L) continue;
+    const int32_t node = NI + (int32_t)hv[q];
+    o.leaf_indices[i] = node;
+    o.leaf_position[node] = i;
+  }
 }
 
 }  // namespace ygg
@@ -869,12 +1223,9 @@ int ygg_radix_build(const uint64_t* sorted_codes, int64_t n, int64_t leaf_size,
   const int L = (int)L64;
   const int T = 2 * L - 1;
   const int NI = L - 1;
-  int rc = fill_u32((uint32_t*)o->scalars, 0u, 8, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_leaves, dim3(grid_for(L, 256)), dim3(256), 0, st, sorted_codes, n,
-                     leaf_size, L, o->leaf_codes, o->node_ranges);
-  YGG_LAUNCH_CHECK();
   if (L == 1) {
+    hipLaunchKernelGGL(k_leaves, dim3(1), dim3(256), 0, st, sorted_codes, n, leaf_size, L,
+                       o->leaf_codes, o->node_ranges, o->scalars);
     hipLaunchKernelGGL(k_single_leaf, dim3(1), dim3(64), 0, st, n, o->parent, o->node_ranges,
                        o->node_level, o->level_offsets, o->nodes_by_level, o->scalars);
     YGG_LAUNCH_CHECK();
@@ -887,8 +1238,21 @@ int ygg_radix_build(const uint64_t* sorted_codes, int64_t n, int64_t leaf_size,
   size_t sbytes = ygg::sort_workspace_bytes(T, 4, 32);
   char* sws = a.take<char>(sbytes);
   if (!penc || !lcount || !skeys || !sws) return YGG_ERR_WORKSPACE;
-  if ((rc = fill_u32(penc, 0u, T, st))) return rc;
-  if ((rc = fill_u32(lcount, 0u, 64, st))) return rc;
+  if (T < kSmallNodes) {
+    if (T < 256 * kSmallItems)
+      hipLaunchKernelGGL(k_radix_small<256>, dim3(1), dim3(256), 0, st, sorted_codes, n, leaf_size,
+                         L, *o);
+    else
+      hipLaunchKernelGGL(k_radix_small<1024>, dim3(1), dim3(1024), 0, st, sorted_codes, n,
+                         leaf_size, L, *o);
+    YGG_LAUNCH_CHECK();
+    return YGG_OK;
+  }
+  hipLaunchKernelGGL(k_leaves, dim3(grid_for(L, 256)), dim3(256), 0, st, sorted_codes, n,
+                     leaf_size, L, o->leaf_codes, o->node_ranges, o->scalars);
+  YGG_LAUNCH_CHECK();
+  // the parent links and the level counts lie side by side
+  if (int rc = fill_u32(penc, 0u, (lcount + 64) - penc, st)) return rc;
   hipLaunchKernelGGL(k_karras, dim3(grid_for(NI, 256)), dim3(256), 0, st, o->leaf_codes, L, n,
                      leaf_size, o->left_child, o->right_child, o->left_is_leaf, o->right_is_leaf,
                      o->node_ranges, penc);
@@ -1000,11 +1364,19 @@ int ygg_octree_meta(const uint64_t* sc, const int32_t* node_ranges, int64_t L64,
       !cplus || !lcount || !lkey || !native || !sws || !scws)
     return YGG_ERR_WORKSPACE;
   int rcode;
-  if ((rcode = fill_u32((uint32_t*)o->scalars, 0u, 4, st))) return rcode;
-  if ((rcode = fill_u32(lcount, 0u, 32, st))) return rcode;
-  if ((rcode = fill_u32(cplus, 0u, (int64_t)M * 8, st))) return rcode;
+  if (M < kSmallNodes) {
+    if (M < 256 * kSmallItems)
+      hipLaunchKernelGGL(k_octree_small<256>, dim3(1), dim3(256), 0, st, sc, node_ranges, L, *o);
+    else
+      hipLaunchKernelGGL(k_octree_small<1024>, dim3(1), dim3(1024), 0, st, sc, node_ranges, L, *o);
+    YGG_LAUNCH_CHECK();
+    return YGG_OK;
+  }
+  // the child slots and the level counts lie side by side
+  if ((rcode = fill_u32(cplus, 0u, (lcount + 32) - cplus, st))) return rcode;
   const int gL = grid_for(L, 256), gM = grid_for(M, 256), gT = grid_for(T, 256);
-  hipLaunchKernelGGL(k_oct_resolve, dim3(gL), dim3(256), 0, st, sc, node_ranges, L, rc, rd);
+  hipLaunchKernelGGL(k_oct_resolve, dim3(gL), dim3(256), 0, st, sc, node_ranges, L, rc, rd,
+                     o->scalars);
   hipLaunchKernelGGL(k_oct_candidates, dim3(gM), dim3(256), 0, st, rc, rd, L, M, caddr);
   YGG_LAUNCH_CHECK();
   if ((rcode = sort_pairs_u64(caddr, nullptr, saddr, order, M, 0, 64, sws, sb, st))) return rcode;
@@ -1037,9 +1409,7 @@ int ygg_octree_meta(const uint64_t* sc, const int32_t* node_ranges, int64_t L64,
   int end_bit = 32 - __builtin_clz((unsigned)M);  // values in [0, M]
   if ((rcode = sort_pairs_u32(lkey, nullptr, stmp, native, L, 0, end_bit, sws, sb, st)))
     return rcode;
-  hipLaunchKernelGGL(k_leaf_order, dim3(gT), dim3(256), 0, st, native, NI, L, T, o->leaf_indices,
-                     o->leaf_position);
-  hipLaunchKernelGGL(k_leaf_order2, dim3(gL), dim3(256), 0, st, native, NI, L, o->leaf_indices,
+  hipLaunchKernelGGL(k_leaf_order, dim3(gL), dim3(256), 0, st, native, NI, L, o->leaf_indices,
                      o->leaf_position);
   YGG_LAUNCH_CHECK();
   return YGG_OK;
@@ -1050,10 +1420,8 @@ int ygg_radix_leaf_order(int64_t num_leaves, int32_t* leaf_indices, int32_t* lea
                          void* stream) {
   if (num_leaves < 1) return YGG_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
-  int L = (int)num_leaves, T = 2 * L - 1, NI = L - 1;
-  hipLaunchKernelGGL(k_leaf_order, dim3(grid_for(T, 256)), dim3(256), 0, st, nullptr, NI, L, T,
-                     leaf_indices, leaf_position);
-  hipLaunchKernelGGL(k_leaf_order2, dim3(grid_for(L, 256)), dim3(256), 0, st, nullptr, NI, L,
+  int L = (int)num_leaves, NI = L - 1;
+  hipLaunchKernelGGL(k_leaf_order, dim3(grid_for(L, 256)), dim3(256), 0, st, nullptr, NI, L,
                      leaf_indices, leaf_position);
   YGG_LAUNCH_CHECK();
   return YGG_OK;

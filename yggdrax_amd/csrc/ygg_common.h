@@ -159,6 +159,55 @@ __device__ __forceinline__ unsigned wave_inclusive_sum(unsigned v) {
   return v;
 }
 
+// Positions of a workgroup's THREADS * ITEMS keys after a stable sort by the
+// digit (key >> shift) & mask of at most 8 bits. Wavefront w holds the keys
+// [w * 64 * ITEMS, ...) of the current order, key k of a lane 64 after key
+// k - 1: it ranks them with ballot matches and digit counters of its own. The
+// caller puts a barrier between a call and the next (s_hist is read last).
+template <int THREADS, int ITEMS, typename K>
+__device__ __forceinline__ void block_digit_positions(
+    const K (&key)[ITEMS], int shift, unsigned mask, uint16_t (*s_hist)[256], uint32_t* s_start,
+    uint32_t* s_wsum, unsigned (&pos)[ITEMS]) {
+  constexpr int kBins = 256, kW = THREADS / YGG_WAVE;
+  static_assert(THREADS >= kBins, "one thread per digit");
+  const int tid = threadIdx.x, w = tid / YGG_WAVE;
+  const unsigned lane = lane_id();
+  for (int i = tid; i < kW * kBins; i += THREADS) (&s_hist[0][0])[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const unsigned d = (unsigned)(key[k] >> shift) & mask;
+    const uint64_t peers = wave_match_bits<8>(d, ~0ull);
+    const unsigned below = mbcnt64(peers);
+    const unsigned before = s_hist[w][d];
+    pos[k] = before + below;
+    if (below == 0) s_hist[w][d] = (uint16_t)(before + (unsigned)__popcll(peers));
+  }
+  __syncthreads();
+  unsigned total = 0, inc = 0;
+  if (tid < kBins) {
+    for (int q = 0; q < kW; ++q) {
+      const unsigned c = s_hist[q][tid];
+      s_hist[q][tid] = (uint16_t)total;  // exclusive prefix over waves
+      total += c;
+    }
+    inc = wave_inclusive_sum(total);
+    if (lane == 63) s_wsum[w] = inc;
+  }
+  __syncthreads();
+  if (tid < kBins) {
+    unsigned run = inc - total;
+    for (int q = 0; q < w; ++q) run += s_wsum[q];
+    s_start[tid] = run;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const unsigned d = (unsigned)(key[k] >> shift) & mask;
+    pos[k] += s_start[d] + s_hist[w][d];
+  }
+}
+
 __device__ __forceinline__ float wave_sum_f(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

@@ -395,7 +395,6 @@ __global__ __launch_bounds__(THREADS) void k_small_sort(const K* __restrict__ ke
                                                         uint32_t* __restrict__ vals_out, int n,
                                                         int begin_bit, int end_bit) {
   constexpr int kBins = 256, kW = THREADS / YGG_WAVE, kCap = THREADS * ITEMS;
-  static_assert(THREADS >= kBins, "one thread per digit");
   __shared__ K s_key[kCap];
   __shared__ uint32_t s_val[kCap];
   __shared__ uint16_t s_hist[kW][kBins];
@@ -405,7 +404,8 @@ __global__ __launch_bounds__(THREADS) void k_small_sort(const K* __restrict__ ke
   const unsigned lane = lane_id();
   const int first = w * YGG_WAVE * ITEMS + (int)lane;
   K key[ITEMS];
-  uint32_t val[ITEMS], rank[ITEMS];
+  uint32_t val[ITEMS];
+  unsigned pos[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const int i = first + k * YGG_WAVE;
@@ -414,41 +414,11 @@ __global__ __launch_bounds__(THREADS) void k_small_sort(const K* __restrict__ ke
   }
   for (int shift = begin_bit; shift < end_bit; shift += 8) {
     const unsigned mask = end_bit - shift < 8 ? (1u << (end_bit - shift)) - 1u : 255u;
-    for (int i = tid; i < kW * kBins; i += THREADS) (&s_hist[0][0])[i] = 0;
-    __syncthreads();
+    block_digit_positions<THREADS, ITEMS>(key, shift, mask, s_hist, s_start, s_wsum, pos);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-      const unsigned d = (unsigned)(key[k] >> shift) & mask;
-      const uint64_t peers = wave_match_bits<8>(d, ~0ull);
-      const unsigned below = mbcnt64(peers);
-      const unsigned before = s_hist[w][d];
-      rank[k] = before + below;
-      if (below == 0) s_hist[w][d] = (uint16_t)(before + (unsigned)__popcll(peers));
-    }
-    __syncthreads();
-    unsigned total = 0, inc = 0;
-    if (tid < kBins) {
-      for (int q = 0; q < kW; ++q) {
-        const unsigned c = s_hist[q][tid];
-        s_hist[q][tid] = (uint16_t)total;  // exclusive prefix over waves
-        total += c;
-      }
-      inc = wave_inclusive_sum(total);
-      if (lane == 63) s_wsum[w] = inc;
-    }
-    __syncthreads();
-    if (tid < kBins) {
-      unsigned run = inc - total;
-      for (int q = 0; q < w; ++q) run += s_wsum[q];
-      s_start[tid] = run;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const unsigned d = (unsigned)(key[k] >> shift) & mask;
-      const unsigned pos = s_start[d] + s_hist[w][d] + rank[k];
-      s_key[pos] = key[k];
-      s_val[pos] = val[k];
+      s_key[pos[k]] = key[k];
+      s_val[pos[k]] = val[k];
     }
     __syncthreads();
     if (shift + 8 < end_bit) {
@@ -838,6 +808,45 @@ __global__ __launch_bounds__(256) void k_scan_apply(const int32_t* __restrict__ 
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = partial[gridDim.x];
 }
 
+// The whole scan of at most kSmallScan counts in one workgroup: 4096 of them
+// per step. Three launches cost the host 12 us, more than this one takes.
+constexpr int kSmallScanThreads = 1024;
+constexpr int64_t kSmallScan = 16384;
+
+__global__ __launch_bounds__(kSmallScanThreads) void k_scan_small(
+    const int32_t* __restrict__ c, const int32_t* __restrict__ gather, int n,
+    int64_t* __restrict__ out) {
+  __shared__ int64_t s_sum[2][kSmallScanThreads / YGG_WAVE];
+  const int w = threadIdx.x / YGG_WAVE;
+  int64_t carry = 0;
+  int buf = 0;
+  for (int base = 0; base < n; base += 4 * kSmallScanThreads, buf = 1 - buf) {
+    const int i = base + 4 * (int)threadIdx.x;
+    int64_t v[4], s = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = i + k < n ? (int64_t)c[gather ? gather[i + k] : i + k] : 0;
+      s += v[k];
+    }
+    const int64_t inc = wave_inclusive_sum64(s);
+    if (lane_id() == YGG_WAVE - 1) s_sum[buf][w] = inc;
+    __syncthreads();  // the next step writes the other buffer
+    int64_t run = carry + inc - s;
+#pragma unroll
+    for (int q = 0; q < kSmallScanThreads / YGG_WAVE; ++q) {
+      const int64_t t = s_sum[buf][q];
+      if (q < w) run += t;
+      carry += t;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (i + k < n) out[i + k] = run;
+      run += v[k];
+    }
+  }
+  if (threadIdx.x == 0) out[n] = carry;
+}
+
 size_t scan_workspace_bytes(int64_t n) {
   return align_up(sizeof(int64_t) * (size_t)((n + kScanTile - 1) / kScanTile + 2));
 }
@@ -847,6 +856,12 @@ int exclusive_scan_i32_to_i64(const int32_t* counts, const int32_t* gather, int6
   if (n <= 0) return fill_u32((uint32_t*)out, 0u, 2, st);
   int64_t nb = (n + kScanTile - 1) / kScanTile;
   if (ws_bytes < scan_workspace_bytes(n)) return YGG_ERR_WORKSPACE;
+  if (n <= kSmallScan) {
+    hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallScanThreads), 0, st, counts, gather,
+                       (int)n, out);
+    YGG_LAUNCH_CHECK();
+    return YGG_OK;
+  }
   int64_t* partial = (int64_t*)ws;
   hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(kScanThreads), 0, st, counts, gather,
                      n, partial);
