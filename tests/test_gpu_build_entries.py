@@ -98,3 +98,29 @@ def test_sort_reorder_async_matches_one_stream(n):
 
 def test_widen_item_layout():
     assert ctypes.sizeof(_lib.WidenItem) == 24
+
+
+@pytest.mark.parametrize("n", [1, 1023, 12288, 12289, 16384, 16385, (1 << 17) - 1, 1 << 17])
+def test_sort_and_bounds_at_path_edges(n):
+    """Bounds of aligned and unaligned positions by one workgroup and by many,
+    codes with and without digit histograms, the inverse with the gather and
+    apart: against numpy."""
+    import yggdrax_amd as ygg
+    print(f"[build entries] edges n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    host = rng.normal(size=(n + 1, 3)).astype(np.float32)
+    mass = torch.from_numpy(rng.random(n, dtype=np.float32)).cuda()
+    both = torch.from_numpy(host).cuda()
+    for pos, h in ((both[:n].clone(), host[:n]), (both[1:], host[1:])):
+        lo, hi = ygg.infer_bounds(pos)
+        span = h.max(0) - h.min(0)
+        pad = np.maximum(span * np.float32(0.05), np.float32(1e-6))
+        assert np.array_equal(lo.cpu().numpy(), h.min(0) - pad)
+        assert np.array_equal(hi.cpu().numpy(), h.max(0) + pad)
+        tree, ps, ms, inv = ygg.build_tree(pos, mass, return_reordered=True, leaf_size=8)
+        codes = ygg.morton_encode(pos, (lo, hi)).view(torch.int64).cpu().numpy()
+        perm = np.argsort(codes, kind="stable")  # 63-bit codes: no sign
+        assert np.array_equal(tree.particle_indices.cpu().numpy(), perm)
+        assert np.array_equal(ps.cpu().numpy(), h[perm])
+        assert np.array_equal(ms.cpu().numpy(), mass.cpu().numpy()[perm])
+        assert np.array_equal(inv.cpu().numpy(), np.argsort(perm))

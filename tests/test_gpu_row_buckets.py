@@ -428,3 +428,52 @@ def test_pair_records_need_the_bucketing(lib):
         scr.data_ptr(), roff.data_ptr(), out.data_ptr(), cnt.data_ptr(), off.data_ptr(),
         ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
     assert rc != 0
+
+
+# one workgroup up to 8192 slots and 4096 keys; beyond, the bucketing kernels
+EDGES = [(1, 0, "uniform"), (1, 1, "uniform"), (63, 1900, "spill"), (4096, 8192, "uniform"),
+         (4097, 8192, "uniform"), (4096, 8193, "skewed")]
+
+
+@pytest.mark.parametrize("rows,n,kind", EDGES)
+def test_near_at_the_workgroup_edge(lib, rows, n, kind):
+    test_near_buckets_match_numpy(lib, rows, n, kind)
+
+
+@pytest.mark.parametrize("T,n", [(3, 0), (63, 950), (4095, 8192), (4097, 8192), (4095, 8193)])
+def test_records_at_the_workgroup_edge(lib, T, n):
+    """Pair records: node a's row gets b and node b's row gets a, the rows of
+    the near lists in leaf order, the far ones in level order."""
+    print(f"[row buckets] records T={T} n={n}", flush=True)
+    rng = np.random.default_rng(T + n)
+    dev = torch.device("cuda")
+    NI = T // 2
+    for far in (False, True):
+        lo = 0 if far else NI
+        a, b = (rng.integers(lo, T, n).astype(np.int32) for _ in range(2))
+        kt, vt = torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev)
+        order = (lo + rng.permutation(T - lo)).astype(np.int32)
+        row_of = np.full(T, -1)
+        row_of[order] = np.arange(T - lo)
+        counts, vals = _expected(np.concatenate([row_of[a], row_of[b]]),
+                                 np.concatenate([b, a]), T - lo)
+        ot = torch.from_numpy(order).to(dev)
+        if far:
+            lvl = torch.from_numpy(rng.integers(0, 30, T).astype(np.int32)).to(dev)
+            got = _far(lib, kt, vt, n, None, T, ot, lvl, 0, records=True)
+            rows = np.repeat(np.arange(T), counts)
+            assert np.array_equal(got["targets"].cpu().numpy()[:2 * n], order[rows])
+            assert np.array_equal(got["levels"].cpu().numpy()[:2 * n],
+                                  lvl.cpu().numpy()[order[rows]])
+            assert np.array_equal(got["counts"].cpu().numpy()[order], counts)
+            assert np.array_equal(got["counts32"].cpu().numpy()[order], counts)
+            off, out = got["lm"], got["sources"]
+            assert torch.equal(got["node_off"][:T][ot.long()], off[:T])
+            assert int(got["node_off"][T]) == 2 * n
+        else:
+            got = _near(lib, kt, vt, n, None, T - lo, 0, leaf_nodes=ot,
+                        nend=max(1, (T - 1).bit_length()))
+            assert np.array_equal(got["counts"].cpu().numpy(), counts)
+            off, out = got["rows"], got["neighbors"]
+        assert np.array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+        assert np.array_equal(_row_sorted(out.cpu().numpy()[:2 * n], counts), vals)

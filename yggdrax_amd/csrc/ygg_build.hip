@@ -104,6 +104,45 @@ __global__ __launch_bounds__(256) void k_bounds_reduce4(const float* __restrict_
   }
 }
 
+// Bounds of at most kSmallBounds points by one workgroup, which writes them
+// itself: three launches cost the host 12 us.
+constexpr int64_t kSmallBounds = 16384;
+
+__global__ __launch_bounds__(1024) void k_bounds_small(const float* __restrict__ pos, int n,
+                                                       float* __restrict__ b6) {
+  __shared__ uint32_t s[1024 / YGG_WAVE][6];
+  uint32_t mn[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, mx[3] = {0u, 0u, 0u};
+#pragma unroll 4
+  for (int i = (int)threadIdx.x; i < n; i += 1024)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint32_t o = f2ord(pos[3 * i + k]);
+      mn[k] = min(mn[k], o);
+      mx[k] = max(mx[k], o);
+    }
+  const int w = threadIdx.x / YGG_WAVE;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    mn[k] = wave_min_u32(mn[k]);
+    mx[k] = wave_max_u32(mx[k]);
+  }
+  if (lane_id() == 0)
+    for (int k = 0; k < 3; ++k) {
+      s[w][k] = mn[k];
+      s[w][3 + k] = mx[k];
+    }
+  __syncthreads();
+  const int d = threadIdx.x;
+  if (d < 3) {
+    uint32_t a = s[0][d], b = s[0][3 + d];
+    for (int q = 1; q < 1024 / YGG_WAVE; ++q) {
+      a = min(a, s[q][d]);
+      b = max(b, s[q][3 + d]);
+    }
+    padded_bounds(ord2f(a), ord2f(b), &b6[d], &b6[3 + d]);
+  }
+}
+
 __global__ void k_bounds_init(uint32_t* acc) {
   if (threadIdx.x < 3) {
     acc[threadIdx.x] = 0xFFFFFFFFu;
@@ -176,16 +215,20 @@ __global__ __launch_bounds__(256) void k_reorder(const float* __restrict__ pos,
 
 // Encode + digit histograms (as k_encode_hist) that also packs (x, y, z, m)
 // into one float4 per particle, so the later reorder gathers one 16-byte
-// record (one cache line) per particle instead of two.
+// record (one cache line) per particle instead of two. Without HIST for a sort
+// that counts its own digits (at most kSmallSort codes).
+template <bool HIST>
 __global__ __launch_bounds__(kEncodeThreads) void k_encode_hist_pack(const float* __restrict__ pos,
                                                           const float* __restrict__ mass,
                                                           int64_t n, const float* __restrict__ b6,
                                                           uint64_t* __restrict__ codes,
                                                           uint32_t* __restrict__ hist,
                                                           float4* __restrict__ packed) {
-  __shared__ uint32_t h[kMortonHistWords];
-  for (int i = threadIdx.x; i < kMortonHistWords; i += blockDim.x) h[i] = 0;
-  __syncthreads();
+  __shared__ uint32_t h[HIST ? kMortonHistWords : 1];
+  if constexpr (HIST) {
+    for (int i = threadIdx.x; i < kMortonHistWords; i += blockDim.x) h[i] = 0;
+    __syncthreads();
+  }
   float lo[3] = {b6[0], b6[1], b6[2]};
   float w[3] = {b6[3] - b6[0], b6[4] - b6[1], b6[5] - b6[2]};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -199,22 +242,31 @@ __global__ __launch_bounds__(kEncodeThreads) void k_encode_hist_pack(const float
       codes[i] = c;
       packed[i] = make_float4(x, y, z, mass ? mass[i] : 0.0f);
     }
+    if constexpr (HIST) {
 #pragma unroll
-    for (int p = 0; p < kMortonPasses; ++p) morton_hist_add(h, c, valid, p);
+      for (int p = 0; p < kMortonPasses; ++p) morton_hist_add(h, c, valid, p);
+    }
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kMortonHistWords; i += blockDim.x)
-    if (h[i]) atomicAdd(&hist[i], h[i]);
+  if constexpr (HIST) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < kMortonHistWords; i += blockDim.x)
+      if (h[i]) atomicAdd(&hist[i], h[i]);
+  }
 }
 
-// Sorted positions and masses: one 16-byte gather per particle. The
-// inverse permutation is written by its own kernel (k_inverse_perm): the
-// gather and the scattered inverse writes together took 682 us at 2^24
-// clustered points on gfx950, apart 360 + 200 us.
+// Sorted positions and masses: one 16-byte gather per particle. From
+// kFusedInverse particles on the inverse permutation is written by its own
+// kernel (k_inverse_perm): the gather and the scattered inverse writes together
+// took 682 us at 2^24 clustered points on gfx950, apart 360 + 200 us. Below,
+// both stay in the caches and the launch is what counts.
+constexpr int64_t kFusedInverse = 1 << 17;
+
+template <typename InvT>
 __global__ __launch_bounds__(256) void k_reorder_packed(const float4* __restrict__ packed,
                                                         const uint32_t* __restrict__ perm,
                                                         int64_t n, float* __restrict__ pos_sorted,
-                                                        float* __restrict__ mass_sorted) {
+                                                        float* __restrict__ mass_sorted,
+                                                        InvT* __restrict__ inv) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const uint32_t p = perm[i];
@@ -223,6 +275,7 @@ __global__ __launch_bounds__(256) void k_reorder_packed(const float4* __restrict
     pos_sorted[3 * i + 1] = r.y;
     pos_sorted[3 * i + 2] = r.z;
     if (mass_sorted) mass_sorted[i] = r.w;
+    if (inv) inv[p] = (InvT)i;
   }
 }
 
@@ -994,6 +1047,11 @@ int ygg_infer_bounds(const float* pos, int64_t n, float* bounds6, void* ws, size
   if (n < 1 || !pos || !bounds6) return YGG_ERR_ARG;
   if (ws_bytes < 24) return YGG_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
+  if (n <= kSmallBounds) {
+    hipLaunchKernelGGL(k_bounds_small, dim3(1), dim3(1024), 0, st, pos, (int)n, bounds6);
+    YGG_LAUNCH_CHECK();
+    return YGG_OK;
+  }
   uint32_t* acc = (uint32_t*)ws;
   hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, st, acc);
   if (((uintptr_t)pos & 15) == 0) {
@@ -1096,10 +1154,15 @@ static int morton_sort_pack(const float* pos, const float* mass, int64_t n, cons
   size_t rest = ygg::sort_workspace_bytes(n, 8, kMortonEndBit, kMortonDigitBits);
   char* sws = a.take<char>(rest);
   if (!packed || !codes || !hist || !sws) return YGG_ERR_WORKSPACE;
-  int rc = fill_u32(hist, 0u, kMortonHistWords, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_encode_hist_pack, dim3(grid_for(n, kEncodeThreads, kEncodeBlocks)),
-                     dim3(kEncodeThreads), 0, st, pos, mass, n, bounds6, codes, hist, packed);
+  int rc = YGG_OK;
+  if (n <= ygg::kSmallSort) {
+    hipLaunchKernelGGL(k_encode_hist_pack<false>, dim3(grid_for(n, 256)), dim3(256), 0, st, pos,
+                       mass, n, bounds6, codes, nullptr, packed);
+  } else {
+    if ((rc = fill_u32(hist, 0u, kMortonHistWords, st))) return rc;
+    hipLaunchKernelGGL(k_encode_hist_pack<true>, dim3(grid_for(n, kEncodeThreads, kEncodeBlocks)),
+                       dim3(kEncodeThreads), 0, st, pos, mass, n, bounds6, codes, hist, packed);
+  }
   YGG_LAUNCH_CHECK();
   if ((rc = sort_pairs_u64(codes, nullptr, sorted_codes, perm, n, 0, kMortonEndBit, sws, rest, st, hist,
                         kMortonDigitBits)))
@@ -1111,8 +1174,15 @@ static int morton_sort_pack(const float* pos, const float* mass, int64_t n, cons
 static int reorder_from_packed(const float4* packed, const uint32_t* perm, int64_t n,
                                float* pos_sorted, float* mass_sorted, void* inverse,
                                int inverse_i64, hipStream_t st) {
-  hipLaunchKernelGGL(k_reorder_packed, dim3(grid_for(n, 256, 8192)), dim3(256), 0, st, packed,
-                     perm, n, pos_sorted, mass_sorted);
+  const dim3 g(grid_for(n, 256, 8192));
+  const bool fused = n < kFusedInverse;
+  if (inverse_i64)
+    hipLaunchKernelGGL(k_reorder_packed<int64_t>, g, dim3(256), 0, st, packed, perm, n, pos_sorted,
+                       mass_sorted, fused ? (int64_t*)inverse : nullptr);
+  else
+    hipLaunchKernelGGL(k_reorder_packed<int32_t>, g, dim3(256), 0, st, packed, perm, n, pos_sorted,
+                       mass_sorted, fused ? (int32_t*)inverse : nullptr);
+  if (fused) inverse = nullptr;
   if (inverse && inverse_i64)
     hipLaunchKernelGGL(k_inverse_perm<int64_t>, dim3(grid_for(n, 256)), dim3(256), 0, st, perm, n,
                        (int64_t*)inverse);

@@ -344,6 +344,9 @@ int sort_pairs_u32(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* k
                    uint32_t* vals_out, int64_t n, int begin_bit, int end_bit, void* ws,
                    size_t ws_bytes, hipStream_t st, int digit_bits = 0);
 
+// Largest sort that one workgroup takes (k_small_sort): 12288 64-bit keys and
+// their values fill 152 KB of LDS. It reads no digit histograms.
+constexpr int64_t kSmallSort = 12288;
 size_t scan_workspace_bytes(int64_t n);
 // Row-key sorts whose last pass writes the far sources / near neighbours
 // and adds the per-row entry counts into row_counts[rows] (zero before the

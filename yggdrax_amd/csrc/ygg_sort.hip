@@ -435,10 +435,6 @@ __global__ __launch_bounds__(THREADS) void k_small_sort(const K* __restrict__ ke
   }
 }
 
-// Largest sort that one workgroup takes (k_small_sort): 12288 64-bit keys and
-// their values fill 152 KB of LDS.
-constexpr int64_t kSmallSort = 12288;
-
 template <typename K>
 static int small_sort(const K* keys_in, const uint32_t* vals_in, K* keys_out, uint32_t* vals_out,
                       int64_t n, int begin_bit, int end_bit, hipStream_t st) {

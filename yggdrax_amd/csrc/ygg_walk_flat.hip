@@ -926,15 +926,23 @@ __global__ __launch_bounds__(256) void k_near_dense(int L, const int64_t* __rest
 
 // Far targets and target levels row by row: one wavefront fills row r's
 // range [off[r], off[r + 1]) with its node and that node's level
-// (coalesced stores; no per-entry key read).
+// (coalesced stores; no per-entry key read). The rows' counts and offsets by
+// node go first, a thread each, in the same launch.
 template <typename OutT>
-__global__ __launch_bounds__(256) void k_far_targets_rows(const int64_t* __restrict__ off,
-                                                          int rows,
-                                                          const int32_t* __restrict__ nbl,
-                                                          const int32_t* __restrict__ node_level,
-                                                          const int64_t* __restrict__ row_sub,
-                                                          OutT* __restrict__ targets,
-                                                          OutT* __restrict__ levels) {
+__global__ __launch_bounds__(256) void k_far_targets_rows(
+    const int64_t* __restrict__ off, int rows, const int32_t* __restrict__ nbl,
+    const int32_t* __restrict__ node_level, const int64_t* __restrict__ row_sub,
+    OutT* __restrict__ targets, OutT* __restrict__ levels, OutT* __restrict__ counts,
+    OutT* __restrict__ node_offsets, int32_t* __restrict__ counts32) {
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < rows;
+       r += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t node = nbl[r];
+    const int64_t o = off[r], c = off[r + 1] - o;
+    counts[node] = (OutT)c;
+    counts32[node] = (int32_t)c;
+    node_offsets[node] = (OutT)o;
+    if (r == 0) node_offsets[rows] = (OutT)off[rows];
+  }
   const unsigned lane = lane_id();
   const int64_t nw = (int64_t)gridDim.x * (blockDim.x / YGG_WAVE);
   for (int64_t r = (int64_t)blockIdx.x * (blockDim.x / YGG_WAVE) + threadIdx.x / YGG_WAVE;
@@ -964,6 +972,68 @@ __global__ __launch_bounds__(256) void k_near_dense_from_list(
     OutT v = (OutT)-1;
     if (o + e < off[r + 1]) v = (OutT)leaf_position[(int64_t)nbrs[o + e]];
     __builtin_nontemporal_store(v, &nlp[i]);
+  }
+}
+
+// The row lists of at most kSmallRowSlots stream slots over at most
+// kSmallRowKeys keys in one workgroup: counts per key in LDS, their scan in list
+// order (row r holds key row_keys[r], or r), and every entry to the next free
+// place of its row. A record (k, v) is an entry v of row k and an entry k of row
+// v. Replaces five launches that take the host 4 us each; 8192 slots are where
+// the two passes over them reach that on one CU.
+constexpr int kSmallRowSlots = 8192, kSmallRowKeys = 4096;
+
+template <typename OutT>
+__global__ __launch_bounds__(1024) void k_rows_small(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals, int n, bool records,
+    uint32_t keys_n, const int32_t* __restrict__ row_keys, int rows, int64_t* __restrict__ off,
+    OutT* __restrict__ out) {
+  constexpr int kPer = kSmallRowKeys / 1024;
+  __shared__ uint32_t s_at[kSmallRowKeys];
+  __shared__ uint32_t s_sum[1024 / YGG_WAVE];
+  const int tid = threadIdx.x, w = tid / YGG_WAVE;
+  for (int i = tid; i < kSmallRowKeys; i += 1024) s_at[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < n; i += 1024) {
+    const uint32_t k = keys[i];
+    if (k < keys_n) atomicAdd(&s_at[k], 1u);
+    if (records) {
+      const uint32_t v = vals[i];
+      if (v < keys_n) atomicAdd(&s_at[v], 1u);
+    }
+  }
+  __syncthreads();
+  uint32_t key[kPer], cnt[kPer];
+  unsigned sum = 0;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int r = tid * kPer + q;
+    key[q] = r < rows ? (row_keys ? (uint32_t)row_keys[r] : (uint32_t)r) : keys_n;
+    cnt[q] = key[q] < keys_n ? s_at[key[q]] : 0u;
+    sum += cnt[q];
+  }
+  const unsigned inc = wave_inclusive_sum(sum);
+  if (lane_id() == YGG_WAVE - 1) s_sum[w] = inc;
+  __syncthreads();
+  unsigned run = inc - sum, total = 0;
+#pragma unroll
+  for (int q = 0; q < 1024 / YGG_WAVE; ++q) {
+    if (q < w) run += s_sum[q];
+    total += s_sum[q];
+  }
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int r = tid * kPer + q;
+    if (r < rows) off[r] = (int64_t)run;
+    if (key[q] < keys_n) s_at[key[q]] = run;
+    run += cnt[q];
+  }
+  if (tid == 0) off[rows] = (int64_t)total;
+  __syncthreads();
+  for (int i = tid; i < n; i += 1024) {
+    const uint32_t k = keys[i], v = vals[i];
+    if (k < keys_n) out[atomicAdd(&s_at[k], 1u)] = (OutT)v;
+    if (records && v < keys_n) out[atomicAdd(&s_at[v], 1u)] = (OutT)k;
   }
 }
 
@@ -1521,6 +1591,27 @@ static int lists_offsets_scatter(const ygg::RowBucketState& bs, const uint32_t* 
   return ygg::row_bucket_scatter(bs, key_offsets, row_sub, out_i64, out, st);
 }
 
+// Whether k_rows_small takes a list of n stream slots over keys_n keys.
+static bool rows_small(int64_t n, const int64_t* count, int64_t keys_n, const int64_t* row_sub,
+                       int end_bit, int digit_bits) {
+  return lists_bucketed(end_bit, digit_bits) && !count && !row_sub && n <= kSmallRowSlots &&
+         keys_n <= kSmallRowKeys;
+}
+
+static int rows_small_launch(const uint32_t* keys, const uint32_t* vals, int64_t n, bool records,
+                             int64_t keys_n, const int32_t* row_keys, int rows, int64_t* off,
+                             int out_i64, void* out, hipStream_t st) {
+  if (n > 0 && !out) return YGG_ERR_ARG;
+  if (out_i64)
+    hipLaunchKernelGGL(k_rows_small<int64_t>, dim3(1), dim3(1024), 0, st, keys, vals, (int)n,
+                       records, (uint32_t)keys_n, row_keys, rows, off, (int64_t*)out);
+  else
+    hipLaunchKernelGGL(k_rows_small<int32_t>, dim3(1), dim3(1024), 0, st, keys, vals, (int)n,
+                       records, (uint32_t)keys_n, row_keys, rows, off, (int32_t*)out);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
 size_t ygg_far_lists_sort_workspace_bytes(int64_t n, int end_bit, int digit_bits) {
   return lists_sort_ws(n, end_bit, digit_bits, nullptr);
 }
@@ -1545,7 +1636,11 @@ int ygg_far_lists_sort(const uint32_t* keys, const uint32_t* vals, int64_t n,
   int rc = lists_sort_split(entries, end_bit, digit_bits, T, ws, ws_bytes, st, &sort_bytes,
                             &row_counts, &scan_ws, &scan_bytes, &key_offsets);
   if (rc) return rc;
-  if (lists_bucketed(end_bit, digit_bits)) {
+  if (rows_small(n, count, T, row_sub, end_bit, digit_bits)) {
+    rc = rows_small_launch(keys, vals, n, pair_records != 0, T,
+                           pair_records ? nodes_by_level : nullptr, T, lm_offsets, out_i64,
+                           sources, st);
+  } else if (lists_bucketed(end_bit, digit_bits)) {
     // pair records hold node ids: counts by node, offsets in level-major
     // order through nodes_by_level
     ygg::RowBucketState bs;
@@ -1563,20 +1658,15 @@ int ygg_far_lists_sort(const uint32_t* keys, const uint32_t* vals, int64_t n,
                                         scan_ws, scan_bytes, st);
   }
   if (rc) return rc;
-  dim3 gr(grid_for(T, 256)), gw(grid_for((int64_t)T, 256 / YGG_WAVE, 16384));
-  if (out_i64) {
+  dim3 gw(grid_for((int64_t)T, 256 / YGG_WAVE, 16384));
+  if (out_i64)
     hipLaunchKernelGGL(k_far_targets_rows<int64_t>, gw, dim3(256), 0, st, lm_offsets, T,
                        nodes_by_level, node_level, row_sub, (int64_t*)targets,
-                       (int64_t*)target_levels);
-    hipLaunchKernelGGL(k_far_rows<int64_t>, gr, dim3(256), 0, st, lm_offsets, T, nodes_by_level,
-                       (int64_t*)counts, (int64_t*)node_offsets, counts32);
-  } else {
+                       (int64_t*)target_levels, (int64_t*)counts, (int64_t*)node_offsets, counts32);
+  else
     hipLaunchKernelGGL(k_far_targets_rows<int32_t>, gw, dim3(256), 0, st, lm_offsets, T,
                        nodes_by_level, node_level, row_sub, (int32_t*)targets,
-                       (int32_t*)target_levels);
-    hipLaunchKernelGGL(k_far_rows<int32_t>, gr, dim3(256), 0, st, lm_offsets, T, nodes_by_level,
-                       (int32_t*)counts, (int32_t*)node_offsets, counts32);
-  }
+                       (int32_t*)target_levels, (int32_t*)counts, (int32_t*)node_offsets, counts32);
   YGG_LAUNCH_CHECK();
   return YGG_OK;
 }
@@ -1606,7 +1696,10 @@ int ygg_near_lists_sort(const uint32_t* keys, const uint32_t* vals, int64_t n,
   int rc = lists_sort_split(entries, end_bit, digit_bits, keys_n, ws, ws_bytes, st, &sort_bytes,
                             &row_counts, &scan_ws, &scan_bytes, &key_offsets);
   if (rc) return rc;
-  if (lists_bucketed(end_bit, digit_bits)) {
+  if (rows_small(n, count, keys_n, row_sub, end_bit, digit_bits)) {
+    rc = rows_small_launch(keys, vals, n, leaf_nodes != nullptr, keys_n, leaf_nodes, L,
+                           row_offsets, out_i64, neighbors, st);
+  } else if (lists_bucketed(end_bit, digit_bits)) {
     ygg::RowBucketState bs;
     rc = ygg::row_bucket_count(keys, vals, leaf_nodes != nullptr, n, count, end_bit, keys_n,
                                leaf_nodes ? (L < keys_n ? L : keys_n) : L,

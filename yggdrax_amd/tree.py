@@ -231,19 +231,22 @@ def _as_positions(positions) -> torch.Tensor:
 
 def infer_bounds(positions) -> tuple[torch.Tensor, torch.Tensor]:
     """yggdrax/bounds.py:11-33 on the GPU."""
+    b6 = _inferred6(_as_positions(positions))
+    return b6[:3], b6[3:]
+
+
+def _inferred6(pos: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
-    pos = _as_positions(positions)
     b6 = torch.empty(6, dtype=torch.float32, device=pos.device)
     ws = _lib.workspace(lib.ygg_bounds_workspace_bytes(), pos.device)
     _lib.check(lib.ygg_infer_bounds(pos.data_ptr(), pos.shape[0], b6.data_ptr(), ws.data_ptr(),
                                     ws.numel(), _lib.stream_ptr(pos.device)), "infer_bounds")
-    return b6[:3], b6[3:]
+    return b6
 
 
 def _bounds6(pos: torch.Tensor, bounds) -> torch.Tensor:
     if bounds is None:
-        lo, hi = infer_bounds(pos)
-        return torch.cat([lo, hi])
+        return _inferred6(pos)
     lo = torch.as_tensor(bounds[0], dtype=torch.float32, device=pos.device).reshape(3)
     hi = torch.as_tensor(bounds[1], dtype=torch.float32, device=pos.device).reshape(3)
     return torch.cat([lo, hi]).contiguous()
@@ -358,8 +361,9 @@ def _build(positions, masses, bounds, *, leaf_size: int, return_reordered: bool,
     L = (n + leaf_size - 1) // leaf_size
     T = 2 * L - 1
     NI = L - 1
-    # both builds' scalar words in one buffer: one host copy reads them
-    scalars = torch.zeros(12, dtype=torch.int32, device=dev)
+    # both builds' scalar words (which they clear) in one buffer: one host
+    # copy reads them
+    scalars = torch.empty(12, dtype=torch.int32, device=dev)
     rad = _alloc_radix(L, dev, scalars[:8])
     rptr = _ptrs(_lib.RadixTopologyPtrs, rad)
     rws = _lib.workspace(lib.ygg_radix_build_workspace_bytes(n, leaf_size), dev)
