@@ -189,6 +189,45 @@ def test_grouped_wide_and_constant_keys(ygg):
     assert exps[1]["class_keys"].shape[0] == 1
 
 
+@pytest.mark.parametrize("n", [300, 70_001, 400_000])
+@pytest.mark.parametrize("zbits", [2, 3, 4, 5, 12])
+def test_grouped_keys_around_one_word(ygg, zbits, n):
+    """Class keys of 62 to 65 and of 72 bits (one word of 63, then two), with
+    classes that differ in the last bit only; runs of equal sort keys of one, of
+    a hundred and of more pairs than are ranked in place. Against the oracle."""
+    from types import SimpleNamespace
+    from yggdrax_amd import grouped_interactions as gi
+    pos, mass = inputs.uniform_cube(1 << 12, 4)
+    ref = oracle.build_tree(pos, mass, leaf_size=4)
+    tree = ygg.build_tree(torch.from_numpy(pos).cuda(), torch.from_numpy(mass).cuda(),
+                          leaf_size=4)
+    level = np.asarray(ref["node_level"])
+    nodes = np.flatnonzero(level == np.bincount(level).argmax())
+    rng = np.random.default_rng(n + zbits)
+    extent = np.asarray(ref["bounds_max"], np.float64) - np.asarray(ref["bounds_min"], np.float64)
+    cell = extent / 2.0 ** level[nodes[0]]
+    top = np.array([2 ** 30 - 64, 2 ** 30 - 64, 2 ** zbits - 1])  # floats of 24 bits
+    steps = np.stack([rng.integers(0, 40, nodes.size) * (t // 39 + (t < 39)) for t in top], 1)
+    steps = np.minimum(steps, top)
+    steps[0], steps[1] = 0, top
+    center = np.zeros((level.size, 3), np.float32)
+    center[nodes] = -(steps * cell).astype(np.float32)
+    src = rng.choice(nodes, n)
+    src[:2] = nodes[:2]
+    tgt = np.full(n, nodes[0])
+    rgeom = {"center": center}
+    exp = oracle.grouped_interactions_from_pairs(ref, rgeom, src, tgt)
+    k = exp["class_keys"].astype(np.int64)
+    bits = sum(int(k[:, j].max() - k[:, j].min()).bit_length() for j in range(5))
+    print("[layouts] key bits", bits, "pairs", n, "classes", k.shape[0], flush=True)
+    assert bits == 60 + zbits
+    g = _grouped_np(gi.build_grouped_interactions_from_pairs(
+        tree, SimpleNamespace(center=torch.from_numpy(center).cuda()),
+        torch.from_numpy(src).cuda(), torch.from_numpy(tgt).cuda()))
+    for f, v in g.items():
+        assert np.array_equal(_bits(v), _bits(exp[f].astype(v.dtype))), f
+
+
 def test_layouts_of_a_single_leaf_tree(ygg):
     """One leaf, no far pairs: dense buffers of one slot and one invalid
     entry; grouped buffers empty."""

@@ -164,9 +164,10 @@ __device__ __forceinline__ int32_t to_i32_like_numpy(double r) {
 }
 
 // Per-axis cell size of a level: max(extent / max(2^level, 1), 1e-12)
-// (grouped_interactions.py:34-38); 2^level and the division by it are exact.
+// (grouped_interactions.py:34-38); the division by 2^level is exact where the
+// quotient is not below 1e-12, so it is a change of exponent.
 __device__ __forceinline__ double cell_size(double extent, int level) {
-  return fmax(extent / fmax(ldexp(1.0, level), 1.0), 1e-12);
+  return fmax(ldexp(extent, -max(level, 0)), 1e-12);
 }
 
 struct GroupGeom {
@@ -182,26 +183,36 @@ struct GroupGeom {
 // Arithmetic is float64 as in the reference's NumPy code: the centre
 // difference, the IEEE division and the round-half-even are all exact
 // restatements, so the key is bit-identical.
-template <typename IdxT>
-__device__ __forceinline__ void group_fields(const IdxT* __restrict__ src,
-                                             const IdxT* __restrict__ tgt, int64_t i,
+struct GroupNode {
+  float c[3];
+  int32_t level;
+};
+
+__device__ __forceinline__ GroupNode group_node(const GroupGeom& g, int64_t v) {
+  return GroupNode{{g.center[3 * v], g.center[3 * v + 1], g.center[3 * v + 2]}, g.level[v]};
+}
+
+__device__ __forceinline__ void group_fields(const GroupNode& t, const GroupNode& s,
                                              const GroupGeom& g, int32_t f[5]) {
-  const int64_t t = (int64_t)tgt[i], s = (int64_t)src[i];
-  const int tl = g.level[t];
-  f[0] = tl;
-  f[1] = g.level[s];
+  f[0] = t.level;
+  f[1] = s.level;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const double ext = (double)g.bmax[a] - (double)g.bmin[a];
-    const double delta = (double)g.center[3 * t + a] - (double)g.center[3 * s + a];
-    f[2 + a] = to_i32_like_numpy(rint(delta / cell_size(ext, tl)));
+    const double delta = (double)t.c[a] - (double)s.c[a];
+    f[2 + a] = to_i32_like_numpy(rint(delta / cell_size(ext, t.level)));
   }
 }
 
+// Pairs per thread and step of the two kernels over the pairs: all their node
+// ids, then all their nodes are on the way before the first is used.
+constexpr int kGroupPer = 4;
+
 // Field-wise min (partials[b][0..4]) and max ([5..9]) of block b's pairs:
 // wavefront shuffles, then one LDS row per wavefront. No atomics, so the
-// reduction costs no cross-XCD traffic.
-constexpr int kMinmaxBlocks = 1024;
+// reduction costs no cross-XCD traffic. The nodes' gathers bound it (2.1e7
+// pairs: 256 us for 0.33 GB of node ids).
+constexpr int kMinmaxBlocks = 2048;
 
 // Pairs naming a node outside [0, T) are skipped and raise *err; the
 // classify call then fails before any kernel reads through them.
@@ -216,19 +227,38 @@ k_group_minmax(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt, int64
     lo[k] = INT32_MAX;
     hi[k] = INT32_MIN;
   }
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t t = (int64_t)tgt[i], s = (int64_t)src[i];
-    if (t < 0 || t >= g.num_nodes || s < 0 || s >= g.num_nodes) {
-      *err = 1;
-      continue;
-    }
-    int32_t f[5];
-    group_fields(src, tgt, i, g, f);
+  const int64_t step = (int64_t)gridDim.x * blockDim.x * kGroupPer;
+  for (int64_t b = blockIdx.x * (int64_t)blockDim.x * kGroupPer + threadIdx.x; b < n; b += step) {
+    int64_t t[kGroupPer], s[kGroupPer];
+    bool ok[kGroupPer];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      lo[k] = min(lo[k], f[k]);
-      hi[k] = max(hi[k], f[k]);
+    for (int q = 0; q < kGroupPer; ++q) {
+      const int64_t i = b + (int64_t)q * blockDim.x;
+      ok[q] = i < n;
+      t[q] = ok[q] ? (int64_t)tgt[i] : 0;
+      s[q] = ok[q] ? (int64_t)src[i] : 0;
+    }
+    GroupNode tn[kGroupPer], sn[kGroupPer];
+#pragma unroll
+    for (int q = 0; q < kGroupPer; ++q) {
+      if (t[q] < 0 || t[q] >= g.num_nodes || s[q] < 0 || s[q] >= g.num_nodes) {
+        *err = 1;
+        ok[q] = false;
+        t[q] = s[q] = 0;
+      }
+      tn[q] = group_node(g, t[q]);
+      sn[q] = group_node(g, s[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kGroupPer; ++q) {
+      int32_t f[5];
+      group_fields(tn[q], sn[q], g, f);
+      if (!ok[q]) continue;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        lo[k] = min(lo[k], f[k]);
+        hi[k] = max(hi[k], f[k]);
+      }
     }
   }
 #pragma unroll
@@ -258,12 +288,22 @@ k_group_minmax(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt, int64
 // Field offsets and widths of the packed key; the fields are concatenated
 // most significant first (target level, source level, dx, dy, dz), each
 // minus its minimum, so unsigned order of the packed value is the
-// lexicographic order of the signed fields. total = sum of widths.
+// lexicographic order of the signed fields. total = sum of widths. The sort
+// key is the top `head` bits of it: all of them, or 63 of a longer key (seven
+// 9-bit passes; 64 where more than 64 would be left).
 struct Pack {
   int32_t min[5];
   int32_t width[5];
   int32_t total;
   int32_t bad;  // a pair named a node outside [0, T)
+  int32_t head;
+};
+
+// The bits of a pair's key below its sort key, and the pair: what the sorted
+// order gathers.
+struct __attribute__((aligned(16))) KeyedPair {
+  uint64_t rest;
+  uint64_t pair;  // target << 32 | source
 };
 
 __global__ void __launch_bounds__(256)
@@ -311,30 +351,58 @@ k_group_pack_params(const int32_t* __restrict__ partials, int nblocks,
     }
     pk->total = total;
     pk->bad = *err;
+    pk->head = total <= 63 ? total : (total > 127 ? 64 : 63);
   }
 }
 
 template <typename IdxT>
-__global__ void k_group_pack(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt,
-                             int64_t n, GroupGeom g, Pack pk, uint64_t* __restrict__ lo_out,
-                             uint64_t* __restrict__ hi_out, uint64_t* __restrict__ pairs) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    int32_t f[5];
-    group_fields(src, tgt, i, g, f);
-    // node ids are below 2^31: one 8-byte record per pair for the emit gather
-    pairs[i] = ((uint64_t)(uint32_t)tgt[i] << 32) | (uint64_t)(uint32_t)src[i];
-    uint64_t lo = 0, hi = 0;
+__global__ void __launch_bounds__(256)
+k_group_pack(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt,
+                int64_t n, GroupGeom g, Pack pk, uint64_t* __restrict__ key_out,
+                             KeyedPair* __restrict__ recs) {
+  const int cut = pk.total - pk.head;  // 0..64
+  const int64_t step = (int64_t)gridDim.x * blockDim.x * kGroupPer;
+  for (int64_t b = blockIdx.x * (int64_t)blockDim.x * kGroupPer + threadIdx.x; b < n; b += step) {
+    int64_t t[kGroupPer], s[kGroupPer];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      const int w = pk.width[k];  // 0..32
-      if (w == 0) continue;
-      const uint64_t u = (uint64_t)((int64_t)f[k] - (int64_t)pk.min[k]);
-      hi = (hi << w) | (lo >> (64 - w));
-      lo = (lo << w) | u;
+    for (int q = 0; q < kGroupPer; ++q) {
+      const int64_t i = b + (int64_t)q * blockDim.x;
+      t[q] = i < n ? (int64_t)tgt[i] : 0;
+      s[q] = i < n ? (int64_t)src[i] : 0;
     }
-    lo_out[i] = lo;
-    if (hi_out) hi_out[i] = hi;
+    GroupNode tn[kGroupPer], sn[kGroupPer];
+#pragma unroll
+    for (int q = 0; q < kGroupPer; ++q) {
+      tn[q] = group_node(g, t[q]);
+      sn[q] = group_node(g, s[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kGroupPer; ++q) {
+      const int64_t i = b + (int64_t)q * blockDim.x;
+      if (i >= n) break;
+      int32_t f[5];
+      group_fields(tn[q], sn[q], g, f);
+      uint64_t lo = 0, hi = 0;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const int w = pk.width[k];  // 0..32
+        if (w == 0) continue;
+        const uint64_t u = (uint64_t)((int64_t)f[k] - (int64_t)pk.min[k]);
+        hi = (hi << w) | (lo >> (64 - w));
+        lo = (lo << w) | u;
+      }
+      uint64_t rest = 0;
+      if (cut == 64) {
+        rest = lo;
+        lo = hi;
+      } else if (cut > 0) {
+        rest = lo & ((1ull << cut) - 1ull);
+        lo = (lo >> cut) | (hi << (64 - cut));
+      }
+      // node ids are below 2^31
+      recs[i] = KeyedPair{rest, ((uint64_t)(uint32_t)t[q] << 32) | (uint64_t)(uint32_t)s[q]};
+      key_out[i] = lo;
+    }
   }
 }
 
@@ -351,79 +419,211 @@ __global__ void k_iota_u32(uint32_t* __restrict__ out, int64_t n) {
     out[i] = (uint32_t)i;
 }
 
-// 1 where sorted position i starts a class: its packed key (lo_s, hi_s,
-// already in sorted order) differs from position i - 1's.
-__global__ void k_group_flags(const uint64_t* __restrict__ lo_s, const uint64_t* __restrict__ hi_s,
-                              int64_t n, int32_t* __restrict__ flags) {
+__global__ void k_rest_keys(const KeyedPair* __restrict__ recs, int64_t n,
+                            uint64_t* __restrict__ out) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
-    flags[i] = i == 0 || lo_s[i] != lo_s[i - 1] || (hi_s && hi_s[i] != hi_s[i - 1]);
+    out[i] = recs[i].rest;
+}
+
+// The pairs and the rests of their keys (if any) in sorted order: one gather of
+// 16-byte records.
+__global__ void __launch_bounds__(256)
+k_group_gather(const KeyedPair* __restrict__ recs, const uint32_t* __restrict__ order, int64_t n,
+               uint64_t* __restrict__ pairs_s, uint64_t* __restrict__ rest_s) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const KeyedPair r = recs[order[i]];
+    pairs_s[i] = r.pair;
+    if (rest_s) rest_s[i] = r.rest;
+  }
+}
+
+// 1 where sorted position i starts a class: its key (key_s, rest_s if any)
+// differs from position i - 1's.
+__global__ void k_group_flags(const uint64_t* __restrict__ key_s,
+                              const uint64_t* __restrict__ rest_s, int64_t n,
+                              int32_t* __restrict__ flags) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    flags[i] = i == 0 || key_s[i] != key_s[i - 1] || (rest_s && rest_s[i] != rest_s[i - 1]);
+}
+
+// Finishes a stable sort by the top 63 bits of longer keys: the positions of
+// one sort key are put in the order of their rests (equal ones stay in theirs),
+// and the classes' first positions are marked. Keys of far pairs hardly ever
+// share 63 bits, so nearly all this does is read the sort keys once, where
+// sorting the rests too takes a third of the whole build: 2.1e7 pairs with
+// 100-bit keys, seven passes and 320 us here against twelve passes and a gather
+// of the second word, 3.4 ms in all against 4.5.
+// A wavefront takes the runs that start among its 64 positions, one after the
+// other, through LDS; a run belongs to one wavefront. A run longer than
+// kTieRun raises *too_long (the order is then not valid): ranking it costs its
+// square, at 512 about what sorting the rests would.
+constexpr int kTieThreads = 256;
+constexpr int kTieRun = 512;
+
+__global__ void __launch_bounds__(kTieThreads)
+k_group_ties(const uint64_t* __restrict__ key_s, int64_t n, uint32_t* __restrict__ order,
+             uint64_t* __restrict__ pairs_s, uint64_t* __restrict__ rest_s,
+             int32_t* __restrict__ flags, int32_t* __restrict__ too_long) {
+  __shared__ uint64_t s_rest[kTieThreads / YGG_WAVE][kTieRun];
+  __shared__ uint64_t s_pair[kTieThreads / YGG_WAVE][kTieRun];
+  __shared__ uint32_t s_ord[kTieThreads / YGG_WAVE][kTieRun];
+  const int w = (int)threadIdx.x / YGG_WAVE, lane = (int)lane_id();
+  const int64_t waves = (int64_t)gridDim.x * (kTieThreads / YGG_WAVE);
+  for (int64_t b = ((int64_t)blockIdx.x * (kTieThreads / YGG_WAVE) + w) * YGG_WAVE; b < n;
+       b += waves * YGG_WAVE) {
+    const int64_t i = b + lane;
+    const bool ok = i < n;
+    const uint64_t k = ok ? key_s[i] : 0;
+    const bool head = ok && (i == 0 || key_s[i - 1] != k);
+    const bool tied = ok && i + 1 < n && key_s[i + 1] == k;
+    if (head && !tied) flags[i] = 1;
+    uint64_t runs = __ballot(head && tied);
+    while (runs) {
+      const int first = __ffsll((unsigned long long)runs) - 1;
+      runs &= runs - 1;
+      const int64_t h = b + first;
+      const uint64_t key = (uint64_t)__shfl((unsigned long long)k, first, YGG_WAVE);
+      int len = 0;
+      while (len <= kTieRun) {
+        const int64_t j = h + len + lane;
+        const uint64_t same = __ballot(j < n && key_s[j] == key);
+        if (~same == 0ull) {
+          len += YGG_WAVE;
+          continue;
+        }
+        len += __ffsll((unsigned long long)~same) - 1;
+        break;
+      }
+      if (len > kTieRun) {
+        if (lane == 0) *too_long = 1;
+        continue;
+      }
+      for (int e = lane; e < len; e += YGG_WAVE) {
+        s_rest[w][e] = rest_s[h + e];
+        s_pair[w][e] = pairs_s[h + e];
+        s_ord[w][e] = order[h + e];
+      }
+      // the wavefront's own LDS: written before it is read, read before the
+      // next run writes it
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (int e = lane; e < len; e += YGG_WAVE) {
+        const uint64_t mine = s_rest[w][e];
+        int rank = 0;
+        bool starts = true;
+        for (int j = 0; j < len; ++j) {
+          const uint64_t o = s_rest[w][j];
+          rank += o < mine || (o == mine && j < e);
+          starts = starts && !(o == mine && j < e);
+        }
+        order[h + rank] = s_ord[w][e];
+        pairs_s[h + rank] = s_pair[w][e];
+        rest_s[h + rank] = mine;
+        flags[h + rank] = starts;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
 }
 
 // class_scan[i] = classes started before sorted position i, so position i
 // belongs to class class_scan[i + 1] - 1 and starts it iff the two differ.
-// A class head decodes its key fields from the sorted packed key.
+// A class head decodes its key fields from its packed key.
+// Bound by its writes: 2.1e7 pairs of as many classes, 64 contiguous bytes and
+// one scattered class id each, 590 us (930 us when the heads' keys were gathered
+// and each thread wrote its own class row).
+constexpr int kEmitThreads = 256;
+
 template <typename IdxT>
-__global__ void k_group_emit(const uint64_t* __restrict__ pairs, int64_t n,
+__global__ void __launch_bounds__(kEmitThreads)
+k_group_emit(const uint64_t* __restrict__ pairs_s, int64_t n,
                              const float* __restrict__ bmin,
                              const float* __restrict__ bmax, const Pack* __restrict__ pkp,
-                             const uint64_t* __restrict__ lo_s, const uint64_t* __restrict__ hi_s,
+                             const uint64_t* __restrict__ key_s,
+                             const uint64_t* __restrict__ rest_s,
                              const uint32_t* __restrict__ order, const int64_t* __restrict__ scan,
                              IdxT* __restrict__ csrc, IdxT* __restrict__ ctgt,
                              IdxT* __restrict__ cids, IdxT* __restrict__ coff,
                              int32_t* __restrict__ ckeys, float* __restrict__ cdisp) {
+  // the rows of a workgroup's classes are contiguous: they leave through LDS
+  __shared__ int32_t s_key[5 * kEmitThreads];
+  __shared__ float s_disp[3 * kEmitThreads];
   const Pack pk = *pkp;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t p = order[i];
-    const int64_t c = scan[i + 1] - 1;
-    const uint64_t tp = pairs[p];
-    csrc[i] = (IdxT)(uint32_t)tp;
-    ctgt[i] = (IdxT)(uint32_t)(tp >> 32);
-    cids[p] = (IdxT)c;
-    if (scan[i + 1] != scan[i]) {
-      coff[c] = (IdxT)i;
-      uint64_t lo = lo_s[i], hi = pk.total > 64 ? hi_s[i] : 0;
-      int32_t f[5];
-#pragma unroll
-      for (int k = 4; k >= 0; --k) {
-        const int w = pk.width[k];
-        uint64_t bits = 0;
-        if (w > 0) {
-          bits = lo & ((1ull << w) - 1ull);
-          lo = (lo >> w) | (hi << (64 - w));
-          hi >>= w;
+  const int cut = pk.total - pk.head;  // 0..64
+  const int tid = (int)threadIdx.x;
+  for (int64_t b = blockIdx.x * (int64_t)kEmitThreads; b < n;
+       b += (int64_t)gridDim.x * kEmitThreads) {
+    const int64_t i = b + tid, end = min(b + kEmitThreads, n);
+    const int64_t c0 = scan[b];  // classes that start before this workgroup's
+    const int rows = (int)(scan[end] - c0);
+    if (i < n) {
+      const int64_t p = order[i];
+      const int64_t c = scan[i + 1] - 1;
+      const uint64_t tp = pairs_s[i];
+      csrc[i] = (IdxT)(uint32_t)tp;
+      ctgt[i] = (IdxT)(uint32_t)(tp >> 32);
+      cids[p] = (IdxT)c;
+      if (scan[i + 1] != scan[i]) {
+        coff[c] = (IdxT)i;
+        const int r = (int)(c - c0);
+        uint64_t lo = key_s[i], hi = 0;
+        if (cut == 64) {
+          hi = lo;
+          lo = rest_s[i];
+        } else if (cut > 0) {
+          hi = lo >> (64 - cut);
+          lo = (lo << cut) | rest_s[i];
         }
-        f[k] = (int32_t)((int64_t)pk.min[k] + (int64_t)bits);
-      }
+        int32_t f[5];
 #pragma unroll
-      for (int k = 0; k < 5; ++k) ckeys[5 * c + k] = f[k];
-      // class displacement = index * target-level cell, rounded to float32
+        for (int k = 4; k >= 0; --k) {
+          const int w = pk.width[k];
+          uint64_t bits = 0;
+          if (w > 0) {
+            bits = lo & ((1ull << w) - 1ull);
+            lo = (lo >> w) | (hi << (64 - w));
+            hi >>= w;
+          }
+          f[k] = (int32_t)((int64_t)pk.min[k] + (int64_t)bits);
+        }
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const double ext = (double)bmax[a] - (double)bmin[a];
-        cdisp[3 * c + a] = (float)((double)f[2 + a] * cell_size(ext, f[0]));
+        for (int k = 0; k < 5; ++k) s_key[5 * r + k] = f[k];
+        // class displacement = index * target-level cell, rounded to float32
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double ext = (double)bmax[a] - (double)bmin[a];
+          s_disp[3 * r + a] = (float)((double)f[2 + a] * cell_size(ext, f[0]));
+        }
       }
+      if (i == n - 1) coff[scan[n]] = (IdxT)n;
     }
-    if (i == n - 1) coff[scan[n]] = (IdxT)n;
+    __syncthreads();
+    for (int k = tid; k < 5 * rows; k += kEmitThreads) ckeys[5 * c0 + k] = s_key[k];
+    for (int k = tid; k < 3 * rows; k += kEmitThreads) cdisp[3 * c0 + k] = s_disp[k];
+    __syncthreads();
   }
 }
 
 // The radix sort ranks at most 2^30 - 1 elements per call.
 constexpr int64_t kMaxGroupedPairs = (1ll << 30) - 1;
 
-// Workspace shared by the classify and emit calls. After classify, lo_s
-// holds the packed keys' low words and hi holds the high words, both in
+// Workspace shared by the classify and emit calls. After classify, pairs_s
+// holds the pairs, key_s the sort keys and rest_s the bits below them, all in
 // sorted order, and pack the packing parameters.
 struct GroupWs {
   int32_t* partials;
-  int32_t* err;
+  int32_t* err;  // [2]: a bad node id, a run of equal sort keys too long
   Pack* pack;
-  uint64_t* lo;
-  uint64_t* hi;
-  uint64_t* hi_in;
-  uint64_t* lo_s;
-  uint64_t* pairs;
+  uint64_t* key;
+  uint64_t* key_s;
+  uint64_t* alt;
+  uint64_t* rest_s;
+  uint64_t* pairs_s;
+  KeyedPair* recs;
   uint32_t* order1;
   int32_t* flags;
   void* sort_ws;
@@ -435,24 +635,28 @@ struct GroupWs {
 static bool group_ws_layout(int64_t n, void* ws, size_t ws_bytes, GroupWs* w, size_t* bytes) {
   Arena a(ws, ws_bytes);
   w->partials = a.take<int32_t>(10 * kMinmaxBlocks);
-  w->err = a.take<int32_t>(1);
+  w->err = a.take<int32_t>(2);
   w->pack = a.take<Pack>(1);
-  w->lo = a.take<uint64_t>((size_t)n);
-  w->hi = a.take<uint64_t>((size_t)n);
-  w->hi_in = a.take<uint64_t>((size_t)n);
-  w->lo_s = a.take<uint64_t>((size_t)n);
-  w->pairs = a.take<uint64_t>((size_t)n);
+  w->key = a.take<uint64_t>((size_t)n);
+  w->key_s = a.take<uint64_t>((size_t)n);
+  w->alt = a.take<uint64_t>((size_t)n);
+  w->rest_s = a.take<uint64_t>((size_t)n);
+  w->pairs_s = w->alt;  // written once the keys are sorted
+  w->recs = a.take<KeyedPair>((size_t)n);
   w->order1 = a.take<uint32_t>((size_t)n);
   w->flags = a.take<int32_t>((size_t)n);
-  w->sort_bytes = sort_workspace_bytes(n, 8, 64);
+  w->sort_bytes = std::max(sort_workspace_bytes(n, 8, 64, 8), sort_workspace_bytes(n, 8, 64, 9));
   w->sort_ws = a.take<char>(w->sort_bytes);
   w->scan_bytes = scan_workspace_bytes(n);
   w->scan_ws = a.take<char>(w->scan_bytes);
   if (bytes) *bytes = a.off;
-  return w->partials && w->err && w->pack && w->lo && w->hi && w->hi_in && w->lo_s && w->pairs &&
-         w->order1 &&
-         w->flags && w->sort_ws && w->scan_ws;
+  return w->partials && w->err && w->pack && w->key && w->key_s && w->alt && w->rest_s &&
+         w->recs && w->order1 && w->flags && w->sort_ws && w->scan_ws;
 }
+
+// Digit width of a class-key sort over `bits` bits: 9 unless 8 takes fewer
+// passes (a pass over 2e7 pairs takes 160 us with 9 bits, 176 us with 8).
+static int group_digit_bits(int bits) { return (bits + 8) / 9 <= (bits + 7) / 8 ? 9 : 8; }
 
 template <typename IdxT>
 int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, const GroupGeom& g,
@@ -460,9 +664,9 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, const GroupGeo
                      size_t ws_bytes, hipStream_t st) {
   GroupWs w;
   if (!group_ws_layout(n, ws, ws_bytes, &w, nullptr)) return YGG_ERR_WORKSPACE;
-  const int mgrid = grid_for(n, 256, kMinmaxBlocks);
+  const int mgrid = grid_for(n, 256 * kGroupPer, kMinmaxBlocks);
   int rc;
-  if ((rc = fill_u32((uint32_t*)w.err, 0u, 1, st))) return rc;
+  if ((rc = fill_u32((uint32_t*)w.err, 0u, 2, st))) return rc;
   hipLaunchKernelGGL(k_group_minmax<IdxT>, dim3(mgrid), dim3(256), 0, st, src, tgt, n, g,
                      w.partials, w.err);
   YGG_LAUNCH_CHECK();
@@ -475,41 +679,59 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, const GroupGeo
   if (pk.bad) return YGG_ERR_ARG;
   const int W = pk.total;
   if (W > 128) return YGG_ERR_UNSUPPORTED;
+  const int cut = W - pk.head;  // bits below the sort key
   const int pgrid = grid_for(n, 256);
-  hipLaunchKernelGGL(k_group_pack<IdxT>, dim3(pgrid), dim3(256), 0, st, src, tgt, n, g, pk, w.lo,
-                     W > 64 ? w.hi : nullptr, w.pairs);
+  hipLaunchKernelGGL(k_group_pack<IdxT>, dim3(grid_for(n, 256 * kGroupPer)), dim3(256), 0, st, src,
+                     tgt, n, g, pk, w.key, w.recs);
   YGG_LAUNCH_CHECK();
   if (W == 0) {  // one class: identity order, all keys zero
     hipLaunchKernelGGL(k_iota_u32, dim3(pgrid), dim3(256), 0, st, order, n);
     YGG_LAUNCH_CHECK();
-    if ((rc = copy_u32((uint32_t*)w.lo_s, (const uint32_t*)w.lo, 2 * n, st))) return rc;
-  } else if (W <= 64) {
-    if ((rc = sort_pairs_u64(w.lo, nullptr, w.lo_s, order, n, 0, W, w.sort_ws, w.sort_bytes,
-                             st)))
-      return rc;
-  } else {
-    // stable LSD over two words: the low word, then the high word carrying
-    // the first order; then the low words gathered into sorted order
-    if ((rc = sort_pairs_u64(w.lo, nullptr, w.lo_s, w.order1, n, 0, 64, w.sort_ws, w.sort_bytes,
-                             st)))
-      return rc;
-    hipLaunchKernelGGL(k_gather_keys, dim3(pgrid), dim3(256), 0, st, w.hi, w.order1, n,
-                       w.hi_in);
-    YGG_LAUNCH_CHECK();
-    if ((rc = sort_pairs_u64(w.hi_in, w.order1, w.hi, order, n, 0, W - 64, w.sort_ws,
-                             w.sort_bytes, st)))
-      return rc;
-    hipLaunchKernelGGL(k_gather_keys, dim3(pgrid), dim3(256), 0, st, w.lo, order, n, w.lo_s);
-    YGG_LAUNCH_CHECK();
-  }
-  hipLaunchKernelGGL(k_group_flags, dim3(pgrid), dim3(256), 0, st, w.lo_s,
-                     W > 64 ? w.hi : nullptr, n, w.flags);
-  YGG_LAUNCH_CHECK();
-  if ((rc = exclusive_scan_i32_to_i64(w.flags, nullptr, scan, n, w.scan_ws, w.scan_bytes, st)))
+    if ((rc = copy_u32((uint32_t*)w.key_s, (const uint32_t*)w.key, 2 * n, st))) return rc;
+  } else if ((rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, pk.head, w.sort_ws,
+                                  w.sort_bytes, st, nullptr, group_digit_bits(pk.head)))) {
     return rc;
+  }
+  hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
+                     cut ? w.rest_s : nullptr);
+  if (cut)
+    hipLaunchKernelGGL(k_group_ties, dim3(grid_for(n, kTieThreads, 4096)), dim3(kTieThreads), 0,
+                       st, w.key_s, n, order, w.pairs_s, w.rest_s, w.flags, w.err + 1);
+  else
+    hipLaunchKernelGGL(k_group_flags, dim3(pgrid), dim3(256), 0, st, w.key_s, nullptr, n, w.flags);
+  YGG_LAUNCH_CHECK();
   int64_t total = 0;
-  YGG_CHECK(hipMemcpyAsync(&total, scan + n, sizeof(total), hipMemcpyDeviceToHost, st));
-  YGG_CHECK(hipStreamSynchronize(st));
+  int32_t too_long = 0;
+  auto count = [&]() -> int {
+    const int e = exclusive_scan_i32_to_i64(w.flags, nullptr, scan, n, w.scan_ws, w.scan_bytes, st);
+    if (e) return e;
+    YGG_CHECK(hipMemcpyAsync(&total, scan + n, sizeof(total), hipMemcpyDeviceToHost, st));
+    if (cut)
+      YGG_CHECK(hipMemcpyAsync(&too_long, w.err + 1, sizeof(too_long), hipMemcpyDeviceToHost, st));
+    YGG_CHECK(hipStreamSynchronize(st));
+    return YGG_OK;
+  };
+  if ((rc = count())) return rc;
+  if (too_long) {
+    // many pairs of one sort key: a stable LSD sort over both words, the rests
+    // first, then the sort keys carrying that order
+    hipLaunchKernelGGL(k_rest_keys, dim3(pgrid), dim3(256), 0, st, w.recs, n, w.alt);
+    YGG_LAUNCH_CHECK();
+    if ((rc = sort_pairs_u64(w.alt, nullptr, w.rest_s, w.order1, n, 0, cut, w.sort_ws,
+                             w.sort_bytes, st, nullptr, group_digit_bits(cut))))
+      return rc;
+    hipLaunchKernelGGL(k_gather_keys, dim3(pgrid), dim3(256), 0, st, w.key, w.order1, n, w.alt);
+    YGG_LAUNCH_CHECK();
+    if ((rc = sort_pairs_u64(w.alt, w.order1, w.key_s, order, n, 0, pk.head, w.sort_ws,
+                             w.sort_bytes, st, nullptr, group_digit_bits(pk.head))))
+      return rc;
+    hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
+                       w.rest_s);
+    hipLaunchKernelGGL(k_group_flags, dim3(pgrid), dim3(256), 0, st, w.key_s, w.rest_s, n,
+                       w.flags);
+    YGG_LAUNCH_CHECK();
+    if ((rc = count())) return rc;
+  }
   *num_classes = total;
   return YGG_OK;
 }
@@ -599,17 +821,17 @@ int ygg_grouped_emit(int64_t num_pairs, int idx_i64, const float* bounds_min,
   GroupWs w;
   if (!group_ws_layout(num_pairs, ws, ws_bytes, &w, nullptr)) return YGG_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid(grid_for(num_pairs, 256));
+  dim3 grid(grid_for(num_pairs, kEmitThreads));
   if (idx_i64)
-    hipLaunchKernelGGL(k_group_emit<int64_t>, grid, dim3(256), 0, st, w.pairs, num_pairs,
-                       bounds_min, bounds_max, w.pack,
-                       w.lo_s, w.hi, order, class_scan, (int64_t*)class_sources,
+    hipLaunchKernelGGL(k_group_emit<int64_t>, grid, dim3(256), 0, st, w.pairs_s, num_pairs,
+                       bounds_min, bounds_max, w.pack, w.key_s, w.rest_s, order, class_scan,
+                       (int64_t*)class_sources,
                        (int64_t*)class_targets, (int64_t*)class_ids, (int64_t*)class_offsets,
                        class_keys, class_displacements);
   else
-    hipLaunchKernelGGL(k_group_emit<int32_t>, grid, dim3(256), 0, st, w.pairs, num_pairs,
-                       bounds_min, bounds_max, w.pack,
-                       w.lo_s, w.hi, order, class_scan, (int32_t*)class_sources,
+    hipLaunchKernelGGL(k_group_emit<int32_t>, grid, dim3(256), 0, st, w.pairs_s, num_pairs,
+                       bounds_min, bounds_max, w.pack, w.key_s, w.rest_s, order, class_scan,
+                       (int32_t*)class_sources,
                        (int32_t*)class_targets, (int32_t*)class_ids, (int32_t*)class_offsets,
                        class_keys, class_displacements);
   YGG_LAUNCH_CHECK();

@@ -780,28 +780,47 @@ __global__ __launch_bounds__(256) void k_scan_partials(int64_t* partial, int64_t
   if (threadIdx.x == 0) partial[nb] = carry;
 }
 
+// A tile in steps of four counts per thread: every load and store of a
+// wavefront covers consecutive bytes (2.1e7 counts: 69 us, 133 us with eight
+// consecutive counts per thread).
 __global__ __launch_bounds__(256) void k_scan_apply(const int32_t* __restrict__ c,
                                                     const int32_t* __restrict__ gather,
                                                     int64_t n, const int64_t* __restrict__ partial,
                                                     int64_t* __restrict__ out) {
-  int64_t b = (int64_t)blockIdx.x * kScanTile;
-  // blocked: thread t owns items [b + t*items, ...)
-  int64_t vals[kScanItems];
-  int64_t s = 0;
-  for (int k = 0; k < kScanItems; ++k) {
-    int64_t i = b + (int64_t)threadIdx.x * kScanItems + k;
-    vals[k] = i < n ? (int64_t)c[gather ? gather[i] : i] : 0;
-    s += vals[k];
-  }
-  int64_t ex;
-  block_exclusive_scan64(s, &ex);
-  int64_t run = partial[blockIdx.x] + ex;
-  for (int k = 0; k < kScanItems; ++k) {
-    int64_t i = b + (int64_t)threadIdx.x * kScanItems + k;
-    if (i < n) out[i] = run;
-    run += vals[k];
+  const int64_t tile = (int64_t)blockIdx.x * kScanTile;
+  int64_t run = partial[blockIdx.x];
+  int64_t vals[kScanItems / 4][4];
+#pragma unroll
+  for (int h = 0; h < kScanItems / 4; ++h)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t i = tile + h * (4 * kScanThreads) + 4 * (int64_t)threadIdx.x + k;
+      vals[h][k] = i < n ? (int64_t)c[gather ? gather[i] : i] : 0;
+    }
+#pragma unroll
+  for (int h = 0; h < kScanItems / 4; ++h) {
+    int64_t s = 0, ex;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s += vals[h][k];
+    const int64_t total = block_exclusive_scan64(s, &ex);
+    int64_t at = run + ex;
+    int64_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      o[k] = at;
+      at += vals[h][k];
+    }
+    const int64_t i = tile + h * (4 * kScanThreads) + 4 * (int64_t)threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + k < n) out[i + k] = o[k];
+    run += total;
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = partial[gridDim.x];
+}
+
+size_t scan_workspace_bytes(int64_t n) {
+  return align_up(sizeof(int64_t) * (size_t)((n + kScanTile - 1) / kScanTile + 2));
 }
 
 // The whole scan of at most kSmallScan counts in one workgroup: 4096 of them
@@ -841,10 +860,6 @@ __global__ __launch_bounds__(kSmallScanThreads) void k_scan_small(
     }
   }
   if (threadIdx.x == 0) out[n] = carry;
-}
-
-size_t scan_workspace_bytes(int64_t n) {
-  return align_up(sizeof(int64_t) * (size_t)((n + kScanTile - 1) / kScanTile + 2));
 }
 
 int exclusive_scan_i32_to_i64(const int32_t* counts, const int32_t* gather, int64_t* out,
