@@ -176,6 +176,7 @@ struct GroupGeom {
   const float* center;   // [T, 3]
   const float* bmin;     // [3]
   const float* bmax;     // [3]
+  const float4* node;    // [T] centre and level, or null
 };
 
 // Key fields of pair i: target level, source level and the rounded
@@ -189,6 +190,10 @@ struct GroupNode {
 };
 
 __device__ __forceinline__ GroupNode group_node(const GroupGeom& g, int64_t v) {
+  if (g.node) {
+    const float4 r = g.node[v];
+    return GroupNode{{r.x, r.y, r.z}, __float_as_int(r.w)};
+  }
   return GroupNode{{g.center[3 * v], g.center[3 * v + 1], g.center[3 * v + 2]}, g.level[v]};
 }
 
@@ -204,6 +209,16 @@ __device__ __forceinline__ void group_fields(const GroupNode& t, const GroupNode
   }
 }
 
+// Centre and level side by side: a pair's nodes come in two cache lines instead
+// of four, which is what bounds the two kernels over the pairs. 2.1e7 pairs: 211 and 258 us, 256 and 310 us
+// without.
+__global__ void k_group_nodes(GroupGeom g, float4* __restrict__ out) {
+  for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < g.num_nodes;
+       v += (int64_t)gridDim.x * blockDim.x)
+    out[v] = make_float4(g.center[3 * v], g.center[3 * v + 1], g.center[3 * v + 2],
+                         __int_as_float(g.level[v]));
+}
+
 // Pairs per thread and step of the two kernels over the pairs: all their node
 // ids, then all their nodes are on the way before the first is used.
 constexpr int kGroupPer = 4;
@@ -211,7 +226,7 @@ constexpr int kGroupPer = 4;
 // Field-wise min (partials[b][0..4]) and max ([5..9]) of block b's pairs:
 // wavefront shuffles, then one LDS row per wavefront. No atomics, so the
 // reduction costs no cross-XCD traffic. The nodes' gathers bound it (2.1e7
-// pairs: 256 us for 0.33 GB of node ids).
+// pairs: 211 us for 0.33 GB of node ids).
 constexpr int kMinmaxBlocks = 2048;
 
 // Pairs naming a node outside [0, T) are skipped and raise *err; the
@@ -454,14 +469,15 @@ __global__ void k_group_flags(const uint64_t* __restrict__ key_s,
 // and the classes' first positions are marked. Keys of far pairs hardly ever
 // share 63 bits, so nearly all this does is read the sort keys once, where
 // sorting the rests too takes a third of the whole build: 2.1e7 pairs with
-// 100-bit keys, seven passes and 320 us here against twelve passes and a gather
-// of the second word, 3.4 ms in all against 4.5.
+// 100-bit keys, seven passes and 220 us here against twelve passes and a gather
+// of the second word, 3.3 ms in all against 4.5.
 // A wavefront takes the runs that start among its 64 positions, one after the
 // other, through LDS; a run belongs to one wavefront. A run longer than
 // kTieRun raises *too_long (the order is then not valid): ranking it costs its
-// square, at 512 about what sorting the rests would.
+// square, and 20 KB of LDS per workgroup let eight of them share a CU (with runs
+// of up to 512, 320 us).
 constexpr int kTieThreads = 256;
-constexpr int kTieRun = 512;
+constexpr int kTieRun = 256;
 
 __global__ void __launch_bounds__(kTieThreads)
 k_group_ties(const uint64_t* __restrict__ key_s, int64_t n, uint32_t* __restrict__ order,
@@ -659,7 +675,7 @@ static bool group_ws_layout(int64_t n, void* ws, size_t ws_bytes, GroupWs* w, si
 static int group_digit_bits(int bits) { return (bits + 8) / 9 <= (bits + 7) / 8 ? 9 : 8; }
 
 template <typename IdxT>
-int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, const GroupGeom& g,
+int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
                      uint32_t* order, int64_t* scan, int64_t* num_classes, void* ws,
                      size_t ws_bytes, hipStream_t st) {
   GroupWs w;
@@ -667,6 +683,14 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, const GroupGeo
   const int mgrid = grid_for(n, 256 * kGroupPer, kMinmaxBlocks);
   int rc;
   if ((rc = fill_u32((uint32_t*)w.err, 0u, 2, st))) return rc;
+  // the table lies where the sort will work, if it fits: not for a tree of more
+  // nodes than pairs
+  if (sizeof(float4) * (size_t)g.num_nodes <= w.sort_bytes) {
+    float4* table = (float4*)w.sort_ws;
+    hipLaunchKernelGGL(k_group_nodes, dim3(grid_for(g.num_nodes, 256)), dim3(256), 0, st, g,
+                       table);
+    g.node = table;
+  }
   hipLaunchKernelGGL(k_group_minmax<IdxT>, dim3(mgrid), dim3(256), 0, st, src, tgt, n, g,
                      w.partials, w.err);
   YGG_LAUNCH_CHECK();
@@ -799,7 +823,7 @@ int ygg_grouped_classify(const void* sources, const void* targets, int64_t num_p
     return YGG_ERR_ARG;
   if (num_pairs > kMaxGroupedPairs) return YGG_ERR_UNSUPPORTED;
   if (num_nodes < 1) return YGG_ERR_ARG;
-  GroupGeom g{num_nodes, node_level, center, bounds_min, bounds_max};
+  GroupGeom g{num_nodes, node_level, center, bounds_min, bounds_max, nullptr};
   hipStream_t st = (hipStream_t)stream;
   if (idx_i64)
     return grouped_classify((const int64_t*)sources, (const int64_t*)targets, num_pairs, g,
