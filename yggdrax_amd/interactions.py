@@ -428,6 +428,12 @@ class _WalkContext:
         # generation 0 holds every root pair, so the queue holds at least those
         Q = max(4, int(queue_cap), 0 if roots is None else int(roots.numel()))
         wf = torch.empty((2, Q), dtype=torch.int64, device=dev)
+        # A resumable walk writes its totals once, after its generations. Others
+        # reserve from them in every chunk: off the cache line of the flags
+        # that every workgroup reads (on it, an emission walk at exact sizes
+        # takes 3.3 ms instead of 1.7 at 2^22 points)
+        counters = (self.counters if emit and grow
+                    else torch.empty(2, dtype=torch.int64, device=dev))
         # the counting walk adds its totals into spread lanes instead of
         # reserving per chunk on two contended addresses
         spread = None if emit else torch.empty(2 * SPREAD_LANES, dtype=torch.int64, device=dev)
@@ -454,7 +460,7 @@ class _WalkContext:
         p.nodes = self.nodes.data_ptr()
         p.wf0, p.wf1 = wf[0].data_ptr(), wf[1].data_ptr()
         p.gen_sizes, p.flags = self.gen_sizes.data_ptr(), self.flags.data_ptr()
-        p.counters = self.counters.data_ptr()
+        p.counters = counters.data_ptr()
         p.far_keys, p.far_vals = _lib.ptr(fk), _lib.ptr(fv)
         p.near_keys, p.near_vals = _lib.ptr(nk), _lib.ptr(nv)
         p.hist_gen, p.node_hist = int(hist_gen), _lib.ptr(node_hist)
