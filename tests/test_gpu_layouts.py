@@ -189,12 +189,13 @@ def test_grouped_wide_and_constant_keys(ygg):
     assert exps[1]["class_keys"].shape[0] == 1
 
 
-@pytest.mark.parametrize("n", [300, 70_001, 400_000])
+@pytest.mark.parametrize("n,same", [(300, 2), (40_001, 2), (40_001, 900), (70_001, 2), (400_000, 2)])
 @pytest.mark.parametrize("zbits", [2, 3, 4, 5, 12])
-def test_grouped_keys_around_one_word(ygg, zbits, n):
+def test_grouped_keys_around_one_word(ygg, zbits, n, same):
     """Class keys of 62 to 65 and of 72 bits (one word of 63, then two), with
-    classes that differ in the last bit only; runs of equal sort keys of one, of
-    a hundred and of more pairs than are ranked in place. Against the oracle."""
+    classes that differ in the last bit only; runs of equal sort keys of one
+    and of sixty pairs, ranked in place; one run too long for that; and of so
+    many that both words are sorted at once. Against the oracle."""
     from types import SimpleNamespace
     from yggdrax_amd import grouped_interactions as gi
     pos, mass = inputs.uniform_cube(1 << 12, 4)
@@ -213,7 +214,8 @@ def test_grouped_keys_around_one_word(ygg, zbits, n):
     center = np.zeros((level.size, 3), np.float32)
     center[nodes] = -(steps * cell).astype(np.float32)
     src = rng.choice(nodes, n)
-    src[:2] = nodes[:2]
+    src[:same] = nodes[1]
+    src[0] = nodes[0]
     tgt = np.full(n, nodes[0])
     rgeom = {"center": center}
     exp = oracle.grouped_interactions_from_pairs(ref, rgeom, src, tgt)

@@ -312,6 +312,7 @@ struct Pack {
   int32_t total;
   int32_t bad;  // a pair named a node outside [0, T)
   int32_t head;
+  int32_t repeats;  // sort keys met again in a sample of kGroupSample pairs
 };
 
 // The bits of a pair's key below its sort key, and the pair: what the sorted
@@ -366,8 +367,70 @@ k_group_pack_params(const int32_t* __restrict__ partials, int nblocks,
     }
     pk->total = total;
     pk->bad = *err;
+    pk->repeats = 0;
     pk->head = total <= 63 ? total : (total > 127 ? 64 : 63);
   }
+}
+
+// The sort key and the bits below it of a pair with fields f.
+__device__ __forceinline__ void pack_key(const int32_t f[5], const Pack& pk, uint64_t& key,
+                                         uint64_t& rest) {
+  uint64_t lo = 0, hi = 0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    const int w = pk.width[k];  // 0..32
+    if (w == 0) continue;
+    const uint64_t u = (uint64_t)((int64_t)f[k] - (int64_t)pk.min[k]);
+    hi = (hi << w) | (lo >> (64 - w));
+    lo = (lo << w) | u;
+  }
+  const int cut = pk.total - pk.head;  // 0..64
+  key = lo;
+  rest = 0;
+  if (cut == 64) {
+    rest = lo;
+    key = hi;
+  } else if (cut > 0) {
+    rest = lo & ((1ull << cut) - 1ull);
+    key = (lo >> cut) | (hi << (64 - cut));
+  }
+}
+
+// How often the sort keys of kGroupSample pairs, evenly spaced, repeat: one
+// workgroup, a table of twice as many slots in LDS. Pairs with bad node ids are
+// left out (the call fails for them).
+constexpr int kGroupSample = 4096;
+
+template <typename IdxT>
+__global__ void __launch_bounds__(1024)
+k_group_sample(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt, int64_t n, GroupGeom g,
+               Pack* __restrict__ pkp) {
+  constexpr unsigned kSlots = 2 * kGroupSample;
+  constexpr unsigned long long kEmpty = ~0ull;
+  __shared__ unsigned long long s_key[kSlots];
+  __shared__ int s_again;
+  const Pack pk = *pkp;
+  if (threadIdx.x == 0) s_again = 0;
+  for (unsigned k = threadIdx.x; k < kSlots; k += 1024) s_key[k] = kEmpty;
+  __syncthreads();
+  const int64_t taken = n < kGroupSample ? n : kGroupSample;
+  for (int64_t q = threadIdx.x; q < taken; q += 1024) {
+    const int64_t i = q * n / taken;
+    const int64_t t = (int64_t)tgt[i], v = (int64_t)src[i];
+    if (t < 0 || t >= g.num_nodes || v < 0 || v >= g.num_nodes) continue;
+    int32_t f[5];
+    group_fields(group_node(g, t), group_node(g, v), g, f);
+    uint64_t key, rest;
+    pack_key(f, pk, key, rest);
+    unsigned slot = (unsigned)((key * 0x9E3779B97F4A7C15ull) >> 51);  // 13 bits
+    for (unsigned probe = 0; probe < kSlots; ++probe, slot = (slot + 1) % kSlots) {
+      const unsigned long long was = atomicCAS(&s_key[slot], kEmpty, (unsigned long long)key);
+      if (was == (unsigned long long)key) atomicAdd(&s_again, 1);
+      if (was == (unsigned long long)key || was == kEmpty) break;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) pkp->repeats = s_again;
 }
 
 template <typename IdxT>
@@ -375,7 +438,6 @@ __global__ void __launch_bounds__(256)
 k_group_pack(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt,
                 int64_t n, GroupGeom g, Pack pk, uint64_t* __restrict__ key_out,
                              KeyedPair* __restrict__ recs) {
-  const int cut = pk.total - pk.head;  // 0..64
   const int64_t step = (int64_t)gridDim.x * blockDim.x * kGroupPer;
   for (int64_t b = blockIdx.x * (int64_t)blockDim.x * kGroupPer + threadIdx.x; b < n; b += step) {
     int64_t t[kGroupPer], s[kGroupPer];
@@ -397,23 +459,8 @@ k_group_pack(const IdxT* __restrict__ src, const IdxT* __restrict__ tgt,
       if (i >= n) break;
       int32_t f[5];
       group_fields(tn[q], sn[q], g, f);
-      uint64_t lo = 0, hi = 0;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        const int w = pk.width[k];  // 0..32
-        if (w == 0) continue;
-        const uint64_t u = (uint64_t)((int64_t)f[k] - (int64_t)pk.min[k]);
-        hi = (hi << w) | (lo >> (64 - w));
-        lo = (lo << w) | u;
-      }
-      uint64_t rest = 0;
-      if (cut == 64) {
-        rest = lo;
-        lo = hi;
-      } else if (cut > 0) {
-        rest = lo & ((1ull << cut) - 1ull);
-        lo = (lo >> cut) | (hi << (64 - cut));
-      }
+      uint64_t lo, rest;
+      pack_key(f, pk, lo, rest);
       // node ids are below 2^31
       recs[i] = KeyedPair{rest, ((uint64_t)(uint32_t)t[q] << 32) | (uint64_t)(uint32_t)s[q]};
       key_out[i] = lo;
@@ -697,6 +744,8 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
   hipLaunchKernelGGL(k_group_pack_params, dim3(1), dim3(256), 0, st, w.partials, mgrid, w.err,
                      w.pack);
   YGG_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_group_sample<IdxT>, dim3(1), dim3(1024), 0, st, src, tgt, n, g, w.pack);
+  YGG_LAUNCH_CHECK();
   Pack pk;
   YGG_CHECK(hipMemcpyAsync(&pk, w.pack, sizeof(Pack), hipMemcpyDeviceToHost, st));
   YGG_CHECK(hipStreamSynchronize(st));
@@ -704,6 +753,13 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
   const int W = pk.total;
   if (W > 128) return YGG_ERR_UNSUPPORTED;
   const int cut = W - pk.head;  // bits below the sort key
+  // r pairs to a sort key show as r sample^2 / 2 n repeats. From about 100 on
+  // ranking the ties, or finding a run too long, costs more than sorting the
+  // rests: with 200 (400) pairs to each of 16384 keys of 83 bits, 0.99 (1.59) ms
+  // sorting both words at once, 1.13 (2.26) ms the other way. The sample costs 40
+  // us at 2.1e7 pairs, 3.2 ms in all.
+  const double sample = (double)std::min<int64_t>(n, kGroupSample);
+  const bool both = cut > 0 && 2.0 * (double)pk.repeats * (double)n > 100.0 * sample * sample;
   const int pgrid = grid_for(n, 256);
   hipLaunchKernelGGL(k_group_pack<IdxT>, dim3(grid_for(n, 256 * kGroupPer)), dim3(256), 0, st, src,
                      tgt, n, g, pk, w.key, w.recs);
@@ -712,13 +768,16 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
     hipLaunchKernelGGL(k_iota_u32, dim3(pgrid), dim3(256), 0, st, order, n);
     YGG_LAUNCH_CHECK();
     if ((rc = copy_u32((uint32_t*)w.key_s, (const uint32_t*)w.key, 2 * n, st))) return rc;
-  } else if ((rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, pk.head, w.sort_ws,
-                                  w.sort_bytes, st, nullptr, group_digit_bits(pk.head)))) {
+  } else if (!both && (rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, pk.head,
+                                           w.sort_ws, w.sort_bytes, st, nullptr,
+                                           group_digit_bits(pk.head)))) {
     return rc;
   }
-  hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
+  if (!both) hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
                      cut ? w.rest_s : nullptr);
-  if (cut)
+  if (both)
+    ;  // below
+  else if (cut)
     hipLaunchKernelGGL(k_group_ties, dim3(grid_for(n, kTieThreads, 4096)), dim3(kTieThreads), 0,
                        st, w.key_s, n, order, w.pairs_s, w.rest_s, w.flags, w.err + 1);
   else
@@ -735,10 +794,10 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
     YGG_CHECK(hipStreamSynchronize(st));
     return YGG_OK;
   };
-  if ((rc = count())) return rc;
-  if (too_long) {
-    // many pairs of one sort key: a stable LSD sort over both words, the rests
-    // first, then the sort keys carrying that order
+  if (!both && (rc = count())) return rc;
+  if (both || too_long) {
+    // a stable LSD sort over both words, the rests first, then the sort keys
+    // carrying that order
     hipLaunchKernelGGL(k_rest_keys, dim3(pgrid), dim3(256), 0, st, w.recs, n, w.alt);
     YGG_LAUNCH_CHECK();
     if ((rc = sort_pairs_u64(w.alt, nullptr, w.rest_s, w.order1, n, 0, cut, w.sort_ws,
