@@ -529,14 +529,42 @@ __device__ __forceinline__ bool walk_chunk(const FlatArgs& a, const int g, const
   return true;
 }
 
+// Whether the walk has stopped (an overflow, or a pause to grow a stream),
+// the same for the whole workgroup. Workgroups of one launch raise the flags
+// while others start, so one thread reads them for its workgroup. Wavefronts
+// reading for themselves could part: if the first one left, the others would
+// go on with LDS words that it never wrote (barriers do not wait for ended
+// wavefronts). s_stop is written again only behind the next barrier.
+__device__ __forceinline__ bool walk_stopped(const FlatArgs& a, int& s_stop) {
+  if (threadIdx.x == 0)
+    s_stop = (atomic_load_agent(&a.flags[0]) | atomic_load_agent(&a.flags[1]) |
+              atomic_load_agent(&a.flags[2]) | atomic_load_agent(&a.flags[3])) != 0;
+  __syncthreads();
+  return s_stop != 0;
+}
+
 template <bool EMIT, int kFlatPer, bool TAGS = false>
 __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
   static_assert(!TAGS || EMIT, "tags are written by the emission walk");
   constexpr int kFlatChunk = kFlatThreads * kFlatPer;
-  if (atomic_load_agent(&a.flags[0]) | atomic_load_agent(&a.flags[1]) |
-      atomic_load_agent(&a.flags[2]) | atomic_load_agent(&a.flags[3]))
-    return;
+  __shared__ WalkShared<kFlatPer, TAGS> sh;
+  // Words of earlier generations, loaded ahead of the first barrier: scalar
+  // loads. Behind it the compiler takes vector loads, which miss to the line
+  // that every chunk's reservation adds to (emission walk of 2^24 clustered
+  // points: 8.2 ms instead of 5.5).
   const int64_t raw = a.gen_sizes[g];
+  unsigned long long bf = 0, bn = 0;
+  if (EMIT && a.gen_fill && g > 0) {
+    const unsigned long long* r = a.gen_fill + (size_t)(g - 1) * kGenRecWords;
+    const unsigned long long c = r[0];
+    bf = r[1] + (c >> 32);
+    bn = r[2] + (c & 0xFFFFFFFFull);
+  }
+  if (EMIT && threadIdx.x == 0) {
+    sh.gbase[0] = bf;
+    sh.gbase[1] = bn;
+  }
+  if (walk_stopped(a, sh.stop)) return;
   const int64_t size = raw < a.queue_cap ? raw : a.queue_cap;
   // Chunks of kFlatChunk pairs. Workgroups are dispatched round-robin over the
   // XCDs (workgroup b on XCD b % X); with xcd_groups = X the chunks split
@@ -555,28 +583,14 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
   // record's offsets plus its final counts, the same in every workgroup;
   // workgroup 0 stores them in record g, also when it has no chunk) and the
   // capacity check that pauses the walk before anything is written.
-  __shared__ WalkShared<kFlatPer, TAGS> sh;
   if (EMIT && a.gen_fill) {
-    if (c_first >= c_end && blockIdx.x != 0) return;
-    if (threadIdx.x == 0) {
-      unsigned long long bf = 0, bn = 0;
-      if (g > 0) {
-        const unsigned long long* r = a.gen_fill + (size_t)(g - 1) * kGenRecWords;
-        const unsigned long long c = r[0];
-        bf = r[1] + (c >> 32);
-        bn = r[2] + (c & 0xFFFFFFFFull);
-      }
-      sh.gbase[0] = bf;
-      sh.gbase[1] = bn;
-      if (blockIdx.x == 0) {
-        a.gen_fill[(size_t)g * kGenRecWords + 1] = bf;
-        a.gen_fill[(size_t)g * kGenRecWords + 2] = bn;
-      }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      a.gen_fill[(size_t)g * kGenRecWords + 1] = bf;
+      a.gen_fill[(size_t)g * kGenRecWords + 2] = bn;
     }
-    __syncthreads();
     if (c_first >= c_end) return;
     const int64_t worst = a.pair_records ? size : 2 * size;
-    if ((int64_t)sh.gbase[0] + worst > a.far_cap || (int64_t)sh.gbase[1] + worst > a.near_cap) {
+    if ((int64_t)bf + worst > a.far_cap || (int64_t)bn + worst > a.near_cap) {
       if (threadIdx.x == 0) atomicMax(&a.flags[3], (uint32_t)(g + 1));
       return;
     }
@@ -637,13 +651,11 @@ constexpr int kPersistChunk = kPersistThreads * kPersistPer;
 
 template <bool TAGS>
 __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, int half, int lo, int hi) {
-  if (atomic_load_agent(&a.flags[0]) | atomic_load_agent(&a.flags[1]) |
-      atomic_load_agent(&a.flags[2]) | atomic_load_agent(&a.flags[3]))
-    return;
   __shared__ WalkShared<kPersistPer, TAGS, kPersistThreads> sh;
   __shared__ uint64_t s_pairs[kPersistChunk];
   // slot g % 2: a wavefront may still read the last generation's
   __shared__ unsigned long long s_ready[2], s_ticket[2];
+  if (walk_stopped(a, sh.stop)) return;
   unsigned long long acc_f = 0, acc_n = 0;
   int g = lo;
   while (g < hi) {
