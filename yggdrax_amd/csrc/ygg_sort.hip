@@ -519,16 +519,23 @@ size_t sort_workspace_bytes(int64_t n, int key_bytes, int range_bits, int digit_
   if (digit_bits == 0) digit_bits = default_digit_bits(key_bytes, range_bits);
   const int passes = passes_for(range_bits, digit_bits);
   const size_t bins = (size_t)1 << digit_bits;
+  // Look-back words of the tiles of m pairs: two buffers in use; the narrower
+  // kinds keep room for every pass, as a workspace sized for one of them is
+  // also used for another.
+  auto lookback = [&](int64_t m) {
+    const size_t buffers = mid_sort(m, key_bytes, digit_bits) ? 2 : (size_t)passes;
+    return buffers * (size_t)num_tiles(m, key_bytes, digit_bits) * bins;
+  };
+  // A workspace for n pairs serves every smaller sort: where the tiles grow
+  // with n, the room stays at least what the last n of the smaller tiles takes.
+  size_t words = lookback(n);
+  for (int64_t last : {kLowSort, kMidSort})
+    if (n > last) words = std::max(words, lookback(last));
   Arena a(nullptr, 0);
-  int64_t t = num_tiles(n, key_bytes, digit_bits);
-  a.take<char>((size_t)n * key_bytes);                              // alternate keys
-  a.take<uint32_t>((size_t)n);                                      // alternate values
-  a.take<uint32_t>((size_t)passes * bins);                          // histograms
-  // tile counters + look-back (two buffers in use; the narrower kinds keep
-  // room for every pass, as a workspace sized for one of them is also used
-  // for another)
-  const size_t buffers = mid_sort(n, key_bytes, digit_bits) ? 2 : (size_t)passes;
-  a.take<uint32_t>((size_t)passes + buffers * t * bins);
+  a.take<char>((size_t)n * key_bytes);          // alternate keys
+  a.take<uint32_t>((size_t)n);                  // alternate values
+  a.take<uint32_t>((size_t)passes * bins);      // histograms
+  a.take<uint32_t>((size_t)passes + words);     // tile counters + look-back
   return a.off;
 }
 
