@@ -477,3 +477,25 @@ def test_records_at_the_workgroup_edge(lib, T, n):
             off, out = got["rows"], got["neighbors"]
         assert np.array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
         assert np.array_equal(_row_sorted(out.cpu().numpy()[:2 * n], counts), vals)
+
+
+@pytest.mark.parametrize("L,n", [(3, 40), (1000, 8192), (2048, 3000), (2048, 8193)])
+def test_near_records_of_no_row_stay_past_the_rows(lib, L, n):
+    """Records that name internal nodes, which are no row of the near lists:
+    the rows hold the leaves' entries and nothing else, whatever the other
+    keys' counts, in one workgroup (up to 8192 records) and beyond."""
+    print(f"[row buckets] records of no row L={L} n={n}", flush=True)
+    rng = np.random.default_rng(L + n)
+    T, leaf_nodes, row_of = _pair_tree(rng, L)
+    a, b = (rng.integers(0, T, n).astype(np.int32) for _ in range(2))
+    a[: n // 3] = 0  # one internal node's count is larger than most rows' starts
+    ke, ve = np.concatenate([row_of[a], row_of[b]]), np.concatenate([b, a])
+    keep = ke >= 0
+    counts, vals = _expected(ke[keep], ve[keep], L)
+    dev = torch.device("cuda")
+    got = _near(lib, torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev), n, None, L, 0,
+                leaf_nodes=torch.from_numpy(leaf_nodes).to(dev), nend=max(1, (T - 1).bit_length()))
+    assert np.array_equal(got["counts"].cpu().numpy(), counts)
+    assert np.array_equal(got["rows"].cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+    nb = got["neighbors"].cpu().numpy()[: int(counts.sum())]
+    assert np.array_equal(_row_sorted(nb, counts), vals)

@@ -1033,6 +1033,12 @@ __global__ __launch_bounds__(1024) void k_rows_small(
     if (q < w) run += s_sum[q];
     total += s_sum[q];
   }
+  if (row_keys) {
+    // a key that is no row's (never in the walk's records) lists its entries
+    // inside the output, past every row's, as k_key_offsets_fill has it
+    for (int i = tid; i < kSmallRowKeys; i += 1024) s_at[i] = total;
+    __syncthreads();
+  }
 #pragma unroll
   for (int q = 0; q < kPer; ++q) {
     const int r = tid * kPer + q;
