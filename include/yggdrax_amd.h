@@ -521,6 +521,13 @@ typedef struct YggFlatWalkParams {
 
 int ygg_walk_flat(const YggFlatWalkParams* params, uint32_t* host_status,
                   int32_t* num_generations, float* gen_ms, void* stream);
+/* The same with a bound of its own on the loads by which a workgroup waits
+ * for a small generation that others of its launch work on (ygg_walk_flat:
+ * 2^20, about a second). A wait that runs out is no overflow: the walk is
+ * repeated with one launch per generation, and *repeated is 1. */
+int ygg_walk_flat_polls(const YggFlatWalkParams* params, uint32_t* host_status,
+                        int32_t* num_generations, float* gen_ms, int32_t polls,
+                        int32_t* repeated, void* stream);
 /* The same walk as exactly max_generations generation launches with no host
  * synchronisation, so a caller can capture it into a HIP graph. Generation
  * sizes, counters and overflow flags stay in device memory (gen_sizes,

@@ -9,6 +9,8 @@ together)."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -61,3 +63,34 @@ def test_walk_profile_keeps_the_lists(case, monkeypatch, profile):
     torch.cuda.synchronize()
     parity.assert_interactions_equal(inter, rint)
     parity.assert_neighbors_equal(nbrs, rnb)
+
+
+@pytest.mark.parametrize("polls", [0, 1, 1 << 20])
+def test_a_wait_that_runs_out_is_no_overflow(case, monkeypatch, polls):
+    """A workgroup that stops waiting for a generation leaves no result: the
+    walk is repeated with one launch per generation, at the same queue."""
+    from yggdrax_amd import _lib
+    from yggdrax_amd import interactions as I
+    ygg, tree, geom, rint, rnb = case
+    print(f"[walk wait] polls={polls}", flush=True)
+    monkeypatch.setattr(I, "_GEN_PROFILES", type(I._GEN_PROFILES)())
+    real, calls = _lib.load(), []
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def ygg_walk_flat(self, p, host_status, ngen, gen_ms, stream):
+            again = ctypes.c_int32(-1)
+            rc = real.ygg_walk_flat_polls(p, host_status, ngen, gen_ms, polls,
+                                          ctypes.byref(again), stream)
+            calls.append(again.value)
+            return rc
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    inter, nbrs = ygg.build_interactions_and_neighbors(tree, geom, theta=0.5, mac_type="dehnen")
+    torch.cuda.synchronize()
+    parity.assert_interactions_equal(inter, rint)
+    parity.assert_neighbors_equal(nbrs, rnb)
+    assert len(calls) == 1  # one walk: no larger queue was tried
+    assert calls[0] == (1 if polls == 0 else 0 if polls > 1 else calls[0])

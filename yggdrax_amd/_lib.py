@@ -163,6 +163,8 @@ _SIGS = {
     "ygg_radix_leaf_order": (_INT, [_I64, _P, _P, _P]),
     "ygg_walk_prepare_nodes": (_INT, [_P, _P, _P, _P, _P, _P, _P, _I64, _INT, _F, _P, _P]),
     "ygg_walk_flat": (_INT, [ctypes.POINTER(FlatWalkParams), _P, ctypes.POINTER(_I32), _P, _P]),
+    "ygg_walk_flat_polls": (_INT, [ctypes.POINTER(FlatWalkParams), _P, ctypes.POINTER(_I32), _P,
+                                   _I32, ctypes.POINTER(_I32), _P]),
     "ygg_row_offsets": (_INT, [_P, _I64, _I64, _P, _P]),
     "ygg_far_lists_from_sorted": (_INT, [_I64, _P, _P, _I64, _P, _P, _P, _INT, _P, _P, _P, _P,
                                          _P, _P, _P]),

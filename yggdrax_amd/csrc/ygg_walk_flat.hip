@@ -37,7 +37,7 @@ struct FlatArgs {
   uint64_t* wf0;
   uint64_t* wf1;
   uint32_t* gen_sizes;
-  uint32_t* flags;                 // [0] queue, [1] far stream, [2] near stream
+  uint32_t* flags;                 // [0] queue (or kWaitRanOut), [1] far, [2] near stream
   unsigned long long* counters;    // [0] far total, [1] near total (emission walk: [0]
                                    // holds far << 32 | near until k_unpack_totals)
   uint32_t* far_keys;
@@ -643,14 +643,20 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
 // generation g's sync words: tickets (3), done chunks << 36 | children so far
 // (4), and what is published of it (5): kPublished | size, kPublished | kJump |
 // generation (go on there), or kPublished | kStopped.
+//
+// A wait ends after `polls` loads at the latest. That marks the walk with
+// kWaitRanOut in flags[0], which is no overflow: the host repeats it with one
+// launch per generation.
 constexpr unsigned long long kPublished = 1ull << 63, kStopped = 1ull << 62, kJump = 1ull << 61;
 constexpr int kTicketWord = 3, kDoneWord = 4, kReadyWord = 5;
-constexpr int kSpinLimit = 1 << 20;  // about a second
+constexpr int kWaitPolls = 1 << 20;  // about a second
+constexpr uint32_t kWaitRanOut = 2u;
 constexpr int kPersistThreads = 1024, kPersistPer = 2;
 constexpr int kPersistChunk = kPersistThreads * kPersistPer;
 
 template <bool TAGS>
-__global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, int half, int lo, int hi) {
+__global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, int half, int lo, int hi,
+                                                                  int polls) {
   __shared__ WalkShared<kPersistPer, TAGS, kPersistThreads> sh;
   __shared__ uint64_t s_pairs[kPersistChunk];
   // slot g % 2: a wavefront may still read the last generation's
@@ -666,13 +672,13 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
       if (g == lo) {
         v = kPublished | atomic_load_agent(&a.gen_sizes[g]);
       } else {
-        for (int spin = 0; spin < kSpinLimit; ++spin) {
+        for (int poll = 0; poll < polls; ++poll) {
           v = atomic_load_agent(&sync[kReadyWord]);
           if (v & kPublished) break;
           __builtin_amdgcn_s_sleep(1);
         }
-        if (!(v & kPublished)) {  // not reached: the walk counts as overflowed
-          atomicOr(&a.flags[0], 1u);
+        if (!(v & kPublished)) {
+          atomicOr(&a.flags[0], kWaitRanOut);
           v = kPublished | kStopped;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -1289,8 +1295,11 @@ static int persist_blocks(int lo, int hi, const uint32_t* hint) {
 static hipEvent_t g_flat_events[2 * 1025];
 static int g_flat_events_ready = 0;
 
-int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* num_generations,
-                  float* gen_ms, void* stream) {
+// The walk; *ran_out where a wait of k_walk_persist ended without its
+// generation, which leaves no result (never with persist false).
+static int walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* num_generations,
+                     float* gen_ms, bool persist, int32_t polls, bool* ran_out, void* stream) {
+  *ran_out = false;
   if (!p || !host_status || !num_generations) return YGG_ERR_ARG;
   if (gen_ms && p->max_generations > 1024) return YGG_ERR_ARG;
   if (gen_ms && !g_flat_events_ready) {
@@ -1344,10 +1353,11 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
   const int blocks = p->grid_blocks > 0 ? p->grid_blocks : 2048;
   int g = g0, batch = p->gen_hint > 0 ? p->gen_hint - g0 : 24;
   if (batch < 2) batch = 2;
+  const int half = G / 2;
+  // (node_hist would hold a repeated walk's counts twice)
+  persist = persist && a.gen_fill && !gen_ms && g0 == 0 && a.xcd_groups <= 1 && !a.node_hist;
   while (true) {
     int end = g + batch < G ? g + batch : G;
-    const int half = G / 2;
-    const bool persist = a.gen_fill && !gen_ms && g0 == 0 && a.xcd_groups <= 1;
     for (int k = g; k < end; ++k) {
       if (persist && k < half && persist_gen(k, a.num_roots, p->num_nodes, p->gen_pairs_hint)) {
         int hi = k + 1;
@@ -1358,10 +1368,10 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
         if (hi == end && hi < half) hi = end = half;  // however many are left
         if (a.far_tags)
           hipLaunchKernelGGL(k_walk_persist<true>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
-                             half, k, hi);
+                             half, k, hi, polls);
         else
           hipLaunchKernelGGL(k_walk_persist<false>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
-                             half, k, hi);
+                             half, k, hi, polls);
         k = hi - 1;
         continue;
       }
@@ -1393,6 +1403,10 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
     }
     YGG_CHECK(hipStreamSynchronize(st));
     const uint32_t* fl = host_status + G + 1;
+    if (fl[0] & kWaitRanOut) {
+      *ran_out = true;
+      return YGG_OK;
+    }
     int done = -1;
     for (int k = 0; k <= end; ++k)
       if (host_status[k] == 0) {
@@ -1428,6 +1442,25 @@ int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* nu
     g = end;
     batch = 8;
   }
+}
+
+int ygg_walk_flat_polls(const YggFlatWalkParams* p, uint32_t* host_status,
+                        int32_t* num_generations, float* gen_ms, int32_t polls, int32_t* repeated,
+                        void* stream) {
+  if (polls < 0 || !repeated) return YGG_ERR_ARG;
+  bool ran_out = false;
+  int rc = walk_flat(p, host_status, num_generations, gen_ms, true, polls, &ran_out, stream);
+  *repeated = ran_out ? 1 : 0;
+  if (rc == YGG_OK && ran_out)
+    rc = walk_flat(p, host_status, num_generations, gen_ms, false, polls, &ran_out, stream);
+  return rc;
+}
+
+int ygg_walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t* num_generations,
+                  float* gen_ms, void* stream) {
+  int32_t repeated = 0;
+  return ygg_walk_flat_polls(p, host_status, num_generations, gen_ms, kWaitPolls, &repeated,
+                             stream);
 }
 
 // The same walk with a fixed number of generation launches and no host
