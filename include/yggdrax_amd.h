@@ -516,7 +516,12 @@ typedef struct YggFlatWalkParams {
                                  at least 256 workgroups, at most grid_blocks) and so only the
                                  launch cost: any grid covers a generation, its workgroups
                                  stepping over the chunks. 0xFFFFFFFF for a generation, or
-                                 NULL for all: grids from the bound roots * 4^g alone. */
+                                 NULL for all: grids from the bound roots * 4^g alone.
+                                 A resumable walk runs its small generations (hinted at up to
+                                 65536 pairs; without a hint, bounded by that, or of a tree of
+                                 at most 16384 nodes) in launches of 64 workgroups for many
+                                 generations, whatever grid_blocks and pairs_per_thread; a
+                                 generation of more than 196608 pairs leaves them. */
 } YggFlatWalkParams;
 
 int ygg_walk_flat(const YggFlatWalkParams* params, uint32_t* host_status,

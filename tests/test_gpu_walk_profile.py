@@ -94,3 +94,46 @@ def test_a_wait_that_runs_out_is_no_overflow(case, monkeypatch, polls):
     parity.assert_neighbors_equal(nbrs, rnb)
     assert len(calls) == 1  # one walk: no larger queue was tried
     assert calls[0] == (1 if polls == 0 else 0 if polls > 1 else calls[0])
+
+
+@pytest.fixture(scope="module")
+def wide_case():
+    """A small tree whose wavefront grows past 196608 pairs (small theta)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    import yggdrax_amd as ygg
+    pos, mass = inputs.plummer_sphere(8192, 3)
+    ref = oracle.build_tree(pos, mass, leaf_size=4)
+    rgeom = oracle.compute_tree_geometry(ref, ref["positions_sorted"])
+    rint, rnb, _ = oracle.build_interactions_and_neighbors(ref, rgeom, theta=0.2,
+                                                            mac_type="dehnen")
+    tree, ps, _, _ = ygg.build_tree(torch.from_numpy(pos).cuda(), torch.from_numpy(mass).cuda(),
+                                    leaf_size=4, return_reordered=True)
+    return ygg, tree, ygg.compute_tree_geometry(tree, ps), rint, rnb
+
+
+@pytest.mark.parametrize("profile", ["none", "true", "tiny", "late"])
+def test_generations_too_large_for_one_launch(wide_case, monkeypatch, profile):
+    """Generations of small trees, or hinted as small, that turn out large
+    leave the launch that runs many: where the wavefront grows past the bound
+    (none, tiny) or at the launch's first generation (late)."""
+    from yggdrax_amd import interactions as I
+    ygg, tree, geom, rint, rnb = wide_case
+    print(f"[walk hand-back] {profile}", flush=True)
+    monkeypatch.setattr(I, "_GEN_PROFILES", type(I._GEN_PROFILES)())
+    kw = dict(theta=0.2, mac_type="dehnen")
+    if profile != "none":
+        ygg.build_interactions_and_neighbors(tree, geom, **kw)
+        (key, (prof, arr)), = I._GEN_PROFILES.items()
+        assert max(prof) > 196608 > prof[0]
+        big = max(range(len(prof)), key=lambda k: prof[k])
+        if profile == "tiny":
+            for k in range(len(prof)):
+                arr[k] = 1
+        elif profile == "late":
+            for k in range(len(prof)):
+                arr[k] = 1 << 20 if k < big else 1
+    inter, nbrs = ygg.build_interactions_and_neighbors(tree, geom, **kw)
+    torch.cuda.synchronize()
+    parity.assert_interactions_equal(inter, rint)
+    parity.assert_neighbors_equal(nbrs, rnb)

@@ -644,6 +644,11 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
 // (4), and what is published of it (5): kPublished | size, kPublished | kJump |
 // generation (go on there), or kPublished | kStopped.
 //
+// A generation of more than kHandBackPairs is left to a launch of its own:
+// whoever finds its size publishes kStopped and puts kHandBack | generation + 1
+// into flags[3], and the host goes on from there with one launch per
+// generation. Sizes are known ahead only from an earlier walk.
+//
 // A wait ends after `polls` loads at the latest. That marks the walk with
 // kWaitRanOut in flags[0], which is no overflow: the host repeats it with one
 // launch per generation.
@@ -651,6 +656,8 @@ constexpr unsigned long long kPublished = 1ull << 63, kStopped = 1ull << 62, kJu
 constexpr int kTicketWord = 3, kDoneWord = 4, kReadyWord = 5;
 constexpr int kWaitPolls = 1 << 20;  // about a second
 constexpr uint32_t kWaitRanOut = 2u;
+constexpr uint32_t kHandBack = 1u << 31;
+constexpr int64_t kHandBackPairs = 3 << 16;
 constexpr int kPersistThreads = 1024, kPersistPer = 2;
 constexpr int kPersistChunk = kPersistThreads * kPersistPer;
 
@@ -671,6 +678,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
       unsigned long long v = 0;
       if (g == lo) {
         v = kPublished | atomic_load_agent(&a.gen_sizes[g]);
+        if ((int64_t)(v & 0xFFFFFFFFull) > kHandBackPairs) {
+          atomicMax(&a.flags[3], kHandBack | (uint32_t)(g + 1));
+          v = kPublished | kStopped;
+        }
       } else {
         for (int poll = 0; poll < polls; ++poll) {
           v = atomic_load_agent(&sync[kReadyWord]);
@@ -759,9 +770,12 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
         const unsigned long long sum = atomicAdd(&sync[kDoneWord], mine) + mine;
         if (sum >> 36 == nchunks) {
           const unsigned long long total = sum & ((1ull << 36) - 1);
-          if (g + 1 < hi)
-            atomic_store_agent(&next[kReadyWord],
-                               kPublished | ((int64_t)total > a.queue_cap ? kStopped : total));
+          if (g + 1 < hi) {
+            const bool over = (int64_t)total > a.queue_cap;
+            const bool large = !over && (int64_t)total > kHandBackPairs;
+            if (large) atomicMax(&a.flags[3], kHandBack | (uint32_t)(g + 2));
+            atomic_store_agent(&next[kReadyWord], kPublished | (over || large ? kStopped : total));
+          }
           s_ticket[g & 1] = nchunks;  // none is left
         } else {
           s_ticket[g & 1] = atomicAdd(&sync[kTicketWord], 1ull);
@@ -1268,28 +1282,28 @@ static int gen_blocks(int k, int64_t roots, int64_t queue_cap, int per, int bloc
 }
 
 // Whether generation k goes to k_walk_persist: by the hint where there is
-// one, else by the bound roots * 4^k and, for small trees, always. Up to
-// kPersistPairs (32 workgroups) a generation takes 5 to 9 us there, against
-// 12 us and a launch; past that the releases outgrow the launch.
+// one, else by the bound roots * 4^k and, for small trees, always, as far as
+// k_walk_persist finds the generations small enough. One of P pairs takes 5 to
+// 9 us there up to kPersistPairs, against 12 us and a launch. Walks of a
+// Plummer sphere without a profile, in us by the pairs of the largest
+// generation:
+//   nodes  largest   all there   large ones handed back   all launched
+//    1023    20 K        356                 356                467
+//    4095    80 K        499                 501                606
+//    4095   264 K        641                 575                614
+//   16383   344 K        814                 656                683
+//   16383   1.1 M       1686                 805                825
+//   16383   4.2 M       4551                1180               1216
 constexpr int64_t kPersistPairs = 65536;
 constexpr int32_t kPersistNodes = 1 << 14;
+// Whatever the hint, as it may be wrong: with 1.5x the hinted chunks instead
+// the steps at 512 to 2^20 points took the same time.
 constexpr int kPersistBlocks = 64;
 static bool persist_gen(int k, int64_t roots, int32_t num_nodes, const uint32_t* hint) {
   if (hint && hint[k] != 0xFFFFFFFFu) return hint[k] <= kPersistPairs;
   int64_t bound = roots;
   for (int i = 0; i < k && bound <= kPersistPairs; ++i) bound *= 4;
   return bound <= kPersistPairs || num_nodes <= kPersistNodes;
-}
-
-// Workgroups for generations [lo, hi): 1.5x the chunks of the largest as
-// hinted, or kPersistBlocks where a size is unknown.
-static int persist_blocks(int lo, int hi, const uint32_t* hint) {
-  int64_t most = 1;
-  for (int k = lo; k < hi; ++k) {
-    if (!hint || hint[k] == 0xFFFFFFFFu) return kPersistBlocks;
-    most = std::max<int64_t>(most, ((int64_t)hint[k] * 3 / 2 + kPersistChunk - 1) / kPersistChunk);
-  }
-  return (int)std::min<int64_t>(most, kPersistBlocks);
 }
 
 static hipEvent_t g_flat_events[2 * 1025];
@@ -1364,13 +1378,12 @@ static int walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t*
         while (hi < end && hi < half &&
                persist_gen(hi, a.num_roots, p->num_nodes, p->gen_pairs_hint))
           ++hi;
-        const int blocks = persist_blocks(k, hi, p->gen_pairs_hint);
         if (hi == end && hi < half) hi = end = half;  // however many are left
         if (a.far_tags)
-          hipLaunchKernelGGL(k_walk_persist<true>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
+          hipLaunchKernelGGL(k_walk_persist<true>, dim3(kPersistBlocks), dim3(kPersistThreads), 0, st, a,
                              half, k, hi, polls);
         else
-          hipLaunchKernelGGL(k_walk_persist<false>, dim3(blocks), dim3(kPersistThreads), 0, st, a,
+          hipLaunchKernelGGL(k_walk_persist<false>, dim3(kPersistBlocks), dim3(kPersistThreads), 0, st, a,
                              half, k, hi, polls);
         k = hi - 1;
         continue;
@@ -1406,6 +1419,14 @@ static int walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t*
     if (fl[0] & kWaitRanOut) {
       *ran_out = true;
       return YGG_OK;
+    }
+    if (fl[3] & kHandBack) {  // generations from here on by launches
+      g = (int)(fl[3] & ~kHandBack) - 1;
+      batch = std::max(p->gen_hint - g, 8);
+      persist = false;
+      hipLaunchKernelGGL(k_flat_resume, dim3(1), dim3(64), 0, st, a);
+      YGG_LAUNCH_CHECK();
+      continue;
     }
     int done = -1;
     for (int k = 0; k <= end; ++k)
