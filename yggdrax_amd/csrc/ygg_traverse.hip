@@ -23,12 +23,9 @@ __global__ void k_prep_nodes(const float* __restrict__ center, const float* __re
                              const float* __restrict__ maxext, const int32_t* __restrict__ left,
                              const int32_t* __restrict__ right,
                              const int32_t* __restrict__ leaf_position, int T, int NI,
-                             const int32_t* __restrict__ nbl, int mac_type, float scale,
-                             NodeRec* __restrict__ out) {
-  // with a level order, thread r takes the node of rank r
-  const int rank = blockIdx.x * blockDim.x + threadIdx.x;
-  if (rank >= T) return;
-  const int k = nbl ? nbl[rank] : rank;
+                             int mac_type, float scale, NodeRec* __restrict__ out) {
+  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= T) return;
   NodeRec r;
   r.cx = center[3 * (int64_t)k];
   r.cy = center[3 * (int64_t)k + 1];
@@ -44,8 +41,16 @@ __global__ void k_prep_nodes(const float* __restrict__ center, const float* __re
   r.left = k < NI ? left[k] : -1;
   r.right = k < NI ? right[k] : -1;
   r.leafpos = k < NI ? -1 : leaf_position[k];
-  r.pad = nbl ? rank : 0;
+  r.pad = 0;
   out[k] = r;
+}
+
+// A launch of its own: a level order that does not name every node (a
+// caller's topology) must not leave a record unwritten, whose children the
+// walk would follow.
+__global__ void k_set_rank(const int32_t* __restrict__ nbl, int T, NodeRec* __restrict__ out) {
+  int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < T) out[nbl[r]].pad = r;
 }
 
 // Batched: records of every system's nodes with batch-global child ids,
@@ -366,8 +371,11 @@ int ygg_walk_prepare_nodes(const float* center, const float* radius, const float
   int T = (int)num_nodes, NI = (T - 1) / 2;
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(k_prep_nodes, dim3(grid_for(T, 256)), dim3(256), 0, st, center, radius,
-                     max_extent, left, right, leaf_position, T, NI, nodes_by_level, mac_type,
-                     dehnen_radius_scale, (NodeRec*)nodes_out);
+                     max_extent, left, right, leaf_position, T, NI, mac_type, dehnen_radius_scale,
+                     (NodeRec*)nodes_out);
+  if (nodes_by_level)
+    hipLaunchKernelGGL(k_set_rank, dim3(grid_for(T, 256)), dim3(256), 0, st, nodes_by_level, T,
+                       (NodeRec*)nodes_out);
   YGG_LAUNCH_CHECK();
   return YGG_OK;
 }
