@@ -721,6 +721,78 @@ static bool group_ws_layout(int64_t n, void* ws, size_t ws_bytes, GroupWs* w, si
 // passes (a pass over 2e7 pairs takes 160 us with 9 bits, 176 us with 8).
 static int group_digit_bits(int bits) { return (bits + 8) / 9 <= (bits + 7) / 8 ? 9 : 8; }
 
+// Class starts counted from w.flags: *total classes, and *too_long if a run of
+// equal sort keys was too long for k_group_ties.
+static int group_count(const GroupWs& w, int64_t n, int64_t* scan, int64_t* total,
+                       int32_t* too_long, hipStream_t st) {
+  if (int rc = exclusive_scan_i32_to_i64(w.flags, nullptr, scan, n, w.scan_ws, w.scan_bytes, st))
+    return rc;
+  YGG_CHECK(hipMemcpyAsync(total, scan + n, sizeof(*total), hipMemcpyDeviceToHost, st));
+  if (too_long)
+    YGG_CHECK(hipMemcpyAsync(too_long, w.err + 1, sizeof(*too_long), hipMemcpyDeviceToHost, st));
+  YGG_CHECK(hipStreamSynchronize(st));
+  return YGG_OK;
+}
+
+// Keys of one word: sorted whole (identity order for the single class of a key
+// without bits).
+static int group_order_one_word(const GroupWs& w, int64_t n, int bits, uint32_t* order,
+                                hipStream_t st) {
+  const int grid = grid_for(n, 256);
+  int rc;
+  if (bits == 0) {
+    hipLaunchKernelGGL(k_iota_u32, dim3(grid), dim3(256), 0, st, order, n);
+    YGG_LAUNCH_CHECK();
+    rc = copy_u32((uint32_t*)w.key_s, (const uint32_t*)w.key, 2 * n, st);
+  } else {
+    rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, bits, w.sort_ws, w.sort_bytes, st,
+                        nullptr, group_digit_bits(bits));
+  }
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_group_gather, dim3(grid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
+                     nullptr);
+  hipLaunchKernelGGL(k_group_flags, dim3(grid), dim3(256), 0, st, w.key_s, nullptr, n, w.flags);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
+// Longer keys that hardly ever share their sort key: sorted by it, and the runs
+// that do put in order in place.
+static int group_order_ties(const GroupWs& w, int64_t n, const Pack& pk, uint32_t* order,
+                            hipStream_t st) {
+  if (int rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, pk.head, w.sort_ws,
+                              w.sort_bytes, st, nullptr, group_digit_bits(pk.head)))
+    return rc;
+  hipLaunchKernelGGL(k_group_gather, dim3(grid_for(n, 256)), dim3(256), 0, st, w.recs, order, n,
+                     w.pairs_s, w.rest_s);
+  hipLaunchKernelGGL(k_group_ties, dim3(grid_for(n, kTieThreads, 4096)), dim3(kTieThreads), 0, st,
+                     w.key_s, n, order, w.pairs_s, w.rest_s, w.flags, w.err + 1);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
+// Longer keys of which many share their sort key: a stable LSD sort over both
+// words, the rests first, then the sort keys carrying that order.
+static int group_order_two_words(const GroupWs& w, int64_t n, const Pack& pk, uint32_t* order,
+                                 hipStream_t st) {
+  const int grid = grid_for(n, 256), cut = pk.total - pk.head;
+  hipLaunchKernelGGL(k_rest_keys, dim3(grid), dim3(256), 0, st, w.recs, n, w.alt);
+  YGG_LAUNCH_CHECK();
+  int rc = sort_pairs_u64(w.alt, nullptr, w.rest_s, w.order1, n, 0, cut, w.sort_ws, w.sort_bytes,
+                          st, nullptr, group_digit_bits(cut));
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_gather_keys, dim3(grid), dim3(256), 0, st, w.key, w.order1, n, w.alt);
+  YGG_LAUNCH_CHECK();
+  rc = sort_pairs_u64(w.alt, w.order1, w.key_s, order, n, 0, pk.head, w.sort_ws, w.sort_bytes, st,
+                      nullptr, group_digit_bits(pk.head));
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_group_gather, dim3(grid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
+                     w.rest_s);
+  hipLaunchKernelGGL(k_group_flags, dim3(grid), dim3(256), 0, st, w.key_s, w.rest_s, n, w.flags);
+  YGG_LAUNCH_CHECK();
+  return YGG_OK;
+}
+
 template <typename IdxT>
 int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
                      uint32_t* order, int64_t* scan, int64_t* num_classes, void* ws,
@@ -760,60 +832,21 @@ int grouped_classify(const IdxT* src, const IdxT* tgt, int64_t n, GroupGeom g,
   // us at 2.1e7 pairs, 3.2 ms in all.
   const double sample = (double)std::min<int64_t>(n, kGroupSample);
   const bool both = cut > 0 && 2.0 * (double)pk.repeats * (double)n > 100.0 * sample * sample;
-  const int pgrid = grid_for(n, 256);
   hipLaunchKernelGGL(k_group_pack<IdxT>, dim3(grid_for(n, 256 * kGroupPer)), dim3(256), 0, st, src,
                      tgt, n, g, pk, w.key, w.recs);
   YGG_LAUNCH_CHECK();
-  if (W == 0) {  // one class: identity order, all keys zero
-    hipLaunchKernelGGL(k_iota_u32, dim3(pgrid), dim3(256), 0, st, order, n);
-    YGG_LAUNCH_CHECK();
-    if ((rc = copy_u32((uint32_t*)w.key_s, (const uint32_t*)w.key, 2 * n, st))) return rc;
-  } else if (!both && (rc = sort_pairs_u64(w.key, nullptr, w.key_s, order, n, 0, pk.head,
-                                           w.sort_ws, w.sort_bytes, st, nullptr,
-                                           group_digit_bits(pk.head)))) {
-    return rc;
-  }
-  if (!both) hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
-                     cut ? w.rest_s : nullptr);
-  if (both)
-    ;  // below
-  else if (cut)
-    hipLaunchKernelGGL(k_group_ties, dim3(grid_for(n, kTieThreads, 4096)), dim3(kTieThreads), 0,
-                       st, w.key_s, n, order, w.pairs_s, w.rest_s, w.flags, w.err + 1);
-  else
-    hipLaunchKernelGGL(k_group_flags, dim3(pgrid), dim3(256), 0, st, w.key_s, nullptr, n, w.flags);
-  YGG_LAUNCH_CHECK();
   int64_t total = 0;
   int32_t too_long = 0;
-  auto count = [&]() -> int {
-    const int e = exclusive_scan_i32_to_i64(w.flags, nullptr, scan, n, w.scan_ws, w.scan_bytes, st);
-    if (e) return e;
-    YGG_CHECK(hipMemcpyAsync(&total, scan + n, sizeof(total), hipMemcpyDeviceToHost, st));
-    if (cut)
-      YGG_CHECK(hipMemcpyAsync(&too_long, w.err + 1, sizeof(too_long), hipMemcpyDeviceToHost, st));
-    YGG_CHECK(hipStreamSynchronize(st));
-    return YGG_OK;
-  };
-  if (!both && (rc = count())) return rc;
+  if (cut == 0) {
+    if ((rc = group_order_one_word(w, n, W, order, st))) return rc;
+    if ((rc = group_count(w, n, scan, &total, nullptr, st))) return rc;
+  } else if (!both) {
+    if ((rc = group_order_ties(w, n, pk, order, st))) return rc;
+    if ((rc = group_count(w, n, scan, &total, &too_long, st))) return rc;
+  }
   if (both || too_long) {
-    // a stable LSD sort over both words, the rests first, then the sort keys
-    // carrying that order
-    hipLaunchKernelGGL(k_rest_keys, dim3(pgrid), dim3(256), 0, st, w.recs, n, w.alt);
-    YGG_LAUNCH_CHECK();
-    if ((rc = sort_pairs_u64(w.alt, nullptr, w.rest_s, w.order1, n, 0, cut, w.sort_ws,
-                             w.sort_bytes, st, nullptr, group_digit_bits(cut))))
-      return rc;
-    hipLaunchKernelGGL(k_gather_keys, dim3(pgrid), dim3(256), 0, st, w.key, w.order1, n, w.alt);
-    YGG_LAUNCH_CHECK();
-    if ((rc = sort_pairs_u64(w.alt, w.order1, w.key_s, order, n, 0, pk.head, w.sort_ws,
-                             w.sort_bytes, st, nullptr, group_digit_bits(pk.head))))
-      return rc;
-    hipLaunchKernelGGL(k_group_gather, dim3(pgrid), dim3(256), 0, st, w.recs, order, n, w.pairs_s,
-                       w.rest_s);
-    hipLaunchKernelGGL(k_group_flags, dim3(pgrid), dim3(256), 0, st, w.key_s, w.rest_s, n,
-                       w.flags);
-    YGG_LAUNCH_CHECK();
-    if ((rc = count())) return rc;
+    if ((rc = group_order_two_words(w, n, pk, order, st))) return rc;
+    if ((rc = group_count(w, n, scan, &total, nullptr, st))) return rc;
   }
   *num_classes = total;
   return YGG_OK;
