@@ -35,7 +35,7 @@ extern "C" {
 /* Stable LSD radix sort of (key, u32 value) pairs over key bits
  * [begin_bit, end_bit), digit_bits (8..11) bits per pass; digit_bits 0 takes
  * ygg_sort_default_digit_bits. The workspace query must use the same
- * digit_bits as the sort. vals_in may be NULL (values become 0..n-1).
+ * digit_bits as the sort; a workspace for n serves every smaller n. vals_in may be NULL (values become 0..n-1).
  * keys_in must differ from keys_out. Replaces the XLA sorts behind
  * jnp.argsort(stable=True) (yggdrax/_tree_impl.py:401, yggdrax/octree.py:259,
  * yggdrax/_interactions_impl.py:1082). */
@@ -229,6 +229,10 @@ int ygg_level_counts(const int32_t* level_offsets, int32_t num_levels, void* out
 int ygg_radix_leaf_order(int64_t num_leaves, int32_t* leaf_indices, int32_t* leaf_position,
                          void* stream);
 
+/* geometry_to_level_major (yggdrax/_geometry_impl.py:342-433): padded
+ * [num_levels][max_nodes] level-major copies of the node geometry; slot j of
+ * level l holds node nodes_by_level[level_offsets[l] + j] while j is below
+ * the level's count, else zeros and node index -1. */
 int ygg_geometry_level_major(const float* center, const float* half_extent, const float* radius,
                              const float* max_extent, const int32_t* nodes_by_level,
                              const int32_t* level_offsets, int32_t num_levels, int64_t max_nodes,

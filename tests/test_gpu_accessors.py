@@ -74,10 +74,10 @@ def test_traversal_diagnostics_lines(system, capsys, monkeypatch):
     assert "[yggdrax.traversal]" not in capsys.readouterr().out
 
 
-@pytest.mark.parametrize("n,leaf", [(5, 8), (511 * 8, 8), (8193, 32), (20_000, 1)])
+@pytest.mark.parametrize("n,leaf", [(5, 8), (128 * 8, 8), (511 * 8, 8), (8193, 32), (20_000, 1)])
 def test_list_tables_against_tensor_formulas(n, leaf):
-    """One leaf, as many rows as threads of a workgroup less one, and rows for
-    the whole grid: the tables and the longest rows."""
+    """One leaf, as many nodes as threads of a workgroup less one, and rows for
+    several workgroups and for the whole grid: the tables and the longest rows."""
     import yggdrax_amd as ygg
     from yggdrax_amd.interactions import _list_tables
     from yggdrax_amd.tree import device_topology

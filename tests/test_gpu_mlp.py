@@ -75,8 +75,8 @@ def test_mlp_gradients_at_row_block_edges(B):
 @pytest.mark.parametrize("T", [1, 15, 17, 512 * 4 * 16 + 7])
 def test_mlp_forward_parent_matches_two_step_features(T):
     """Feature 4 made inside the kernel against the same feature written by
-    ygg_mlp_far_counts and log2 here (a tile's edges, and more tiles than one
-    round of the grid). exp2/log2 differ between the two in their last bits:
+    ygg_mlp_far_counts and log2 here (a tile's edges, and tiles for most of the
+    grid). exp2/log2 differ between the two in their last bits:
     1e-5 covers 2^-20 of a feature times the layers' gains."""
     from yggdrax_amd import _lib, learned
     lib = _lib.load()
@@ -97,6 +97,30 @@ def test_mlp_forward_parent_matches_two_step_features(T):
     up = parent.clamp(min=0).long()
     x[:, 4] = torch.where(parent >= 0, torch.log2(1.0 + far[up].double()) / 16.0, 0.0).float()
     torch.testing.assert_close(y, model.forward(x), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("n,leaf", [(5, 8), (9, 1), (24_580, 1), (200_000, 3)])
+def test_node_prediction_is_the_two_step_one(n, leaf):
+    """The second pass with feature 4 made in the kernel against the features
+    written twice, bit for bit, the operations being the same: one node, a
+    partial tile, and 1 and 2.7 rounds of the grid (768 workgroups of four
+    16-node tiles)."""
+    import yggdrax_amd as ygg
+    from yggdrax_amd import _lib, inputs, learned
+    lib = _lib.load()
+    pos, mass = inputs.plummer_sphere(n, 9)
+    tree, ps, _, _ = ygg.build_tree(torch.from_numpy(pos).cuda(), torch.from_numpy(mass).cuda(),
+                                    leaf_size=leaf, return_reordered=True)
+    geom = ygg.compute_tree_geometry(tree, ps)
+    dt = learned.device_topology(tree)
+    model = learned.CapacityModel(learned.init_params(3))
+    first = model.forward(learned.features(dt, geom, None))
+    far = torch.empty(dt.num_nodes, device=first.device)
+    _lib.check(lib.ygg_mlp_far_counts(first.data_ptr(), dt.num_nodes, float(model.scale[0]),
+                                      far.data_ptr(), _lib.stream_ptr(far.device)), "far counts")
+    want = model.forward(learned.features(dt, geom, far))
+    assert torch.equal(model.predict_nodes(tree, geom), want)
+    assert dt.num_nodes > 768 * 4 * 16 or n < 24_580
 
 
 def test_mlp_training_reduces_loss():

@@ -2,10 +2,10 @@
 profile (ygg_walk_flat's gen_pairs_hint): a profile only sizes the grids
 and the first batch of launches, so the lists stay those of the oracle
 with no profile, with the true profile, and with a profile that is far
-too small (one workgroup then runs every generation) or too short
-(generations past it launch from the bound alone), or names every third
-generation a large one (launches between generations that one launch runs
-together)."""
+too small (one launch of few workgroups then runs every generation) or too
+short (generations past it go by the bound and the tree's size alone), or
+names every third generation a large one (launches between generations that
+one launch runs together)."""
 
 from __future__ import annotations
 

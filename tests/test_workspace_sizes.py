@@ -49,7 +49,10 @@ def test_workspace_never_shrinks(name):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,sized_for", [(3 << 16, (3 << 16) + 1), (3 << 16, 200000),
-                                         (12288, 12289), (3 << 19, (3 << 19) + 1)])
+                                         (12288, 12289), (12289, 12289),
+                                         ((3 << 16) + 1, (3 << 16) + 1),
+                                         (3 << 19, (3 << 19) + 1),
+                                         ((3 << 19) + 1, (3 << 19) + 1)])
 def test_sort_in_a_workspace_of_a_larger_one(n, sized_for):
     lib = _lib.load()
     dev = torch.device("cuda")

@@ -53,8 +53,8 @@ __device__ __forceinline__ void merge_into(Box8& a, const Box8& b) {
   }
 }
 
-// Three floats to a load of 12 bytes, four points to three loads of 16; points
-// start at any multiple of 4 bytes.
+// Four floats in one load of 16 bytes at any multiple of 4 bytes: three of them
+// hold four points.
 struct __attribute__((packed, aligned(4))) Float4u {
   float v[4];
 };

@@ -124,8 +124,8 @@ __device__ __forceinline__ void hidden_layer(const u32x4_t (&a)[4][2], Bias bias
   }
 }
 
-// Log-scaled far count of a parent node (feature 4) from its predicted
-// log2 rate.
+// Feature 4: a parent node's far count (scale * 2^y of its predicted log2
+// rate), log-scaled.
 __device__ __forceinline__ float far_feature(float far) {
   return log2f(1.0f + fmaxf(far, 0.0f)) / 16.0f;
 }

@@ -503,10 +503,9 @@ static inline int64_t num_tiles(int64_t n, int key_bytes, int digit_bits) {
 // on ties). Measured on gfx950: 3.3e8 (u32, u32) pairs with 18-bit keys sort
 // in 4.4 ms with two 9-bit passes (4.9 ms with two 10-bit passes); 1.5e8
 // pairs with 19-bit keys in 2.31 ms with two 10-bit passes against 3.0 ms
-// (three 9-bit) and 3.23 ms (three 8-bit). 64-bit Morton codes keep 8-bit
-// digits (2^24 keys: 1.49 ms, against 1.72 ms with 9-bit and 2.8-4.8 ms
-// with 10- or 11-bit digits). Every width remains available to the
-// autotuner.
+// (three 9-bit) and 3.23 ms (three 8-bit). 64-bit keys default to 8 bits; the
+// Morton sorts ask for 9 (kMortonDigitBits: seven passes instead of eight, on
+// tiles made for them). Every width remains available to the autotuner.
 int default_digit_bits(int key_bytes, int range_bits) {
   if (key_bytes != 4) return 8;
   int best = 8;
