@@ -523,9 +523,10 @@ typedef struct YggFlatWalkParams {
                                  NULL for all: grids from the bound roots * 4^g alone.
                                  A resumable walk runs its small generations (hinted at up to
                                  65536 pairs; without a hint, bounded by that, or of a tree of
-                                 at most 16384 nodes) in launches of 64 workgroups for many
-                                 generations, whatever grid_blocks and pairs_per_thread; a
-                                 generation of more than 196608 pairs leaves them. */
+                                 at most 16384 nodes) in launches of 16 to 64 workgroups for
+                                 many generations, whatever grid_blocks and pairs_per_thread; a
+                                 generation that turns out large (98304 to 196608 pairs, by the
+                                 workgroups) leaves them. */
 } YggFlatWalkParams;
 
 int ygg_walk_flat(const YggFlatWalkParams* params, uint32_t* host_status,

@@ -116,7 +116,8 @@ def wide_case():
 def test_generations_too_large_for_one_launch(wide_case, monkeypatch, profile):
     """Generations of small trees, or hinted as small, that turn out large
     leave the launch that runs many: where the wavefront grows past the bound
-    (none, tiny) or at the launch's first generation (late)."""
+    of 64 workgroups (none) or of 16 (tiny), or at the launch's first
+    generation (late)."""
     from yggdrax_amd import interactions as I
     ygg, tree, geom, rint, rnb = wide_case
     print(f"[walk hand-back] {profile}", flush=True)

@@ -644,8 +644,9 @@ __global__ __launch_bounds__(256) void k_walk_flat(FlatArgs a, int g) {
 // (4), and what is published of it (5): kPublished | size, kPublished | kJump |
 // generation (go on there), or kPublished | kStopped.
 //
-// A generation of more than kHandBackPairs is left to a launch of its own:
-// whoever finds its size publishes kStopped and puts kHandBack | generation + 1
+// A generation of more than kHandBackPairs, or of more than kHandBackRounds
+// chunks a workgroup, is left to a launch of its own: whoever finds its size
+// publishes kStopped and puts kHandBack | generation + 1
 // into flags[3], and the host goes on from there with one launch per
 // generation. Sizes are known ahead only from an earlier walk.
 //
@@ -658,6 +659,7 @@ constexpr int kWaitPolls = 1 << 20;  // about a second
 constexpr uint32_t kWaitRanOut = 2u;
 constexpr uint32_t kHandBack = 1u << 31;
 constexpr int64_t kHandBackPairs = 3 << 16;
+constexpr int kHandBackRounds = 3;
 constexpr int kPersistThreads = 1024, kPersistPer = 2;
 constexpr int kPersistChunk = kPersistThreads * kPersistPer;
 
@@ -669,6 +671,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
   // slot g % 2: a wavefront may still read the last generation's
   __shared__ unsigned long long s_ready[2], s_ticket[2];
   if (walk_stopped(a, sh.stop)) return;
+  const int64_t most =
+      min(kHandBackPairs, (int64_t)gridDim.x * (kHandBackRounds * kPersistChunk));
   unsigned long long acc_f = 0, acc_n = 0;
   int g = lo;
   while (g < hi) {
@@ -678,7 +682,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
       unsigned long long v = 0;
       if (g == lo) {
         v = kPublished | atomic_load_agent(&a.gen_sizes[g]);
-        if ((int64_t)(v & 0xFFFFFFFFull) > kHandBackPairs) {
+        if ((int64_t)(v & 0xFFFFFFFFull) > most) {
           atomicMax(&a.flags[3], kHandBack | (uint32_t)(g + 1));
           v = kPublished | kStopped;
         }
@@ -772,7 +776,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_walk_persist(FlatArgs a, in
           const unsigned long long total = sum & ((1ull << 36) - 1);
           if (g + 1 < hi) {
             const bool over = (int64_t)total > a.queue_cap;
-            const bool large = !over && (int64_t)total > kHandBackPairs;
+            const bool large = !over && (int64_t)total > most;
             if (large) atomicMax(&a.flags[3], kHandBack | (uint32_t)(g + 2));
             atomic_store_agent(&next[kReadyWord], kPublished | (over || large ? kStopped : total));
           }
@@ -1296,14 +1300,26 @@ static int gen_blocks(int k, int64_t roots, int64_t queue_cap, int per, int bloc
 //   16383   4.2 M       4551                1180               1216
 constexpr int64_t kPersistPairs = 65536;
 constexpr int32_t kPersistNodes = 1 << 14;
-// Whatever the hint, as it may be wrong: with 1.5x the hinted chunks instead
-// the steps at 512 to 2^20 points took the same time.
-constexpr int kPersistBlocks = 64;
+constexpr int kPersistBlocks = 64, kPersistMinBlocks = 16;
 static bool persist_gen(int k, int64_t roots, int32_t num_nodes, const uint32_t* hint) {
   if (hint && hint[k] != 0xFFFFFFFFu) return hint[k] <= kPersistPairs;
   int64_t bound = roots;
   for (int i = 0; i < k && bound <= kPersistPairs; ++i) bound *= 4;
   return bound <= kPersistPairs || num_nodes <= kPersistNodes;
+}
+
+// Workgroups for generations [lo, hi): kPersistBlocks where a size is unknown,
+// else 1.5x the chunks of the largest as hinted. Every workgroup that waits asks
+// the same words: at 10 007 points 167 us with 1 to 16 workgroups, 181 with 64
+// (512 points: 50.7, 52.0 and 54.0 us with 1, 16 and 64). At least 16, as a hint
+// may be too small.
+static int persist_blocks(int lo, int hi, const uint32_t* hint) {
+  int64_t most = kPersistMinBlocks;
+  for (int k = lo; k < hi; ++k) {
+    if (!hint || hint[k] == 0xFFFFFFFFu) return kPersistBlocks;
+    most = std::max<int64_t>(most, ((int64_t)hint[k] * 3 / 2 + kPersistChunk - 1) / kPersistChunk);
+  }
+  return (int)std::min<int64_t>(most, kPersistBlocks);
 }
 
 static hipEvent_t g_flat_events[2 * 1025];
@@ -1378,12 +1394,13 @@ static int walk_flat(const YggFlatWalkParams* p, uint32_t* host_status, int32_t*
         while (hi < end && hi < half &&
                persist_gen(hi, a.num_roots, p->num_nodes, p->gen_pairs_hint))
           ++hi;
+        const int workgroups = persist_blocks(k, hi, p->gen_pairs_hint);
         if (hi == end && hi < half) hi = end = half;  // however many are left
         if (a.far_tags)
-          hipLaunchKernelGGL(k_walk_persist<true>, dim3(kPersistBlocks), dim3(kPersistThreads), 0, st, a,
+          hipLaunchKernelGGL(k_walk_persist<true>, dim3(workgroups), dim3(kPersistThreads), 0, st, a,
                              half, k, hi, polls);
         else
-          hipLaunchKernelGGL(k_walk_persist<false>, dim3(kPersistBlocks), dim3(kPersistThreads), 0, st, a,
+          hipLaunchKernelGGL(k_walk_persist<false>, dim3(workgroups), dim3(kPersistThreads), 0, st, a,
                              half, k, hi, polls);
         k = hi - 1;
         continue;
